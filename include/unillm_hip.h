@@ -75,7 +75,7 @@ extern "C" {
 #define UNILLM_PATH_GEMV 1         /* fused dequant + GEMV (VALU int8 dot), m <= 4 */
 #define UNILLM_PATH_DECODE_MFMA 2  /* batched decode, f16 MFMA, fp32 accumulate */
 #define UNILLM_PATH_PREFILL_MFMA 3 /* prefill, LDS-staged f16 MFMA (x rows scaled by powers of two), fp32 accumulate */
-#define UNILLM_PATH_DENSE 4        /* dense weights: f32 GEMM (rocBLAS), the only path they take */
+#define UNILLM_PATH_DENSE 4        /* dense weights: f32 products (GEMV; split-part MFMA GEMM), the only path they take */
 
 typedef struct unillm_qweight unillm_qweight;
 typedef struct unillm_kv_cache unillm_kv_cache;
@@ -93,7 +93,7 @@ const char* unillm_hip_last_error(void);
 /* Upload one GGUF Q4_0 / Q5_0 / Q8_0 / Q4_K / Q5_K / Q6_K tensor ([n, k]: n * k/32 blocks
  * of 18 / 22 / 34 B, or n * k/256 blocks of 144 / 176 / 210 B), or a dense F32 / F16 / BF16 one
  * (n * k elements of 4 / 2 / 2 B), to the device, repacked there into the kernels'
- * layout (dense: f32 rows).  Replaces
+ * layout (dense: rows in their own type).  Replaces
  * `QMatMul::from_arc(Arc::new(qtensor))` at
  * crates/runtime/src/weight_loader_core.rs:569-571 (the QTensor read at :545).
  * layout_flags must be 0 (reserved). */

@@ -1,0 +1,86 @@
+"""The dense weights' GEMV and split-part GEMM at the edges of their tiles and plans.
+
+Against float64 of the exactly widened weights: an f32 sum over k rounds at most once a
+product, so 1e-6 normwise up to k 4096 (an f32 GEMM measures 5.8e-7 there).  Non-finite
+operands are compared with the f32 product of the same rows.
+"""
+import pytest
+import torch
+
+from unillm_amd import QuantLinear
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-6
+DTYPES = [torch.float32, torch.float16, torch.bfloat16]
+
+
+def _err(y, ref):
+    return ((y.double() - ref).norm() / ref.norm()).item()
+
+
+def _make(m, n, k, dtype, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    w = (torch.randn(n, k, device="cuda", generator=g) * 0.05).to(dtype)
+    return w, torch.randn(m, k, device="cuda", generator=g)
+
+
+# m: the GEMV's token counts (1, 2, 4, 8) and past its LDS limit (3 x 11008, 8 x 4104),
+# tiles of 64 and 128 rows with remainders; n: 1, and around the 128 / 256 column tiles;
+# k: one element, odd, around the padding to 64, split and unsplit
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (1, 255, 511), (2, 257, 4096), (3, 40, 11008),
+                                   (7, 130, 520), (8, 129, 4096), (8, 129, 4104), (9, 1, 63),
+                                   (63, 256, 64), (64, 257, 65), (65, 127, 2048), (129, 300, 4096),
+                                   (400, 129, 200)])
+def test_dense_edges(dtype, m, n, k):
+    print(f"dense edges {dtype} m={m} n={n} k={k}", flush=True)
+    w, x = _make(m, n, k, dtype, 31 * m + n + k)
+    ql = QuantLinear.from_dense(w)
+    ref = x.double() @ w.double().t()
+    y = ql.forward(x)
+    assert _err(y, ref) < TOL
+    assert torch.equal(ql.forward(x), y)
+    r = torch.randn_like(y)
+    want = r.double() + ref
+    assert _err(ql.forward_add(x, r), want) < TOL
+    # x at a 4-byte offset
+    buf = torch.empty(m * k + 1, device="cuda")
+    buf[1:] = x.reshape(-1)
+    assert torch.equal(ql.forward(buf[1:].view(m, k)), y)
+
+
+# rows of very different size, and weights in the subnormal range of f16
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m", [2, 40])
+def test_dense_wide_ranges(dtype, m):
+    n, k = 200, 512
+    w, x = _make(m, n, k, dtype, 5)
+    w[::3] = (w[::3].float() * 1e-4).to(dtype)
+    x *= torch.logspace(-12, 12, m, device="cuda")[:, None]
+    x[:, 7] *= 1e4  # one outlier a row
+    ql = QuantLinear.from_dense(w)
+    y, ref = ql.forward(x), x.double() @ w.double().t()
+    # an f32 dot's own bound, element by element: its error is relative to sum |x w|
+    size = x.double().abs() @ w.double().abs().t()
+    assert ((y.double() - ref).abs() / size).max().item() < TOL
+
+
+# infinities and NaNs go where the f32 product takes them, and nowhere else
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(4, 100, 256), (70, 300, 256), (40, 64, 2048)])
+def test_dense_non_finite(dtype, m, n, k):
+    w, x = _make(m, n, k, dtype, 9)
+    w = w.abs().clamp_min(0.0078125).to(dtype)  # no zeros: inf * w stays inf
+    w[:, 4] = 1.0  # exact in one part: the lower parts are zero
+    x[0, 4] = float("inf")
+    x[1, 9] = float("-inf")
+    x[2, 11] = float("nan")
+    w[5, 20] = float("inf")
+    ql = QuantLinear.from_dense(w)
+    y, ref = ql.forward(x), (x.double() @ w.double().t()).float()
+    assert torch.equal(y.isnan(), ref.isnan())
+    assert torch.equal(y.isinf(), ref.isinf())
+    assert torch.equal(y[y.isinf()], ref[ref.isinf()])
+    fin = ref.isfinite()
+    assert ((y - ref)[fin].norm() / ref[fin].norm()).item() < TOL

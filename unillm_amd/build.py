@@ -25,8 +25,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCES = ["capi.hip", "weights.hip", "gemv.hip", "decode.hip", "prefill.hip", "attention.hip",
            "dense.hip"]
-# the dense (F32 / F16 / BF16) weights' f32 GEMM
-LIBS = ["-L/opt/rocm/lib", "-lrocblas", "-Wl,-rpath,/opt/rocm/lib"]
+LIBS = []  # libraries the link adds besides HIP's own
 HOST_SOURCES = ["gguf.cpp", "unillm_host.cpp"]
 HOST_LIB = os.path.join(HERE, "libunillm_host.so")
 HOST_TEST = os.path.join(os.path.dirname(HERE), "tests", "cpp", "test_host")

@@ -149,9 +149,11 @@ int alloc_weight(int qtype, int64_t n, int64_t k, QWeight** out) {
     w->n = n;
     w->k = k;
     w->kb = is_dense(qtype) ? 0 : k / QK;
-    w->row_bytes = is_dense(qtype) ? 4 * k : row_bytes_for(w->qtype, w->kb);
+    w->row_bytes = is_dense(qtype) ? dense_row_bytes(qtype, k) : row_bytes_for(w->qtype, w->kb);
     // + a 256-byte tail slot for the scale reduction run at create
-    w->bytes = (((size_t)n * (size_t)w->row_bytes + 255) & ~(size_t)255) + 256;
+    const size_t held = (size_t)n * (size_t)w->row_bytes +
+                        (is_dense(qtype) ? dense_extra_bytes(qtype, n) : 0);
+    w->bytes = ((held + 255) & ~(size_t)255) + 256;
     void* mem = nullptr;
     hipError_t e = hipMalloc(&mem, w->bytes);
     if (e != hipSuccess) {
@@ -178,7 +180,7 @@ int finish_weight(QWeight* w, hipStream_t s) {
     uint32_t* slot = reinterpret_cast<uint32_t*>(w->base + w->bytes - 256);
     uint32_t bits[2] = {0, 0};
     hipError_t e;
-    if (is_dense(w->qtype)) {  // f32 rows: no scales to range
+    if (is_dense(w->qtype)) {  // plain values: no scales to range
         w->f16_exp = 0;
         if ((e = hipStreamSynchronize(s)) != hipSuccess) return fail_hip(e, "weight upload");
         return UNILLM_OK;
@@ -395,7 +397,7 @@ int fail_launch(hipError_t e, const std::string& what) {
 }
 
 // A dense weight's call: the layer norm (if any) into the stream's workspace (slot 0),
-// the f32 GEMM, and for SwiGLU the product into slot 1 and the elementwise pass.
+// the f32 product, and for SwiGLU the product into slot 1 and the elementwise pass.
 int dense_impl(const unillm_qweight* w, const float* x, int64_t m, float* y, int path,
                hipStream_t s, int epi, const NormArgs& norm, const std::string& what,
                void* fixed_ws) {
@@ -404,16 +406,9 @@ int dense_impl(const unillm_qweight* w, const float* x, int64_t m, float* y, int
                     what + ": a dense (F32 / F16 / BF16) weight takes the dense path only");
     if (fixed_ws)
         return fail(UNILLM_ERR_UNSUPPORTED,
-                    what + ": the no-allocation entry point takes quantized weights only "
-                           "(the dense path's GEMM library)");
-    if (m > (int64_t)INT32_MAX)
-        return fail(UNILLM_ERR_INVALID_ARG, what + ": m too large for the f32 GEMM");
+                    what + ": the no-allocation entry point takes quantized weights only");
     hipError_t e = hipSuccess;
-    auto failed = [&](const std::string& where) {
-        const std::string d = dense_error();
-        if (e == hipErrorUnknown && !d.empty()) return fail(UNILLM_ERR_HIP, what + ": " + d);
-        return fail_launch(e, what + ": " + where);
-    };
+    auto failed = [&](const std::string& where) { return fail_launch(e, what + ": " + where); };
     if (norm.gamma) {
         void* xn = nullptr;
         if ((e = stream_workspace(s, (size_t)m * (size_t)w->k * sizeof(float), &xn, 0)) != hipSuccess)
@@ -429,7 +424,7 @@ int dense_impl(const unillm_qweight* w, const float* x, int64_t m, float* y, int
             return failed("workspace");
         out = static_cast<float*>(ws);
     }
-    if ((e = launch_dense(*w, x, m, out, s, epi == kEpiAdd)) != hipSuccess) return failed("f32 GEMM");
+    if ((e = launch_dense(*w, x, m, out, s, epi == kEpiAdd)) != hipSuccess) return failed("dense product");
     if (out != y && (e = launch_swiglu(out, m, w->n / 2, y, s)) != hipSuccess)
         return failed("SwiGLU launch");
     return UNILLM_OK;
@@ -593,11 +588,11 @@ int unillm_hip_qmatmul_reserve(const unillm_qweight* w, int64_t m, int swiglu, v
     if (int rc = ensure_init()) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (is_dense(w->qtype)) {
-        // the f32 GEMM's handle, slot 0 (a fused norm's rows), slot 1 (SwiGLU's product)
+        // slot 0 (a fused norm's rows), slot kDenseSlot (x in parts, split-k slabs),
+        // slot 1 (SwiGLU's product)
         void* p = nullptr;
-        hipError_t e = dense_prepare(s);
-        if (e == hipSuccess)
-            e = stream_workspace(s, (size_t)m * (size_t)w->k * sizeof(float), &p, 0);
+        hipError_t e = stream_workspace(s, (size_t)m * (size_t)w->k * sizeof(float), &p, 0);
+        if (e == hipSuccess) e = stream_workspace(s, dense_workspace_bytes(*w, m), &p, kDenseSlot);
         if (e == hipSuccess && swiglu)
             e = stream_workspace(s, (size_t)m * (size_t)w->n * sizeof(float), &p, 1);
         return e == hipSuccess ? UNILLM_OK : fail_launch(e, "reserve");
@@ -638,8 +633,7 @@ int unillm_hip_dequant(const unillm_qweight* w, float* out_dev, void* stream) {
     if (!aligned16(out_dev)) return fail(UNILLM_ERR_INVALID_ARG, "out must be 16-byte aligned");
     if (int rc = ensure_init()) return rc;
     hipError_t e = is_dense(w->qtype)
-                       ? hipMemcpyAsync(out_dev, w->base, (size_t)w->n * (size_t)w->k * sizeof(float),
-                                        hipMemcpyDeviceToDevice, static_cast<hipStream_t>(stream))
+                       ? launch_dense_widen(*w, out_dev, static_cast<hipStream_t>(stream))
                        : launch_dequant(*w, out_dev, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? UNILLM_OK : fail_hip(e, "dequant launch");
 }

@@ -4,32 +4,124 @@
 // tensor, and its forward multiplies in f32 (the Tensor variant: x.matmul(w.t())).
 // The reference's loader wraps every *_proj.weight / lm_head.weight tensor in a
 // QMatMul whatever its GGML type (crates/runtime/src/weight_loader_core.rs:554-571),
-// so a GGUF with F16 projections takes this variant.  Here such a weight is held as
-// f32 rows [n][k] (F16 and BF16 widen exactly, as candle's dequantize does) and the
-// product is one f32 GEMM through rocBLAS: there is no dequant to fuse, so a plain
-// library GEMM is the kernel.  The epilogues keep their meaning: the residual add is
-// the GEMM's beta = 1, the layer norm a row pass into the stream's workspace first,
-// SwiGLU the elementwise pass after the product.
+// so a GGUF with F16 projections takes this variant.  A weight is held in its own type
+// (a widening to f32 would double the bytes a decode step streams) as rows of
+// row_bytes, k padded with zeros to a multiple of 64 (an F16 row times the power of two
+// that puts its largest magnitude in [2^14, 2^15): exact, and undone on the output by the
+// factors behind the rows), and the product is f32:
+//
+//  - dense_gemv_kernel (m <= 8 where x fits in LDS): the weights widen in registers
+//    and every product is an f32 FMA.  Bound by the weight stream.
+//  - dense_gemm_kernel: 16-bit matrix cores at f32's precision.  x is split exactly
+//    into three 16-bit parts (xsplit_kernel), an F16 or BF16 weight is one part as it
+//    stands, an F32 weight is split in registers into three bf16 parts; the products
+//    of parts down to 2^-16 of the leading one are summed in f32 (3 per weight for F16
+//    and BF16, which is all of them; 6 for F32: the three left out are below 2^-24).
+//    gfx950's 16-bit matrix cores run 16 times its f32 ones, so 3 or 6 of them are
+//    still 5 or 2.7 times faster, and the error against f64 is below an f32 GEMM's,
+//    which rounds once a k (profiles/dense_weights.md has both).
+//
+// Both give the same bits on every call (no atomics; split-k slabs add in order), and
+// an F16 or BF16 weight on the GEMV the same bits as its widened F32 copy.  A
+// non-finite x or weight makes 0 * inf terms in the split products, and scaled F16 rows
+// can overflow where the product does not: an output that comes out non-finite is
+// recomputed as a plain f32 dot (dense_dot), so infinities propagate as f32 products
+// would.
+#include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
-#include <rocblas/rocblas.h>
 
+#include <algorithm>
 #include <mutex>
-#include <string>
 
 #include "internal.hpp"
+#include "lds.hpp"
 
 namespace unillm {
 namespace {
 
-// dst[i] = src[i] widened to f32 (F16: the half value; BF16: the upper 16 bits of an f32)
-__global__ __launch_bounds__(256) void widen_kernel(const uint16_t* __restrict__ src,
-                                                    float* __restrict__ dst, int64_t count,
-                                                    int bf16) {
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kKPad = 64;  // rows are padded with zeros to a multiple of this many weights
+
+int64_t padded_k(int64_t k) { return (k + kKPad - 1) / kKPad * kKPad; }
+
+// an F16 weight's row factors, behind its rows
+float* dense_wsc(const QWeight& w) {
+    return w.qtype == UNILLM_QTYPE_F16
+               ? reinterpret_cast<float*>(w.base + (size_t)w.n * (size_t)w.row_bytes)
+               : nullptr;
+}
+
+// ---- upload, dequant, layer norm ---------------------------------------------------------
+
+// dst row r (row_bytes) <- src row r (k elements of ES bytes, ES-aligned); the padding
+// was zeroed when the weight was allocated
+template <class T>
+__global__ __launch_bounds__(256) void dense_upload_kernel(const T* __restrict__ src,
+                                                           uint8_t* __restrict__ dst, int64_t n,
+                                                           int64_t k, int64_t row_bytes) {
+    const int64_t count = n * k;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const uint16_t v = src[i];
-        dst[i] = bf16 ? __uint_as_float((uint32_t)v << 16) : __half2float(__ushort_as_half(v));
+         i += (int64_t)gridDim.x * blockDim.x)
+        reinterpret_cast<T*>(dst + i / k * row_bytes)[i % k] = src[i];
+}
+
+// the same for F16, each row scaled (wsc[row] <- the undoing factor); a workgroup a row
+__global__ __launch_bounds__(256) void dense_upload_f16_kernel(const uint16_t* __restrict__ src,
+                                                               uint8_t* __restrict__ dst,
+                                                               int64_t k, int64_t row_bytes,
+                                                               float* __restrict__ wsc) {
+    __shared__ uint32_t red[4];
+    const uint16_t* sr = src + (int64_t)blockIdx.x * k;
+    uint16_t* dr = reinterpret_cast<uint16_t*>(dst + (int64_t)blockIdx.x * row_bytes);
+    uint32_t mx = 0;  // largest finite magnitude (its bits order like the value)
+    for (int64_t i = threadIdx.x; i < k; i += 256) {
+        const uint32_t a = sr[i] & 0x7FFFu;
+        if (a < 0x7C00u) mx = max(mx, a);
     }
+    for (int d = 32; d > 0; d >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, d));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    mx = max(max(red[0], red[1]), max(red[2], red[3]));
+    int e = 15;
+    if (mx) (void)frexpf(__half2float(__ushort_as_half((uint16_t)mx)), &e);
+    const int sh = max(15 - e, 0);  // never down: nothing is rounded
+    const float up = ldexpf(1.0f, sh);
+    for (int64_t i = threadIdx.x; i < k; i += 256)
+        dr[i] = __half_as_ushort(__float2half(__half2float(__ushort_as_half(sr[i])) * up));
+    if (threadIdx.x == 0) wsc[blockIdx.x] = ldexpf(1.0f, -sh);
+}
+
+// weight i of a row (F16: scaled back by its row's factor)
+template <int QT>
+__device__ __forceinline__ float widen1(const uint8_t* row, int64_t i, float wsc) {
+    if constexpr (QT == UNILLM_QTYPE_F32) return reinterpret_cast<const float*>(row)[i];
+    const uint16_t v = reinterpret_cast<const uint16_t*>(row)[i];
+    if constexpr (QT == UNILLM_QTYPE_F16) return __half2float(__ushort_as_half(v)) * wsc;
+    return __uint_as_float((uint32_t)v << 16);
+}
+
+// the factor of a row (F16), 1 otherwise
+template <int QT>
+__device__ __forceinline__ float row_factor(const float* wsc, int64_t row) {
+    if constexpr (QT == UNILLM_QTYPE_F16) return wsc[row];
+    return 1.0f;
+}
+
+// out[n, k] f32 <- the weight's values, widened exactly
+template <int QT>
+__global__ __launch_bounds__(256) void dense_widen_kernel(const uint8_t* __restrict__ base,
+                                                          int64_t row_bytes,
+                                                          const float* __restrict__ wsc,
+                                                          float* __restrict__ out, int64_t n,
+                                                          int64_t k) {
+    const int64_t count = n * k;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
+         i += (int64_t)gridDim.x * blockDim.x)
+        out[i] = widen1<QT>(base + i / k * row_bytes, i % k, row_factor<QT>(wsc, i / k));
 }
 
 // out[r] = (x[r] - mean) / sqrt(var + eps) * gamma (+ beta), one workgroup a row: the
@@ -62,52 +154,609 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict_
         orow[i] = (xr[i] - mean) / sd * norm.gamma[i] + (norm.beta ? norm.beta[i] : 0.0f);
 }
 
-// One rocBLAS handle per process (the library uses one device), with a workspace
-// of its own so that no call allocates (HIP-graph capture records no allocation);
-// atomics off, so a product is the same bits every call.
-constexpr size_t kBlasWorkspace = (size_t)64 << 20;
-std::mutex g_blas_mutex;
-rocblas_handle g_blas = nullptr;
-void* g_blas_ws = nullptr;
-thread_local std::string g_dense_error;
+// The plain f32 dot of one output: what an output that came out non-finite is
+// recomputed with.
+template <int QT>
+__device__ __noinline__ float dense_dot(const float* x, const uint8_t* row, int64_t k, float wsc) {
+    float s = 0.0f;
+    for (int64_t i = 0; i < k; ++i) s = fmaf(x[i], widen1<QT>(row, i, wsc), s);
+    return s;
+}
 
-const char* blas_status(rocblas_status st) { return rocblas_status_to_string(st); }
+__device__ __forceinline__ bool non_finite(float v) {
+    return (__float_as_uint(v) & 0x7F800000u) == 0x7F800000u;
+}
 
-// The handle, created on first use (never while `s` is being captured).
-hipError_t blas_handle(hipStream_t s, rocblas_handle* out) {
-    if (!g_blas) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        hipError_t e = hipStreamIsCapturing(s, &cs);
-        if (e != hipSuccess) return e;
-        if (cs != hipStreamCaptureStatusNone) {
-            g_dense_error = "the f32 GEMM's handle is created on first use, which cannot happen "
-                            "while the stream is being captured; reserve before capture";
-            return hipErrorStreamCaptureUnsupported;
-        }
-        rocblas_handle h = nullptr;
-        rocblas_status st = rocblas_create_handle(&h);
-        if (st != rocblas_status_success) {
-            g_dense_error = std::string("rocblas_create_handle: ") + blas_status(st);
-            return hipErrorUnknown;
-        }
-        void* ws = nullptr;
-        if ((e = hipMalloc(&ws, kBlasWorkspace)) != hipSuccess) {
-            (void)rocblas_destroy_handle(h);
-            return e;
-        }
-        if ((st = rocblas_set_workspace(h, ws, kBlasWorkspace)) != rocblas_status_success ||
-            (st = rocblas_set_atomics_mode(h, rocblas_atomics_not_allowed)) !=
-                rocblas_status_success) {
-            g_dense_error = std::string("rocBLAS handle set-up: ") + blas_status(st);
-            (void)rocblas_destroy_handle(h);
-            (void)hipFree(ws);
-            return hipErrorUnknown;
-        }
-        g_blas = h;
-        g_blas_ws = ws;
+// ---- GEMV, m <= 8 ------------------------------------------------------------------------
+// One workgroup of 16 waves a CU; a wave takes rows wave, wave + W, ...; lane l holds
+// the 8 consecutive weights of groups l, l + 64, ... of the row (one 16-byte load; two
+// for F32), U groups requested ahead of the ones being multiplied, so 128 bytes a lane
+// stay in flight across row ends.  x sits in LDS as two planes of 4 floats a group:
+// every read is 16 consecutive bytes a lane, free of bank conflicts.  Bound by the
+// weight stream: F16 k4096 n11008 (90 MB) 17.0 us a call (5.3 TB/s), against 228 us as
+// an f32 library GEMM of rows widened to f32.
+constexpr int kGemvThreads = 1024;
+constexpr int64_t kGemvLds = 128 << 10;
+
+template <int QT>
+struct Row8 {  // 8 weights as loaded
+    static constexpr int L = QT == UNILLM_QTYPE_F32 ? 2 : 1;
+    u32x4 v[L];
+};
+
+template <int QT>
+__device__ __forceinline__ Row8<QT> load8(const uint8_t* row, int g) {
+    Row8<QT> r;
+#pragma unroll
+    for (int i = 0; i < Row8<QT>::L; ++i)
+        r.v[i] = *reinterpret_cast<const u32x4*>(row + ((int64_t)g * Row8<QT>::L + i) * 16);
+    return r;
+}
+
+template <int QT>
+__device__ __forceinline__ float elem8(const Row8<QT>& r, int e) {
+    if constexpr (QT == UNILLM_QTYPE_F32) return __uint_as_float(r.v[e / 4][e % 4]);
+    const uint32_t u = r.v[0][e / 2];
+    if constexpr (QT == UNILLM_QTYPE_F16)
+        return (float)__builtin_bit_cast(_Float16, (uint16_t)(e % 2 ? u >> 16 : u & 0xFFFFu));
+    return __uint_as_float(e % 2 ? u & 0xFFFF0000u : u << 16);
+}
+
+// M: the token count the code is built for (m <= M; x past m is zero and not stored)
+template <int QT, int M>
+__global__ __launch_bounds__(kGemvThreads, 1) void dense_gemv_kernel(
+    const uint8_t* __restrict__ base, int64_t row_bytes, const float* __restrict__ wsc,
+    const float* __restrict__ x, int m, int64_t n, int k, float* __restrict__ y, int add) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    f32x4* xs = reinterpret_cast<f32x4*>(smem);  // [M][2][G]
+    const int G = (k + 7) / 8;
+    const int lane = threadIdx.x & 63;
+    const int64_t wave = (int64_t)(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
+    const int64_t waves = (int64_t)(kGemvThreads / 64) * gridDim.x;
+    constexpr int U = QT == UNILLM_QTYPE_F32 ? 4 : M <= 4 ? 8 : 4;
+    const int T = (G + 64 * U - 1) / (64 * U);  // batches of U groups a lane in a row
+
+    auto request = [&](int64_t row, int t, Row8<QT>(&r)[U]) {
+        const uint8_t* p = base + row * row_bytes;
+#pragma unroll
+        for (int u = 0; u < U; ++u) r[u] = load8<QT>(p, min((t * U + u) * 64 + lane, G - 1));
+    };
+    // the first batch is in flight while x is staged
+    Row8<QT> cur[U], nxt[U];
+    if (wave < n) request(wave, 0, cur);
+    float* xf = reinterpret_cast<float*>(smem);
+    for (int i = threadIdx.x; i < M * G * 8; i += kGemvThreads) {
+        const int t = i / (G * 8), c = i % (G * 8);
+        // plane (c / 4) % 2, group c / 8
+        xf[((t * 2 + (c / 4) % 2) * G + c / 8) * 4 + c % 4] =
+            t < m && c < k ? x[(int64_t)t * k + c] : 0.0f;
     }
-    *out = g_blas;
-    return hipSuccess;
+    __syncthreads();
+
+    for (int64_t row = wave; row < n; row += waves) {
+        float acc[M];
+#pragma unroll
+        for (int t = 0; t < M; ++t) acc[t] = 0.0f;
+        for (int b = 0; b < T; ++b) {
+            const bool last = b + 1 == T;
+            const int64_t nrow = last ? row + waves : row;
+            if (nrow < n) request(nrow, last ? 0 : b + 1, nxt);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int g = (b * U + u) * 64 + lane;
+                if (g < G) {
+#pragma unroll
+                    for (int t = 0; t < M; ++t) {
+                        const f32x4 lo = xs[(t * 2) * G + g], hi = xs[(t * 2 + 1) * G + g];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[t] = fmaf(elem8<QT>(cur[u], e), lo[e], acc[t]);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            acc[t] = fmaf(elem8<QT>(cur[u], 4 + e), hi[e], acc[t]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) cur[u] = nxt[u];
+        }
+#pragma unroll
+        for (int t = 0; t < M; ++t) {
+            float s = acc[t];
+            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+            if (lane == 0 && t < m) {
+                if constexpr (QT == UNILLM_QTYPE_F16) {
+                    const float f = wsc[row];
+                    s *= f;
+                    if (non_finite(s)) s = dense_dot<QT>(x + (int64_t)t * k, base + row * row_bytes, k, f);
+                }
+                float* dst = y + (int64_t)t * n + row;
+                *dst = add ? *dst + s : s;
+            }
+        }
+    }
+}
+
+int64_t gemv_m(int64_t m) { return m <= 2 ? m : m <= 4 ? 4 : 8; }
+int64_t gemv_lds(int64_t m, int64_t k) { return gemv_m(m) * ((k + 7) / 8) * 32; }
+
+// x in LDS: 8 tokens take k <= 4096, 4 take 8192, one 32768
+bool dense_gemv_supports(const QWeight& w, int64_t m) {
+    return m <= 8 && gemv_lds(m, w.k) <= kGemvLds;
+}
+
+template <int QT, int M>
+hipError_t launch_gemv_m(const QWeight& w, const float* x, int64_t m, float* y, hipStream_t s,
+                         int add) {
+    static const bool attr = hipFuncSetAttribute((const void*)dense_gemv_kernel<QT, M>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 (int)kGemvLds) == hipSuccess;
+    if (!attr) return hipErrorInvalidValue;
+    // wave numbers run across workgroups, so few rows still spread over the CUs
+    const int blocks = (int)std::min<int64_t>(device_info().cu_count, w.n);
+    dense_gemv_kernel<QT, M><<<blocks, kGemvThreads, gemv_lds(m, w.k), s>>>(
+        w.base, w.row_bytes, dense_wsc(w), x, (int)m, w.n, (int)w.k, y, add);
+    return hipGetLastError();
+}
+
+template <int QT>
+hipError_t launch_gemv_qt(const QWeight& w, const float* x, int64_t m, float* y, hipStream_t s,
+                          int add) {
+    switch (gemv_m(m)) {
+        case 1: return launch_gemv_m<QT, 1>(w, x, m, y, s, add);
+        case 2: return launch_gemv_m<QT, 2>(w, x, m, y, s, add);
+        case 4: return launch_gemv_m<QT, 4>(w, x, m, y, s, add);
+        default: return launch_gemv_m<QT, 8>(w, x, m, y, s, add);
+    }
+}
+
+// ---- x in three 16-bit parts -------------------------------------------------------------
+// xp[p][m][kp]: x = part 0 + part 1 + part 2 exactly (rows padded with zeros to kp).
+// bf16 parts (BF16 and F32 weights): each part the upper 16 bits of what is left (8
+// significant bits each, 24 in all; truncation never overflows).  f16 parts (F16
+// weights): the row is first scaled by the power of two that puts its largest magnitude
+// in [2^14, 2^15), undone on the output by rs[row]; each part is what is left rounded to
+// f16 (11 bits each, so the parts hold 2^-40 of the row's largest value).  A non-finite
+// value keeps its kind in part 0, the others zero.  One workgroup a row; bound by its
+// bytes (4 in, 6 out an element).
+template <bool F16P>
+__global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x, int64_t k,
+                                                     int64_t kp, uint16_t* __restrict__ xp,
+                                                     int64_t plane, float* __restrict__ rs) {
+    const float* xr = x + (int64_t)blockIdx.x * k;
+    uint16_t* o = xp + (int64_t)blockIdx.x * kp;
+    const int tid = threadIdx.x;
+    float up = 1.0f;
+    if constexpr (F16P) {
+        __shared__ uint32_t red[4];
+        uint32_t mx = 0;  // largest finite magnitude (its bits order like the value)
+        for (int64_t i = tid; i < k; i += 256) {
+            const uint32_t a = __float_as_uint(xr[i]) & 0x7FFFFFFFu;
+            if (a < 0x7F800000u) mx = max(mx, a);
+        }
+        for (int d = 32; d > 0; d >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, d));
+        if ((tid & 63) == 0) red[tid >> 6] = mx;
+        __syncthreads();
+        mx = max(max(red[0], red[1]), max(red[2], red[3]));
+        int e = 0;
+        if (mx) (void)frexpf(__uint_as_float(mx), &e);
+        // |x| < 2^e; the factors stay normal f32 (a row below 2^-111 keeps fewer bits)
+        const int sh = min(max(15 - e, -113), 126);
+        up = ldexpf(1.0f, sh);
+        if (tid == 0) rs[blockIdx.x] = ldexpf(1.0f, -sh);
+    }
+    for (int64_t i = tid; i < kp; i += 256) {
+        const float v = i < k ? xr[i] : 0.0f;
+        uint16_t p0, p1 = 0, p2 = 0;
+        const bool finite = (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u;
+        if constexpr (F16P) {
+            const float s = v * up;
+            const _Float16 h0 = (_Float16)s;
+            p0 = __builtin_bit_cast(uint16_t, h0);
+            if (finite) {
+                const float r1 = s - (float)h0;
+                const _Float16 h1 = (_Float16)r1;
+                const float r2 = r1 - (float)h1;
+                p1 = __builtin_bit_cast(uint16_t, h1);
+                p2 = __builtin_bit_cast(uint16_t, (_Float16)r2);
+            }
+        } else {
+            const uint32_t u = __float_as_uint(v);
+            p0 = (uint16_t)(u >> 16);
+            if (finite) {
+                const float r1 = v - __uint_as_float(u & 0xFFFF0000u);
+                const uint32_t u1 = __float_as_uint(r1);
+                const float r2 = r1 - __uint_as_float(u1 & 0xFFFF0000u);
+                p1 = (uint16_t)(u1 >> 16);
+                p2 = (uint16_t)(__float_as_uint(r2) >> 16);
+            } else if (u & 0x007FFFFFu) {
+                p0 |= 0x40;  // a NaN whose upper mantissa bits are zero stays a NaN
+            }
+        }
+        o[i] = p0;
+        o[plane + i] = p1;
+        o[2 * plane + i] = p2;
+    }
+}
+
+// ---- GEMM --------------------------------------------------------------------------------
+// Tile BM x BN, k in steps of 32, eight waves in a 2 x 4 grid of (BM / 2) x (BN / 4)
+// blocks of 16 x 16 x 32 MFMAs.  Operands reach LDS by direct global -> LDS loads
+// through a ring of 4 stages; a step's first fragments are read during the
+// last MFMAs of the step before, so a step starts straight into its MFMAs:
+//   A  [3 parts][BM rows][64 B], the 16-byte chunk c of row r in slot c ^ f(r / 4 % 4),
+//      f = 0 3 2 1: the 16 lanes that an LDS read serves together touch all banks once;
+//   B  [BN rows][64 B], the same (F32: [BN][128 B], chunk c in slot c ^ r % 8).
+// Bound by the matrix cores at three products a weight (BF16 m512 k4096 n11008: 158 us a
+// call, 293 TFLOP/s of f32 product, against 451 us as an f32 library GEMM; 172 tiles on 256
+// CUs) and by the weight stream and the split's fixed cost at few rows (m16: 35 us).
+template <int QT, int BM>
+struct DTile {
+    static constexpr bool F32W = QT == UNILLM_QTYPE_F32;
+    static constexpr int BN = F32W ? 128 : 256;
+    static constexpr int NP = 3;
+    static constexpr int A = NP * BM * 64;
+    static constexpr int B = BN * (F32W ? 128 : 64);
+    static constexpr int STAGE = A + B;
+    static constexpr int STAGES = 4;
+    static constexpr int BYTES = STAGES * STAGE;
+    static constexpr int AI = A / 1024, BI = B / 1024;     // direct loads a stage
+    static constexpr int AW = (AI + 7) / 8, BW = BI / 8;   // a wave
+    static constexpr int DMA = AW + BW;
+    static constexpr int TI = BM / 32, TJ = BN / 64;       // 16 x 16 tiles a wave
+};
+
+__device__ __forceinline__ uint32_t swz64(uint32_t row) { return (4u - ((row >> 2) & 3u)) & 3u; }
+
+template <bool F16P>
+__device__ __forceinline__ f32x4 mfma_parts(u32x4 a, u32x4 b, f32x4 c) {
+    if constexpr (F16P)
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                      __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                       __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// two f32 (as bits) -> their upper halves packed, lo in the low half
+__device__ __forceinline__ uint32_t pack_hi(uint32_t lo, uint32_t hi) {
+    return __builtin_amdgcn_perm(hi, lo, 0x07060302u);
+}
+
+// 8 f32 weights -> three bf16 parts (truncation, as xsplit_kernel's; an infinity's or a
+// NaN's lower parts come out NaN: the output is recomputed)
+__device__ __forceinline__ void split8(const u32x4 (&w)[2], u32x4 (&p)[3]) {
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        const uint32_t a = w[h / 2][2 * (h % 2)], b = w[h / 2][2 * (h % 2) + 1];
+        p[0][h] = pack_hi(a, b);
+        const float a1 = __uint_as_float(a) - __uint_as_float(a & 0xFFFF0000u);
+        const float b1 = __uint_as_float(b) - __uint_as_float(b & 0xFFFF0000u);
+        const uint32_t ua = __float_as_uint(a1), ub = __float_as_uint(b1);
+        p[1][h] = pack_hi(ua, ub);
+        const float a2 = a1 - __uint_as_float(ua & 0xFFFF0000u);
+        const float b2 = b1 - __uint_as_float(ub & 0xFFFF0000u);
+        p[2][h] = pack_hi(__float_as_uint(a2), __float_as_uint(b2));
+    }
+}
+
+template <int QT, int BM>
+__global__ __launch_bounds__(512, 1) void dense_gemm_kernel(
+    const uint8_t* __restrict__ base, int64_t row_bytes, const float* __restrict__ wsc,
+    const uint16_t* __restrict__ xp, int64_t plane, int64_t kp, const float* __restrict__ rs, const float* __restrict__ x,
+    int64_t k, float* __restrict__ y, int64_t M, int64_t N, int tiles_n, int tiles, int units_pad,
+    int S, int add, float* __restrict__ part) {
+    using D = DTile<QT, BM>;
+    constexpr bool F16P = QT == UNILLM_QTYPE_F16;
+    constexpr int TI = D::TI, TJ = D::TJ, NP = D::NP;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+
+    // unit u = (k slice sp, m-tile, n-tile), a contiguous run of units per XCD
+    const int u = (blockIdx.x % 8) * (units_pad / 8) + blockIdx.x / 8;
+    if (u >= tiles * S) return;
+    const int sp = u / tiles, t = u % tiles;
+    const int64_t m0 = (int64_t)(t / tiles_n) * BM, n0 = (int64_t)(t % tiles_n) * D::BN;
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rw = wv / 4, cw = wv % 4;
+    // this slice's steps, always whole pairs
+    const int kpairs = (int)(kp / kKPad);
+    const int ks0 = 2 * (int)((int64_t)sp * kpairs / S);
+    const int nks = 2 * (int)((int64_t)(sp + 1) * kpairs / S) - ks0;
+
+    // direct-load sources at step 0 (rows past the end re-read the last row)
+    const uint8_t* asrc[D::AW];
+    const uint8_t* bsrc[D::BW];
+    uint32_t adst[D::AW], bdst[D::BW];
+#pragma unroll
+    for (int q = 0; q < D::AW; ++q) {
+        const int i = (wv * D::AW + q) % D::AI;  // an uneven split loads a part twice
+        const int r = i % (BM / 16) * 16 + lane / 4;
+        const int c = (lane % 4) ^ swz64(r);
+        asrc[q] = reinterpret_cast<const uint8_t*>(
+            xp + (i / (BM / 16)) * plane + min(m0 + r, M - 1) * kp + c * 8);
+        adst[q] = i * 1024;
+    }
+#pragma unroll
+    for (int q = 0; q < D::BW; ++q) {
+        const int i = wv * D::BW + q;
+        const int r = D::F32W ? i * 8 + lane / 8 : i * 16 + lane / 4;
+        const int c = D::F32W ? (lane % 8) ^ (r % 8) : (lane % 4) ^ swz64(r);
+        bsrc[q] = base + min(n0 + r, N - 1) * row_bytes + c * 16;
+        bdst[q] = D::A + i * 1024;
+    }
+    auto issue = [&](int j) {  // the direct loads of step ks0 + j
+        uint8_t* st = smem + (j % D::STAGES) * D::STAGE;
+        const int64_t ko = (int64_t)(ks0 + j) * 64;
+#pragma unroll
+        for (int q = 0; q < D::AW; ++q) dma16(asrc[q] + ko, st + adst[q]);
+#pragma unroll
+        for (int q = 0; q < D::BW; ++q) dma16(bsrc[q] + (D::F32W ? 2 * ko : ko), st + bdst[q]);
+    };
+
+    // fragment offsets in a stage: A row (BM / 2) rw + 16 i + fr, B row (BN / 4) cw + 16 j + fr
+    const uint32_t g = lane / 16, fr = lane % 16;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+    const uint32_t aoff = lds0 + ((BM / 2) * rw + fr) * 64 + (g ^ swz64(fr)) * 16;
+    const uint32_t brow = (D::BN / 4) * cw + fr;
+    const uint32_t boff0 = lds0 + D::A + (D::F32W ? brow * 128 + ((2 * g) ^ (fr % 8)) * 16
+                                                  : brow * 64 + (g ^ swz64(fr)) * 16);
+    const uint32_t boff1 = lds0 + D::A + brow * 128 + ((2 * g + 1) ^ (fr % 8)) * 16;
+
+    constexpr int BL = D::F32W ? 2 : 1;
+    struct Frags {
+        u32x4 a[NP];       // row tile 0
+        u32x4 b[TJ][BL];
+    };
+    auto read_first = [&](int j, Frags& f) {
+        const uint32_t st = (uint32_t)((j % D::STAGES) * D::STAGE);
+        constexpr_for<TJ>([&](auto J) {
+            f.b[J.value][0] = lds_read128<J.value * 16 * (D::F32W ? 128 : 64)>(st + boff0);
+            if constexpr (D::F32W) f.b[J.value][1] = lds_read128<J.value * 16 * 128>(st + boff1);
+        });
+        constexpr_for<NP>([&](auto P) { f.a[P.value] = lds_read128<P.value * BM * 64>(st + aoff); });
+    };
+    auto wait_first = [&](Frags& f) {
+        static_assert(TJ == 4 || (TJ == 2 && BL == 2), "fragments named below");
+        asm volatile("s_waitcnt lgkmcnt(0)"
+                     : "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.a[2]), "+v"(f.b[0][0]),
+                       "+v"(f.b[TJ == 4 ? 1 : 0][BL - 1]), "+v"(f.b[TJ == 4 ? 2 : 1][0]),
+                       "+v"(f.b[TJ - 1][BL - 1]));
+    };
+
+    f32x4 acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    f32x4 low[D::F32W ? TI : 1][D::F32W ? TJ : 1] = {};
+
+    // prologue: three stages in flight; step 0's first fragments read
+    constexpr int AHEAD = D::STAGES - 1;
+#pragma unroll
+    for (int d = 0; d < AHEAD; ++d)
+        if (d < nks) issue(d);
+    if (nks > 2) wait_vmcnt<2 * D::DMA>();
+    else wait_vmcnt<D::DMA>();
+    __builtin_amdgcn_s_barrier();
+    Frags f0, f1;
+    read_first(0, f0);
+    wait_first(f0);
+    // step j: wait for this wave's loads of step j + 1 and meet the others (so stage
+    // j + 1 is whole, and stage j - 1, whose slot step j + 3 takes, is no longer read)
+    auto step = [&](int j, Frags& f, Frags& nf) {
+        if (j + 2 < nks) wait_vmcnt<D::DMA>();
+        else wait_vmcnt<0>();
+        __builtin_amdgcn_s_barrier();
+        if (j + AHEAD < nks) issue(j + AHEAD);
+        const uint32_t st = (uint32_t)((j % D::STAGES) * D::STAGE);
+        u32x4 wb[TJ][NP];
+        if constexpr (D::F32W) {
+#pragma unroll
+            for (int q = 0; q < TJ; ++q) split8(f.b[q], wb[q]);
+        }
+        u32x4 a[2][NP];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) a[0][p] = f.a[p];
+        constexpr_for<TI>([&](auto I) {
+            constexpr int i = I.value;
+            // the reads may land in registers of products just consumed: keep the wait
+            // states after an MFMA that the compiler keeps before its own LDS reads
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_nop 7");
+            if constexpr (i + 1 < TI)
+                constexpr_for<NP>([&](auto P) {
+                    a[(i + 1) % 2][P.value] =
+                        lds_read128<P.value * BM * 64 + (i + 1) * 1024>(st + aoff);
+                });
+            else if (j + 1 < nks)
+                read_first(j + 1, nf);
+            __builtin_amdgcn_sched_barrier(0);  // (left free, the reads sink behind the MFMAs)
+            if constexpr (D::F32W) {
+                // the small products in sums of their own: one rounding of the large sum a
+                // 32 k, as with F16 and BF16 (in one sum, 1.3e-7 against 0.8e-7 for an f32
+                // GEMM at k 64)
+#pragma unroll
+                for (int q = 0; q < TJ; ++q) {
+                    low[i][q] = mfma_parts<false>(a[i % 2][2], wb[q][0], low[i][q]);
+                    acc[i][q] = mfma_parts<false>(a[i % 2][0], wb[q][0], acc[i][q]);
+                }
+#pragma unroll
+                for (int q = 0; q < TJ; ++q)
+                    low[i][q] = mfma_parts<false>(a[i % 2][0], wb[q][2], low[i][q]);
+#pragma unroll
+                for (int q = 0; q < TJ; ++q)
+                    low[i][q] = mfma_parts<false>(a[i % 2][1], wb[q][1], low[i][q]);
+#pragma unroll
+                for (int q = 0; q < TJ; ++q)
+                    low[i][q] = mfma_parts<false>(a[i % 2][1], wb[q][0], low[i][q]);
+#pragma unroll
+                for (int q = 0; q < TJ; ++q)
+                    low[i][q] = mfma_parts<false>(a[i % 2][0], wb[q][1], low[i][q]);
+            } else {
+#pragma unroll
+                for (int p = NP - 1; p >= 0; --p)
+#pragma unroll
+                    for (int q = 0; q < TJ; ++q)
+                        acc[i][q] = mfma_parts<F16P>(a[i % 2][p], f.b[q][0], acc[i][q]);
+            }
+            if constexpr (i + 1 < TI)
+                asm volatile("s_waitcnt lgkmcnt(0)"
+                             : "+v"(a[(i + 1) % 2][0]), "+v"(a[(i + 1) % 2][1]),
+                               "+v"(a[(i + 1) % 2][2]));
+            else if (j + 1 < nks)
+                wait_first(nf);
+        });
+    };
+    for (int j = 0; j < nks; j += 2) {
+        step(j, f0, f1);
+        step(j + 1, f1, f0);
+    }
+
+    if constexpr (D::F32W) {
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int q = 0; q < TJ; ++q) acc[i][q] += low[i][q];
+    }
+    // epilogue: lane holds rows 4 g + e, column fr of each 16 x 16 tile
+#pragma unroll
+    for (int q = 0; q < TJ; ++q) {
+        const int64_t col = n0 + (D::BN / 4) * cw + 16 * q + fr;
+        if (col >= N) continue;
+        const float wf = row_factor<QT>(wsc, col);
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int64_t row = m0 + (BM / 2) * rw + 16 * i + 4 * g + e;
+                if (row >= M) continue;
+                if (S > 1) {
+                    part[((int64_t)sp * M + row) * N + col] = acc[i][q][e];
+                    continue;
+                }
+                float v = acc[i][q][e];
+                if constexpr (F16P) v = v * wf * rs[row];
+                if (non_finite(v)) v = dense_dot<QT>(x + row * k, base + col * row_bytes, k, wf);
+                float* dst = y + row * N + col;
+                *dst = add ? *dst + v : v;
+            }
+    }
+}
+
+// y (+)= the S slabs of a split k in slice order (scaled back for F16)
+template <int QT>
+__global__ __launch_bounds__(256) void dense_sum_kernel(const float* __restrict__ part, int S,
+                                                        int64_t M, int64_t N,
+                                                        const float* __restrict__ rs,
+                                                        const uint8_t* __restrict__ base,
+                                                        int64_t row_bytes,
+                                                        const float* __restrict__ wsc,
+                                                        const float* __restrict__ x, int64_t k,
+                                                        int add, float* __restrict__ y) {
+    const int64_t MN = M * N;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < MN;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t row = i / N, col = i % N;
+        float v = part[i];
+        for (int sl = 1; sl < S; ++sl) v += part[sl * MN + i];
+        const float wf = row_factor<QT>(wsc, col);
+        if constexpr (QT == UNILLM_QTYPE_F16) v = v * wf * rs[row];
+        if (non_finite(v)) v = dense_dot<QT>(x + row * k, base + col * row_bytes, k, wf);
+        y[i] = add ? y[i] + v : v;
+    }
+}
+
+// Tile height and k split: the cheapest of 64- and 128-row tiles with k in up to 16
+// slices (at least 4 pairs of steps each, at most two workgroups a CU), by what a
+// workgroup's pair of steps was measured to take (64 / 128 rows: 1.5 / 2.35 us, F32 1.75
+// / 2.65) times the rounds over the CUs, plus a split's slabs written and read once
+// (3.5 TB/s) and the summing launch.  Measured against every choice, BF16 us a call:
+// k4096 n11008 m300 157.9 (128 rows, 129 tiles on 256 CUs) -> 107.0 (64 rows, 215),
+// m512 158.7 (128, one slice; 64: 199.8); k4096 n2048 m128 36.2 -> 29.1 (64 rows in 12).
+struct DensePlan {
+    int bm, S;
+};
+constexpr int64_t kDenseMaxSlices = 16;
+constexpr int64_t kDenseMaxRounds = 2;  // workgroups a CU when k is split
+
+int64_t dense_bn(const QWeight& w) { return w.qtype == UNILLM_QTYPE_F32 ? 128 : 256; }
+
+DensePlan dense_plan(const QWeight& w, int64_t m) {
+    const int64_t cus = device_info().cu_count, kpairs = padded_k(w.k) / kKPad;
+    const int64_t tiles_n = (w.n + dense_bn(w) - 1) / dense_bn(w);
+    const bool f32 = w.qtype == UNILLM_QTYPE_F32;
+    DensePlan best{128, 1};
+    int64_t least = INT64_MAX;
+    for (int bm : {64, 128}) {
+        const int64_t pair_ns = bm == 64 ? (f32 ? 1750 : 1500) : (f32 ? 2650 : 2350);
+        const int64_t tiles = (m + bm - 1) / bm * tiles_n;
+        for (int64_t S = 1; S <= kDenseMaxSlices; ++S) {
+            if (S > 1 && (S > kpairs / 4 || tiles * S > kDenseMaxRounds * cus)) break;
+            const int64_t rounds = (tiles * S + cus - 1) / cus;
+            int64_t ns = rounds * ((kpairs + S - 1) / S) * pair_ns;
+            if (S > 1) ns += 3000 + S * m * w.n * 8 / 3500;
+            if (ns < least) {
+                least = ns;
+                best = {bm, (int)S};
+            }
+        }
+    }
+    return best;
+}
+
+size_t up256(size_t b) { return (b + 255) / 256 * 256; }
+
+// x parts | row factors | slabs
+size_t dense_bytes(const QWeight& w, int64_t m, int64_t slab_rows) {
+    return up256((size_t)3 * m * padded_k(w.k) * 2) + up256((size_t)m * 4) +
+           (size_t)slab_rows * w.n * 4;
+}
+
+template <int QT, int BM>
+hipError_t launch_gemm_bm(const QWeight& w, const float* x, int64_t m, float* y, int S, void* ws,
+                          hipStream_t s, int add) {
+    using D = DTile<QT, BM>;
+    static const bool attr = hipFuncSetAttribute((const void*)dense_gemm_kernel<QT, BM>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 D::BYTES) == hipSuccess;
+    if (!attr) return hipErrorInvalidValue;
+    const int64_t kp = padded_k(w.k), plane = m * kp;
+    uint16_t* xp = static_cast<uint16_t*>(ws);
+    float* rs = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + up256((size_t)3 * plane * 2));
+    float* part = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(rs) + up256((size_t)m * 4));
+    xsplit_kernel<QT == UNILLM_QTYPE_F16><<<(unsigned)m, 256, 0, s>>>(x, w.k, kp, xp, plane, rs);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const int64_t tiles_n = (w.n + D::BN - 1) / D::BN;
+    const int64_t tiles = (m + BM - 1) / BM * tiles_n;
+    if (tiles * S > (int64_t)INT32_MAX - 8) return hipErrorInvalidValue;
+    const int units_pad = (int)((tiles * S + 7) / 8 * 8);
+    dense_gemm_kernel<QT, BM><<<units_pad, 512, D::BYTES, s>>>(
+        w.base, w.row_bytes, dense_wsc(w), xp, plane, kp, rs, x, w.k, y, m, w.n, (int)tiles_n, (int)tiles,
+        units_pad, S, add, part);
+    if ((e = hipGetLastError()) != hipSuccess || S == 1) return e;
+    const int blocks =
+        (int)std::min<int64_t>((m * w.n + 255) / 256, 8 * (int64_t)device_info().cu_count);
+    dense_sum_kernel<QT><<<blocks, 256, 0, s>>>(part, S, m, w.n, rs, w.base, w.row_bytes,
+                                                dense_wsc(w), x, w.k, add, y);
+    return hipGetLastError();
+}
+
+std::mutex g_dense_mutex;
+
+template <int QT>
+hipError_t launch_dense_qt(const QWeight& w, const float* x, int64_t m, float* y, hipStream_t s,
+                           int add) {
+    if (dense_gemv_supports(w, m)) return launch_gemv_qt<QT>(w, x, m, y, s, add);
+    const DensePlan p = dense_plan(w, m);
+    // a call's launches stay together: threads that share a stream share its workspace
+    std::lock_guard<std::mutex> lock(g_dense_mutex);
+    void* ws = nullptr;
+    const hipError_t e = stream_workspace(s, dense_bytes(w, m, p.S > 1 ? p.S * m : 0), &ws, kDenseSlot);
+    if (e != hipSuccess) return e;
+    return p.bm == 64 ? launch_gemm_bm<QT, 64>(w, x, m, y, p.S, ws, s, add)
+                      : launch_gemm_bm<QT, 128>(w, x, m, y, p.S, ws, s, add);
 }
 
 }  // namespace
@@ -118,16 +767,48 @@ bool is_dense(int qtype) {
 
 int dense_elem_bytes(int qtype) { return qtype == UNILLM_QTYPE_F32 ? 4 : 2; }
 
-std::string dense_error() { return g_dense_error; }
+size_t dense_extra_bytes(int qtype, int64_t n) {
+    return qtype == UNILLM_QTYPE_F16 ? (size_t)n * sizeof(float) : 0;
+}
+
+int64_t dense_row_bytes(int qtype, int64_t k) { return padded_k(k) * dense_elem_bytes(qtype); }
 
 hipError_t launch_dense_upload(const QWeight& w, const void* src, hipStream_t s) {
     const int64_t count = w.n * w.k;
-    if (w.qtype == UNILLM_QTYPE_F32)
-        return hipMemcpyAsync(w.base, src, (size_t)count * 4, hipMemcpyDeviceToDevice, s);
+    if (w.qtype == UNILLM_QTYPE_F16) {
+        dense_upload_f16_kernel<<<(unsigned)w.n, 256, 0, s>>>(static_cast<const uint16_t*>(src),
+                                                              w.base, w.k, w.row_bytes, dense_wsc(w));
+        return hipGetLastError();
+    }
+    if (w.k % kKPad == 0)
+        return hipMemcpyAsync(w.base, src, (size_t)count * dense_elem_bytes(w.qtype),
+                              hipMemcpyDeviceToDevice, s);
     const int blocks = (int)std::min<int64_t>((count + 255) / 256, 8 * device_info().cu_count);
-    widen_kernel<<<blocks, 256, 0, s>>>(static_cast<const uint16_t*>(src),
-                                        reinterpret_cast<float*>(w.base), count,
-                                        w.qtype == UNILLM_QTYPE_BF16);
+    if (w.qtype == UNILLM_QTYPE_F32)
+        dense_upload_kernel<<<blocks, 256, 0, s>>>(static_cast<const uint32_t*>(src), w.base, w.n,
+                                                   w.k, w.row_bytes);
+    else
+        dense_upload_kernel<<<blocks, 256, 0, s>>>(static_cast<const uint16_t*>(src), w.base, w.n,
+                                                   w.k, w.row_bytes);
+    return hipGetLastError();
+}
+
+hipError_t launch_dense_widen(const QWeight& w, float* out, hipStream_t s) {
+    const int64_t count = w.n * w.k;
+    const int blocks = (int)std::min<int64_t>((count + 255) / 256, 8 * device_info().cu_count);
+    switch (w.qtype) {
+        case UNILLM_QTYPE_F32:
+            dense_widen_kernel<UNILLM_QTYPE_F32><<<blocks, 256, 0, s>>>(w.base, w.row_bytes, dense_wsc(w), out,
+                                                               w.n, w.k);
+            break;
+        case UNILLM_QTYPE_F16:
+            dense_widen_kernel<UNILLM_QTYPE_F16><<<blocks, 256, 0, s>>>(w.base, w.row_bytes, dense_wsc(w), out,
+                                                               w.n, w.k);
+            break;
+        default:
+            dense_widen_kernel<UNILLM_QTYPE_BF16><<<blocks, 256, 0, s>>>(w.base, w.row_bytes, dense_wsc(w), out,
+                                                               w.n, w.k);
+    }
     return hipGetLastError();
 }
 
@@ -137,33 +818,26 @@ hipError_t launch_norm_rows(const float* x, int64_t m, int64_t k, const NormArgs
     return hipGetLastError();
 }
 
-hipError_t dense_prepare(hipStream_t s) {
-    std::lock_guard<std::mutex> lock(g_blas_mutex);
-    rocblas_handle h = nullptr;
-    return blas_handle(s, &h);
+// A bound for every call of up to m rows: the GEMV takes none; slices x rows of a split
+// are at most kDenseMaxSlices m, and at most 128 kDenseMaxRounds CUs / (column tiles).
+size_t dense_workspace_bytes(const QWeight& w, int64_t m) {
+    const int64_t tiles_n = (w.n + dense_bn(w) - 1) / dense_bn(w);
+    const int64_t rows =
+        padded_k(w.k) / kKPad < 8
+            ? 0  // never split
+            : std::min<int64_t>(kDenseMaxSlices * m,
+                                128 * kDenseMaxRounds * (int64_t)device_info().cu_count / tiles_n);
+    return dense_bytes(w, m, rows);
 }
 
-// y[m, n] = x[m, k] W^T (+ y when add): row-major y is the column-major n x m
-// matrix W x^T, i.e. sgemm(op(A) = A^T with A = W as a column-major k x n matrix,
-// B = x as a column-major k x m matrix).
 hipError_t launch_dense(const QWeight& w, const float* x, int64_t m, float* y, hipStream_t s,
                         int add) {
-    std::lock_guard<std::mutex> lock(g_blas_mutex);
-    rocblas_handle h = nullptr;
-    hipError_t e = blas_handle(s, &h);
-    if (e != hipSuccess) return e;
-    rocblas_status st = rocblas_set_stream(h, s);
-    const float alpha = 1.0f, beta = add ? 1.0f : 0.0f;
-    if (st == rocblas_status_success)
-        st = rocblas_sgemm(h, rocblas_operation_transpose, rocblas_operation_none, (rocblas_int)w.n,
-                           (rocblas_int)m, (rocblas_int)w.k, &alpha,
-                           reinterpret_cast<const float*>(w.base), (rocblas_int)w.k, x,
-                           (rocblas_int)w.k, &beta, y, (rocblas_int)w.n);
-    if (st != rocblas_status_success) {
-        g_dense_error = std::string("rocblas_sgemm: ") + blas_status(st);
-        return hipErrorUnknown;
+    switch (w.qtype) {
+        case UNILLM_QTYPE_F32: return launch_dense_qt<UNILLM_QTYPE_F32>(w, x, m, y, s, add);
+        case UNILLM_QTYPE_F16: return launch_dense_qt<UNILLM_QTYPE_F16>(w, x, m, y, s, add);
+        case UNILLM_QTYPE_BF16: return launch_dense_qt<UNILLM_QTYPE_BF16>(w, x, m, y, s, add);
+        default: return hipErrorInvalidValue;
     }
-    return hipSuccess;
 }
 
 }  // namespace unillm

@@ -168,8 +168,10 @@ const DeviceInfo& device_info();
 // of a SwiGLU call off the GEMV path (both live during that call); slot 2 the
 // rotated queries and the per-chunk partials of decode attention; slot 3 an
 // aligned copy of x; slot kSyncSlot the batched decode's arrival tickets, zeroed
-// when allocated (every launch leaves them zero again).
+// when allocated (every launch leaves them zero again); slot kDenseSlot a dense
+// weight's x in 16-bit parts and its split-k slabs.
 constexpr int kSyncSlot = 4;
+constexpr int kDenseSlot = 5;
 hipError_t stream_workspace(hipStream_t s, size_t bytes, void** out, int slot = 0);
 // UNILLM_DEBUG_LAUNCH=1 prints each kernel's launch shape to stderr.
 bool debug_launch();
@@ -232,21 +234,24 @@ hipError_t launch_x_to_f16_rows(const float* x, int64_t m, int64_t k, void* out,
 // gu[m, 2 I] (the SwiGLU of the MFMA paths, after their store)
 hipError_t launch_swiglu(const float* gu, int64_t m, int64_t I, float* act, hipStream_t s);
 
-// Dense (F32 / F16 / BF16) weights: f32 rows [n][k] at base (row_bytes = 4 k).
+// Dense (F32 / F16 / BF16) weights: rows in the weight's own type, k padded with zeros
+// (dense_row_bytes a row); F16 rows are held scaled by a power of two each.
 bool is_dense(int qtype);
 int dense_elem_bytes(int qtype);
-// the weight's f32 rows from its GGUF elements at src (device memory), on s
+int64_t dense_row_bytes(int qtype, int64_t k);
+size_t dense_extra_bytes(int qtype, int64_t n);  // behind the rows: F16's row factors
+// the weight's rows from its GGUF elements at src (device memory), on s
 hipError_t launch_dense_upload(const QWeight& w, const void* src, hipStream_t s);
-// y = x W^T (add: y += x W^T) in f32; the GEMM's handle is created on first use
-// (dense_prepare creates it ahead, outside any capture)
+// out[n, k] f32 <- the weight's values
+hipError_t launch_dense_widen(const QWeight& w, float* out, hipStream_t s);
+// y = x W^T (add: y += x W^T) at f32's precision; past the GEMV it takes the stream's
+// slot kDenseSlot, whose size for any call of up to m rows is dense_workspace_bytes
 hipError_t launch_dense(const QWeight& w, const float* x, int64_t m, float* y, hipStream_t s,
                         int add);
-hipError_t dense_prepare(hipStream_t s);
+size_t dense_workspace_bytes(const QWeight& w, int64_t m);
 // the layer norm of each row of x into out (f32), ops_fn::layer_norm's two passes
 hipError_t launch_norm_rows(const float* x, int64_t m, int64_t k, const NormArgs& norm,
                             float* out, hipStream_t s);
-// the message of the last failing dense call on this thread
-std::string dense_error();
 
 // Attention (attention.hip): RoPE at positions len .. len + m - 1 on the fused QKV
 // rows qkv[m, (H + 2 KVH) hd], k / v appended to the cache, causal softmax

@@ -66,8 +66,8 @@ class QuantLinear:
     @classmethod
     def from_dense(cls, w: torch.Tensor,
                    stream: torch.cuda.Stream | None = None) -> "QuantLinear":
-        """A dense [n, k] device tensor (float32, float16 or bfloat16), kept as f32 rows
-        and multiplied in f32, as candle's QMatMul keeps a dense GGUF tensor."""
+        """A dense [n, k] device tensor (float32, float16 or bfloat16), kept in its own type
+        and multiplied in f32, as candle's QMatMul multiplies a dense GGUF tensor."""
         qtype = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}.get(w.dtype)
         if qtype is None or w.dim() != 2 or not w.is_cuda:
             raise ValueError("w must be a 2-D float32 / float16 / bfloat16 device tensor")

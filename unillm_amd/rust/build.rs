@@ -21,9 +21,8 @@ const SOURCES: &[&str] = &[
     "dense.hip",
 ];
 
-// Libraries the link adds: the dense (F32 / F16 / BF16) weights' f32 GEMM.  Keep in step
-// with LIBS in unillm_amd/build.py.
-const LIBS: &[&str] = &["-L/opt/rocm/lib", "-lrocblas", "-Wl,-rpath,/opt/rocm/lib"];
+// Libraries the link adds besides HIP's own.  Keep in step with LIBS in unillm_amd/build.py.
+const LIBS: &[&str] = &[];
 
 const FLAGS: &[&str] = &[
     "--offload-arch=gfx950",
