@@ -1,0 +1,102 @@
+"""The prompt attention kernel over its plans: block heights, pairing, key splits, tails.
+
+Against float64 attention with RoPE at the reference's f32 angles (positions times f32
+frequencies, llama.rs:827-883).  The products keep f32's 24 bits and sum in f32: 1e-6
+normwise (the f32 matrix cores measured 3.8e-7 at the same shapes).
+"""
+import math
+
+import pytest
+import torch
+
+from unillm_amd import KvCache
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-6
+
+
+def _rope(t, pos, hd):
+    e = torch.arange(0, hd, 2, device="cuda", dtype=torch.float32) / hd
+    inv = 1.0 / torch.pow(torch.tensor(10000.0, dtype=torch.float64, device="cuda"),
+                          e.double()).float()
+    ang = (pos.float()[:, None] * inv).double()[:, None, :]
+    a, b = t[..., : hd // 2], t[..., hd // 2:]
+    return torch.cat([a * ang.cos() - b * ang.sin(), a * ang.sin() + b * ang.cos()], -1)
+
+
+def _reference(x, H, KVH, hd, past):
+    """x: every token's qkv row; the outputs of tokens past .. (each from its own keys only)."""
+    n = x.shape[0]
+    q, k, v = x.double().split([H * hd, KVH * hd, KVH * hd], -1)
+    pos = torch.arange(n, device="cuda")
+    q, k = _rope(q.view(n, H, hd), pos, hd), _rope(k.view(n, KVH, hd), pos, hd)
+    v = v.view(n, KVH, hd)
+    out = torch.empty(n - past, H, hd, dtype=torch.float64, device="cuda")
+    seen = pos[None, :] <= pos[past:, None]
+    for h in range(H):
+        g = h // (H // KVH)
+        s = (q[past:, h] @ k[:, g].t()) / math.sqrt(hd)
+        p = torch.softmax(s.masked_fill(~seen, -math.inf), -1)
+        out[:, h] = torch.where(seen[:, :, None], p[:, :, None] * v[None, :, g], 0.0).sum(1) \
+            if n <= 256 else p @ v[:, g]
+    return out.view(n - past, H * hd)
+
+
+def _run(x, H, KVH, hd, past, room=0):
+    kv = KvCache(KVH, hd, x.shape[0] + room)
+    if past:
+        kv.attention(x[:past].contiguous(), H)
+    return kv.attention(x[past:].contiguous(), H)
+
+
+# one query tile to many blocks; odd and even block counts; a past that leaves tiles and
+# steps unaligned, fits one step, or is longer than the prompt; a full and a roomy cache
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("m,past,H,KVH", [(17, 0, 4, 4), (33, 31, 4, 1), (64, 0, 16, 8),
+                                          (65, 1000, 8, 2), (128, 63, 8, 8), (129, 64, 4, 4),
+                                          (300, 5, 16, 4), (513, 0, 32, 32), (1100, 77, 8, 8),
+                                          (40, 3000, 32, 4)])
+def test_prompt_plans(hd, m, past, H, KVH):
+    print(f"prompt hd={hd} m={m} past={past} H={H} KVH={KVH}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + past)
+    x = torch.randn(past + m, (H + 2 * KVH) * hd, device="cuda", generator=g)
+    ref = _reference(x, H, KVH, hd, past)
+    out = _run(x, H, KVH, hd, past, room=m % 3 * 50)
+    assert ((out.double() - ref).norm() / ref.norm()).item() < TOL
+    assert torch.equal(_run(x, H, KVH, hd, past), out)
+
+
+# large and small scores, and running maxima that keep rising (the lazy rescale)
+@pytest.mark.parametrize("scale", [0.0, 1e-3, 6.0])
+def test_prompt_score_ranges(scale):
+    H, KVH, hd, m = 4, 2, 64, 200
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(m, (H + 2 * KVH) * hd, device="cuda", generator=g)
+    x[:, : (H + KVH) * hd] *= scale * torch.linspace(0.5, 1.5, m, device="cuda")[:, None]
+    ref = _reference(x, H, KVH, hd, 0)
+    out = _run(x, H, KVH, hd, 0)
+    # a score of size s rounds to 2^-24 s in f32, and so do its exponentials
+    assert ((out.double() - ref).norm() / ref.norm()).item() < TOL * max(1.0, 36 * scale / 6)
+
+
+# non-finite keys and values reach exactly the outputs that see them, as in f32
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("what", ["v_inf", "v_nan", "k_inf", "q_nan"])
+def test_prompt_non_finite(hd, what):
+    H, KVH, m, past = 4, 2, 100, 37
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(past + m, (H + 2 * KVH) * hd, device="cuda", generator=g)
+    bad = float("nan") if what.endswith("nan") else float("inf")
+    col = {"q": 5, "k": H * hd + 5, "v": (H + KVH) * hd + 5}[what[0]]
+    x[past + 50, col] = bad
+    if what == "v_inf":
+        x[3, col + hd] = -bad  # in the past, the other kv head
+    ref = _reference(x, H, KVH, hd, past).float()
+    out = _run(x, H, KVH, hd, past)
+    assert torch.equal(out.isnan(), ref.isnan())
+    assert torch.equal(out.isinf(), ref.isinf())
+    assert torch.equal(out[out.isinf()], ref[ref.isinf()])
+    fin = ref.isfinite()
+    assert fin.any()
+    assert ((out - ref)[fin].norm() / ref[fin].norm()).item() < TOL

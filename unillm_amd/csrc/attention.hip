@@ -49,6 +49,7 @@
 #include <type_traits>
 
 #include "internal.hpp"
+#include "split.hpp"
 
 namespace unillm {
 namespace {
@@ -461,13 +462,14 @@ int64_t chunk_len(int64_t L, int64_t KVH) {
 
 // ---- prompt-length calls (m H / KVH beyond a decode step) ---------------------------------
 //
-// rope_append_kernel, a workgroup per (token t, head): q heads rotated at position
-// len + t and scaled by 1 / sqrt(hd) into the workspace qw[H][m][hd]; k heads rotated
-// and, with v, appended to the cache (the decode kernel's formulas, so either path
-// writes the same cache).  Then, for hd 64 and 128, attn_prefill_mfma on the f32 matrix
-// cores (further down; with its key range split, attn_merge_split_kernel after it);
-// for hd 256, attn_prefill_kernel, a workgroup per (block of BQ queries, head h):
-// flash-style causal attention over the cache in f32 --
+// rope_append_kernel, a workgroup per (token t, head h0 + blockIdx.y): k heads rotated at
+// position len + t and, with v, appended to the cache (the decode kernel's formulas, so
+// either path writes the same cache); for hd 256 also q heads, rotated and scaled by
+// 1 / sqrt(hd), into the workspace qw[H][m][hd].  Then, for hd 64 and 128,
+// attn_prompt_kernel on the matrix cores (further down; it rotates its own queries; with
+// its key range split, attn_merge_split_kernel after it); for hd 256,
+// attn_prefill_kernel, a workgroup per (block of BQ queries, head h): flash-style causal
+// attention over the cache in f32 --
 //   - the block's queries Q^T [hd][BQ] stay in LDS; the key positions run in tiles of BK
 //     (K^T [hd][BK] and V [BK][hd] in LDS), only up to the block's last query position;
 //   - thread (tr, tc) of 16 x 16 computes scores for rows tr RT .. and columns tc CT ..
@@ -484,11 +486,11 @@ template <int D>
 __global__ __launch_bounds__(D / 2) void rope_append_kernel(
     const float* __restrict__ qkv, int m, int H, int KVH, int* __restrict__ state, float scale,
     const float* __restrict__ inv_freq, float* __restrict__ kc, float* __restrict__ vc,
-    int max_seq, float* __restrict__ qw) {
+    int max_seq, float* __restrict__ qw, int h0) {
     constexpr int HALF = D / 2;
     const int len = state[0];
-    const int t = blockIdx.x, hh = blockIdx.y, p = threadIdx.x;
-    if (t == 0 && hh == 0 && p == 0) state[2] = len;  // this call's length, for the next kernel
+    const int t = blockIdx.x, hh = h0 + blockIdx.y, p = threadIdx.x;
+    if (t == 0 && blockIdx.y == 0 && p == 0) state[2] = len;  // this call's length, for the next kernel
     if (len + m > max_seq) return;  // overflow: nothing appended; the attention kernel reports it
     const float* row = qkv + (int64_t)t * (H + 2 * KVH) * D;
     float sn, cs;
@@ -646,82 +648,116 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float* __restri
     }
 }
 
-// ---- prompt-length attention on the f32 matrix cores (hd 64 and 128) ------------------------
+// ---- prompt-length attention on the matrix cores (hd 64 and 128) ---------------------------
 //
-// attn_prefill_mfma<D, NW>: a workgroup per (NW / 2 pairs of 32-query tiles, head h), NW
-// waves, each owning one tile (the pairing below balances the causal work).  Everything is f32: v_mfma_f32_32x32x2f32
-// multiplies f32 operands exactly and accumulates in f32, like the FMA loop above, so
-// the numbers match it to summation order.  The products are formed transposed so that
-// no row reduction crosses more than two lanes and P never leaves the registers:
-//   S^T [32 keys][32 queries] = K . Q^T -- the MFMA's A operand is a key row (lane l:
-//     key l % 32), B is the wave's queries (lane l: query l % 32), and MFMA s contracts
-//     dimensions s and D / 2 + s (lane half l / 32 takes one of each pair), so a lane
-//     reads its key's dimensions as float4s from LDS and keeps its query's half in
-//     registers for the whole kernel;
+// attn_prompt_kernel<D, QT>: a workgroup per (block of QT 32-query tiles, or two such
+// blocks one after the other; head h), 2 QT waves: wave w takes query tile w % QT and every
+// second key tile (kh = w / QT), and the two waves of a tile merge their sums at the block's
+// end.  Both products keep f32's precision on the bf16 matrix cores: q, k, v and the
+// exponentials p are split exactly into three bf16 parts (split.hpp), and the six products
+// of parts that reach 2^-24 are summed in f32, the five small ones of q k in a sum of their
+// own.  The products are formed transposed so that no row reduction crosses more than two
+// lanes and P never leaves the registers:
+//   S^T [32 keys][32 queries] = K . Q^T (v_mfma_f32_32x32x16_bf16: A lane l holds key
+//     l % 32, dimensions 8 (l / 32) .. + 7 of each 16; B the same of query l % 32, rotated
+//     (RoPE), scaled and split once a block by the tile's two waves: part 0 in registers,
+//     parts 1 and 2 in LDS, which leaves registers for two waves a SIMD);
 //   a lane's 16 accumulators are 16 keys of ONE query (rows 8 (r / 4) + 4 (l / 32) +
 //     r % 4, column l % 32): the query's max and sum over the tile are a 16-value
 //     register reduction and one exchange with lane l ^ 32;
-//   O^T [D][32 queries] += V^T . P^T -- MFMA s contracts keys 8 (s / 4) + s % 4 and the
-//     same + 4, exactly the two keys whose exponentials lanes l and l ^ 32 hold in
-//     accumulator s: B is the lane's own p[s], A is V[that key][32 t + l % 32] (D / 32
-//     output tiles).
-// Key tiles of 32 positions (K and V rows padded to D + 4 floats in LDS) are double
-// buffered: tile k + 1 is read into registers while tile k is computed and stored to
-// LDS after it.  A wave skips the tiles wholly past its last query (causal) but keeps
-// loading and meeting the others.  Same length and overflow handling as
-// attn_prefill_kernel.
+//   O^T [D][32 queries] += V^T . P^T: MFMA kb contracts, in lane half hf, the 8 keys whose
+//     exponentials that lane holds in accumulators 8 kb .. 8 kb + 7, so B is the lane's
+//     own p and V^T is staged in that key order (chunk 2 kb + hf of a row).
+// A step stages two key tiles of 32 positions in LDS as parts: K [2][3][32 keys][2 D bytes]
+// and V^T [2][3][D][64 bytes], 16-byte chunks XOR-swizzled so that the 16 lanes a read
+// serves together touch all banks once.  A thread's staging task is 8 dimensions of a key or
+// 8 keys of a dimension.  V is split and stored after the wave's q k products, the next
+// step's K after its p v products, each meeting the others at one barrier: every split
+// runs beside another wave's MFMAs, without a second buffer.
+// Bound by the matrix cores (12 D / 16 MFMAs of 32 cycles a tile and wave) with the softmax
+// and the splits' VALU work beside them.  With the causal mask a block's work grows with
+// its position: taking blocks i and last - i one after the other gives every workgroup the
+// same (a form that paired a low and a high tile in two waves of one workgroup left one
+// wave a SIMD half the time).  Measured, kernel alone: m2048, 32 heads of 128: 239 us (144
+// TFLOP/s of f32 product; 391 on the f32 matrix cores, 270 in the paired form), m500 behind
+// 777, 32 heads of 64 over 4: 45 us and the merge's 4.6 (65.6 and 4.8).  At m2048 the matrix
+// cores are busy 41 % and the VALU 30 % of the cycles, and hardly at once.
+// A non-finite k or v makes 0 * inf terms in the split products: a query whose sum or
+// output comes out non-finite is recomputed in plain f32.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-template <int D, int NW>
-struct MfmaPrefillLds {
-    static constexpr int ROW = D + 4;                     // padded row (floats)
-    static constexpr int TILE = 32 * ROW;                 // one of K or V, or a wave's queries
-    static constexpr size_t BYTES = (size_t)2 * 2 * TILE * sizeof(float);  // 2 stages x (K, V)
-    static constexpr int LPT = 2 * 32 * D / 4 / (64 * NW);  // float4 loads a thread per tile
+constexpr float kLog2e = 1.44269504088896340736f;
+
+__device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// 8 f32 (vector v, from element o) -> three parts
+template <class V>
+__device__ __forceinline__ void split8(const V& v, int o, u32x4 (&p)[3]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        uint32_t a, b, c;
+        split2(__float_as_uint(v[o + 2 * j]), __float_as_uint(v[o + 2 * j + 1]), a, b, c);
+        p[0][j] = a;
+        p[1][j] = b;
+        p[2][j] = c;
+    }
+}
+
+template <int D, int QT>
+struct PromptLds {
+    static constexpr int NW = 2 * QT;         // waves
+    static constexpr int KROW = 2 * D;        // bytes of a key's part
+    static constexpr int KP = 32 * KROW;      // a plane of K
+    static constexpr int VP = 64 * D;         // a plane of V^T (the same size)
+    static constexpr int TILE = 3 * KP;       // a staged K or V tile
+    static constexpr int V0 = 2 * TILE;       // K tiles | V tiles | query parts 1 and 2
+    static constexpr int Q1 = 4 * TILE;       // [QT][D / 16][2][64 lanes][16 B]
+    static constexpr int BYTES = Q1 + QT * (D / 16) * 2048;
+    static constexpr int TASKS = 8 * D / (64 * NW);  // staging tasks a thread for two K (or V) tiles
+    // a block's first query parts, and its odd waves' sums, pass through the staging tiles
+    static_assert(QT * (D / 16) * 1024 <= 4 * TILE && QT * (2 * D + 8) * 64 <= 4 * TILE, "");  // (a redone query too)
+    // the slot of chunk c in key row r: 8 or 16 chunks a row
+    __device__ static uint32_t kslot(uint32_t r, uint32_t c) {
+        return D == 128 ? c ^ (r & 15) : c ^ ((r >> 1) & 7);
+    }
+    __device__ static uint32_t vslot(uint32_t d, uint32_t c) { return c ^ ((d >> 2) & 3); }
 };
 
-template <int D, int NW>
-__global__ __launch_bounds__(64 * NW) void attn_prefill_mfma(const float* __restrict__ qw, int m,
-                                                             int H, int KVH,
-                                                             int* __restrict__ state,
-                                                             const float* __restrict__ kc,
-                                                             const float* __restrict__ vc,
-                                                             int max_seq, float* __restrict__ out,
-                                                             float* __restrict__ part) {
-    using L = MfmaPrefillLds<D, NW>;
-    constexpr int HALF = D / 2, OT = D / 32, ROW = L::ROW;
-    extern __shared__ __attribute__((aligned(16))) float sm[];
+template <int D, int QT>
+__global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
+    const float* __restrict__ qkv, int m, int H, int KVH, int* __restrict__ state, float scale,
+    const float* __restrict__ inv_freq, const float* __restrict__ kc,
+    const float* __restrict__ vc, int max_seq, int blocks, int paired, float* __restrict__ out,
+    float* __restrict__ part) {
+    using L = PromptLds<D, QT>;
+    constexpr int OT = D / 32, NB = D / 16, NT = 128 * QT;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int h = blockIdx.y, g = h / (H / KVH);
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hf = lane >> 5;
-    // The head's T tiles of 32 queries are paired (i, T - 1 - i), so that under the
-    // causal mask every pair holds the same work (the middle tile of an odd T has no
-    // partner); workgroup b takes pairs b NW / 2 .. + NW / 2 - 1, waves w < NW / 2
-    // their low tiles and the others their high ones (one of each a SIMD).  -1: no
-    // tile for this wave.
-    const int T = (m + 31) / 32, P = (T + 1) / 2;
-    auto tile_of = [&](int w) {
-        const int i = (int)blockIdx.x * (NW / 2) + w % (NW / 2);
-        if (i >= P) return -1;
-        if (w < NW / 2) return i;
-        return T - 1 - i > i ? T - 1 - i : -1;
-    };
-    const int mytile = tile_of(wv);  // wave-uniform
-    int top = 0;                     // the workgroup's last tile
-#pragma unroll
-    for (int w = 0; w < NW; ++w) top = max(top, tile_of(w));
-    // gridDim.z > 1: this workgroup takes split blockIdx.z of the key tiles and writes
-    // partials (max, sum, unnormalized o) for attn_merge_kernel, which then also
-    // advances the length or reports the overflow
+    const int qt = wv % QT, kh = wv / QT;
+    // gridDim.z > 1: this workgroup takes split blockIdx.z of each block's key tiles and
+    // writes partials (max, sum, unnormalized o) for attn_merge_split_kernel, which then
+    // also advances the length or reports the overflow
     const int S = gridDim.z, z = blockIdx.z;
     const int len = state[2];
+    const int other = paired ? blocks - 1 - (int)blockIdx.x : (int)blockIdx.x;  // the second block
+    const int nblk = other != (int)blockIdx.x ? 2 : 1;
     if (len + m > max_seq) {
         if (S == 1) {
-            if (mytile >= 0)
-                for (int i = lane; i < 32 * D; i += 64) {
-                    const int q = 32 * mytile + i / D;
-                    if (q < m) out[(int64_t)q * H * D + (int64_t)h * D + i % D] = __builtin_nanf("");
+            for (int bi = 0; bi < nblk; ++bi) {
+                const int q0 = (bi ? other : (int)blockIdx.x) * 32 * QT;
+                for (int i = tid; i < 32 * QT * D; i += NT) {
+                    const int qq = q0 + i / D;
+                    if (qq < m) out[(int64_t)qq * H * D + (int64_t)h * D + i % D] = __builtin_nanf("");
                 }
+            }
             if (blockIdx.x == 0 && h == 0 && tid == 0) state[1] = 1;
         }
         return;
@@ -731,189 +767,361 @@ __global__ __launch_bounds__(64 * NW) void attn_prefill_mfma(const float* __rest
     const float* kg = kc + (int64_t)g * max_seq * D;
     const float* vg = vc + (int64_t)g * max_seq * D;
 
-    // this lane's query (rows past m, and a wave without a tile, repeat the last one),
-    // its half of the dimensions in one vector (a vector stays in registers)
-    const int qi = mytile >= 0 ? 32 * mytile + col : m;
-    typedef float qhalf_t __attribute__((ext_vector_type(HALF)));
-    qhalf_t qr;
-    {
-        const float* qrow = qw + ((int64_t)h * m + min(qi, m - 1)) * D + hf * HALF;
-#pragma unroll
-        for (int u = 0; u < HALF / 4; ++u) {
-            const float4 v = *reinterpret_cast<const float4*>(qrow + 4 * u);
-            qr[4 * u] = v.x;
-            qr[4 * u + 1] = v.y;
-            qr[4 * u + 2] = v.z;
-            qr[4 * u + 3] = v.w;
-        }
-    }
-    const int qpos = len + qi;  // this lane's query position
-    // the wave's last query position (-1: no tile, every key tile skipped)
-    const int wave_last = mytile >= 0 ? len + min(32 * mytile + 31, m - 1) : -1;
-    const int last_pos = len + min(32 * top + 31, m - 1);
-    const int ntiles = last_pos / 32 + 1;
-    const int kt0 = z * ntiles / S, kt1 = (z + 1) * ntiles / S;  // this workgroup's key tiles
-
-    // tile loads: float4 f = i (64 NW) + tid, i < LPT, over [K rows 0..31 | V rows 0..31];
-    // the staged floats sit in one vector (a vector stays in registers)
-    typedef float stage_t __attribute__((ext_vector_type(4 * L::LPT)));
+    // staging task i of this thread, f = i NT + tid < 8 D: tile f / (4 D) of the step's two;
+    // K: 8 dimensions 8 c .. of key row r; V: dimension d, the 8 keys of chunk ch
+    typedef float stage_t __attribute__((ext_vector_type(8 * L::TASKS)));
     stage_t st;
-    auto src_of = [&](int i, int kt) {
-        const int f = i * 64 * NW + tid;
-        const int which = f / (32 * D / 4), r = (f / (D / 4)) % 32, c = f % (D / 4);
-        return (which ? vg : kg) + (int64_t)min(kt * 32 + r, total - 1) * D + 4 * c;
-    };
-    auto dst_of = [&](int i) {
-        const int f = i * 64 * NW + tid;
-        const int which = f / (32 * D / 4), r = (f / (D / 4)) % 32, c = f % (D / 4);
-        return which * L::TILE + r * ROW + 4 * c;
-    };
-
-    float mrun = -INFINITY, lrun = 0.0f;
-    f32x16 o[OT];
+    // (a tile past the filled length repeats the last row, always masked; whole tiles take
+    // addresses of a uniform base and a lane's fixed offset)
+    auto request = [&](const float* cache, int n, auto IsV) {
+        int ti = tid;  // opaque: offsets are recomputed, not kept in registers
+        asm volatile("" : "+v"(ti));
+        auto each = [&](auto Whole) {
 #pragma unroll
-    for (int t = 0; t < OT; ++t)
+            for (int i = 0; i < L::TASKS; ++i) {
+                const int tile = (i * NT + 64 * wv) / (4 * D);  // (wave-uniform)
+                const int kt = Whole.value ? 2 * n + tile : min(2 * n + tile, (total - 1) / 32);
+                const int lim = total - 1 - 32 * kt;
+                const float* src = cache + (int64_t)kt * (32 * D);
+                const int f = (i * NT + ti) % (4 * D);
+                if constexpr (IsV.value) {
+                    const int d = f % D, ch = f / D;
+                    const int k0 = 16 * (ch / 2) + 4 * (ch % 2);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) o[t][e] = 0.0f;
-
-#pragma unroll
-    for (int i = 0; i < L::LPT; ++i) {
-        const float4 v = *reinterpret_cast<const float4*>(src_of(i, kt0));
-        *reinterpret_cast<float4*>(sm + (kt0 & 1) * 2 * L::TILE + dst_of(i)) = v;
-    }
-    __syncthreads();
-    for (int kt = kt0; kt < kt1; ++kt) {
-        const float* Ks = sm + (kt & 1) * 2 * L::TILE;
-        const float* Vs = Ks + L::TILE;
-        const bool more = kt + 1 < kt1;
-        const bool live = kt * 32 <= wave_last;  // wave-uniform: tiles past the wave's last query skipped
-        f32x16 s;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) s[e] = 0.0f;
-        if (live) {
-            // S^T = K . Q^T, the next float4 of the key row read ahead of the MFMAs
-            const float* krow = Ks + col * ROW + hf * HALF;
-            // two accumulators (dimension pairs alternate), so consecutive MFMAs do not
-            // wait on each other's results
-            f32x16 s2;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) s2[e] = 0.0f;
-            float4 kv = *reinterpret_cast<const float4*>(krow);
-#pragma unroll
-            for (int u = 0; u < HALF / 4; ++u) {
-                const float4 kn =
-                    u + 1 < HALF / 4 ? *reinterpret_cast<const float4*>(krow + 4 * (u + 1)) : kv;
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qr[4 * u], s, 0, 0, 0);
-                s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qr[4 * u + 1], s2, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qr[4 * u + 2], s, 0, 0, 0);
-                s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qr[4 * u + 3], s2, 0, 0, 0);
-                kv = kn;
-            }
-            s += s2;
-        }
-        // the next tile's rows requested while this one's softmax and p v run
-        if (more) {
-#pragma unroll
-            for (int i = 0; i < L::LPT; ++i) {
-                const float4 v = *reinterpret_cast<const float4*>(src_of(i, kt + 1));
-                st[4 * i] = v.x;
-                st[4 * i + 1] = v.y;
-                st[4 * i + 2] = v.z;
-                st[4 * i + 3] = v.w;
-            }
-        }
-        if (live) {
-            // causal mask and the query's running max / sum
-            float tmax = -INFINITY;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int kpos = kt * 32 + 8 * (r / 4) + 4 * hf + r % 4;
-                if (kpos > qpos || kpos >= total) s[r] = -INFINITY;
-                tmax = fmaxf(tmax, s[r]);
-            }
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-            const float mnew = fmaxf(mrun, tmax);
-            const float alpha = mnew == -INFINITY ? 1.0f : expf(mrun - mnew);
-            float tsum = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float p = s[r] == -INFINITY ? 0.0f : expf(s[r] - mnew);
-                s[r] = p;
-                tsum += p;
-            }
-            tsum += __shfl_xor(tsum, 32, 64);
-            lrun = lrun * alpha + tsum;
-            mrun = mnew;
-            // O^T = alpha O^T + V^T . P^T.  The rescale moves the accumulators through
-            // the VALU, so it runs only when some query's running max changed (alpha
-            // is then < 1 somewhere in the wave; after the first tiles it rarely is).
-            if (__any(alpha != 1.0f)) {
-#pragma unroll
-                for (int t = 0; t < OT; ++t)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
-            }
-            // two output tiles at a time, their MFMAs interleaved (independent chains),
-            // the tiles' 32 V values read ahead
-#pragma unroll
-            for (int t = 0; t < OT; t += 2) {
-                float vv[2][16];
-#pragma unroll
-                for (int a = 0; a < 2; ++a)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        vv[a][r] = Vs[(8 * (r / 4) + 4 * hf + r % 4) * ROW + 32 * (t + a) + col];
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[0][r], s[r], o[t], 0, 0, 0);
-                    o[t + 1] =
-                        __builtin_amdgcn_mfma_f32_32x32x2f32(vv[1][r], s[r], o[t + 1], 0, 0, 0);
+                    for (int j = 0; j < 8; ++j) {
+                        const int r = k0 + 8 * (j / 4) + j % 4;
+                        st[8 * i + j] = src[(Whole.value ? r : min(r, lim)) * D + d];
+                    }
+                } else {
+                    const int r = f / (D / 8), c = f % (D / 8);
+                    const float* row = src + (Whole.value ? r : min(r, lim)) * D + 8 * c;
+                    const float4 a = *reinterpret_cast<const float4*>(row);
+                    const float4 b = *reinterpret_cast<const float4*>(row + 4);
+                    st[8 * i] = a.x, st[8 * i + 1] = a.y, st[8 * i + 2] = a.z, st[8 * i + 3] = a.w;
+                    st[8 * i + 4] = b.x, st[8 * i + 5] = b.y, st[8 * i + 6] = b.z, st[8 * i + 7] = b.w;
                 }
             }
-        }
-        if (more) {
-            float* base = sm + ((kt + 1) & 1) * 2 * L::TILE;
+        };
+        if (64 * (n + 1) <= total) each(std::true_type{});
+        else each(std::false_type{});
+    };
+    auto request_k = [&](int n) { request(kg, n, std::false_type{}); };
+    auto request_v = [&](int n) { request(vg, n, std::true_type{}); };
+    auto store = [&](auto IsV) {
 #pragma unroll
-            for (int i = 0; i < L::LPT; ++i)
-                *reinterpret_cast<float4*>(base + dst_of(i)) =
-                    make_float4(st[4 * i], st[4 * i + 1], st[4 * i + 2], st[4 * i + 3]);
-        }
-        __syncthreads();
-    }
-    if (S > 1) {
-        // partials as attn_merge_kernel reads them: (max, sum) at [q H + h][S], o at
-        // [q H + h][S][hd] after all the pairs (a query with no live tile in this split
-        // leaves (-inf, 0) and zeros, weight 0 in the merge)
-        if (qi < m) {
-            const int64_t qc = ((int64_t)qi * H + h) * S + z;
-            if (hf == 0) *reinterpret_cast<float2*>(part + 2 * qc) = make_float2(mrun, lrun);
-            float* prow = part + (int64_t)m * H * S * 2 + qc * D + 4 * hf;
+        for (int i = 0; i < L::TASKS; ++i) {
+            const int f = i * NT + tid;
+            uint32_t off;
+            if constexpr (IsV.value) {
+                const uint32_t d = f % D, ch = f / D % 4;
+                off = L::V0 + f / (4 * D) * L::TILE + d * 64 + L::vslot(d, ch) * 16;
+            } else {
+                const uint32_t r = f / (D / 8) % 32, c = f % (D / 8);
+                off = f / (4 * D) * L::TILE + r * L::KROW + L::kslot(r, c) * 16;
+            }
+            u32x4 p[3];
+            split8(st, 8 * i, p);
 #pragma unroll
-            for (int t = 0; t < OT; ++t)
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    *reinterpret_cast<float4*>(prow + 32 * t + 8 * u) =
-                        make_float4(o[t][4 * u], o[t][4 * u + 1], o[t][4 * u + 2], o[t][4 * u + 3]);
+            for (int q = 0; q < 3; ++q)
+                *reinterpret_cast<u32x4*>(lds + off + q * L::KP) = p[q];
         }
-        return;
-    }
-    // O[q][32 t + 8 u + 4 hf + 0..3] = o[t][4 u + 0..3] / l, a float4 each
-    if (qi < m) {
-        const float inv = 1.0f / lrun;
-        float* orow = out + (int64_t)qi * H * D + (int64_t)h * D + 4 * hf;
+    };
+    constexpr std::false_type kK;
+    constexpr std::true_type kV;
+
+    const uint8_t* Ks = lds + kh * L::TILE;
+    const uint8_t* Vs = lds + L::V0 + kh * L::TILE;
+    const uint32_t voff = col * 64, vsw = L::vslot(col, 0);
+
+    for (int bi = 0; bi < nblk; ++bi) {
+        const int t0 = (bi ? other : (int)blockIdx.x) * QT;  // the block's first query tile
+        const int mytile = t0 + qt;
+        // the wave's last query position (below 0: no queries, every key tile skipped)
+        const int wave_last = 32 * mytile < m ? len + min(32 * mytile + 31, m - 1) : -1;
+        const int last_pos = len + min(32 * (t0 + QT) - 1, m - 1);
+        const int steps = (last_pos / 32 + 2) / 2;  // pairs of key tiles
+        const int n0 = z * steps / S, n1 = (z + 1) * steps / S;  // this workgroup's
+        if (n0 < n1) request_k(n0);
+
+        // this lane's query (rows past m repeat the last one): dimensions 16 b + 8 hf .. + 7
+        // rotated at its position, scaled and split; the tile's two waves do half the
+        // dimension pairs each and exchange them through LDS
+        const int qi = 32 * mytile + col;
+        const int qpos = len + qi;
+        u32x4 q[NB];
+        uint8_t* q1 = lds + L::Q1 + (qt * NB * 128 + lane) * 16;  // parts 1, 2 at (2 b + i - 1) 1024
+        {
+            uint8_t* qx = lds + (qt * NB * 64 + lane) * 16;  // part 0 of block b at b * 1024
+            __syncthreads();  // the staging tiles are free (the block before is done)
+            const int qr = min(qi, m - 1);
+            const float* row = qkv + (int64_t)qr * (H + 2 * KVH) * D + (int64_t)h * D;
+            typedef float f32x8 __attribute__((ext_vector_type(8)));
+#pragma unroll
+            for (int bb = 0; bb < NB / 4; ++bb) {
+                const int b = kh * (NB / 4) + bb;
+                f32x8 lo, hi;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int p = 16 * b + 8 * hf + j;
+                    float sn, cs;
+                    sincosf((float)(len + qr) * inv_freq[p], &sn, &cs);
+                    const float a = row[p], c = row[p + D / 2];
+                    lo[j] = (a * cs - c * sn) * scale;
+                    hi[j] = (a * sn + c * cs) * scale;
+                }
+                u32x4 pl[3], ph[3];
+                split8(lo, 0, pl);
+                split8(hi, 0, ph);
+                *reinterpret_cast<u32x4*>(qx + b * 1024) = pl[0];
+                *reinterpret_cast<u32x4*>(qx + (b + NB / 2) * 1024) = ph[0];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    *reinterpret_cast<u32x4*>(q1 + (2 * b + i) * 1024) = pl[1 + i];
+                    *reinterpret_cast<u32x4*>(q1 + (2 * (b + NB / 2) + i) * 1024) = ph[1 + i];
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int b = 0; b < NB; ++b) q[b] = *reinterpret_cast<const u32x4*>(qx + b * 1024);
+            __syncthreads();
+        }
+        if (n0 < n1) {
+            store(kK);
+            request_v(n0);
+        }
+
+        // the exponentials' reference, in units of log2 e (p = exp2(s log2 e - mrun))
+        float mrun = -INFINITY, lrun = 0.0f;
+        f32x16 o[OT];
 #pragma unroll
         for (int t = 0; t < OT; ++t)
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                *reinterpret_cast<float4*>(orow + 32 * t + 8 * u) =
-                    make_float4(o[t][4 * u] * inv, o[t][4 * u + 1] * inv, o[t][4 * u + 2] * inv,
-                                o[t][4 * u + 3] * inv);
+            for (int e = 0; e < 16; ++e) o[t][e] = 0.0f;
+        for (int n = n0; n < n1; ++n) {
+            __syncthreads();  // K of step n is staged, V of step n - 1 read
+            const int kt = 2 * n + kh;
+            // wave-uniform: tiles past the wave's last query skipped
+            const bool live = kt * 32 <= wave_last;
+            f32x16 s, sl;
+            // (the odd waves split V before their products, the even ones after: one's VALU
+            // work runs beside the other's MFMAs)
+            auto stage_v = [&] {
+                store(kV);
+                if (n + 1 < n1) request_k(n + 1);
+            };
+            if (kh == 1) stage_v();
+            if (live) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) s[e] = 0.0f, sl[e] = 0.0f;
+                // the next block's parts are read ahead of a block's MFMAs; two chains
+                // alternate, so no MFMA waits for the one before it
+                u32x4 k[2][5];
+                auto read = [&](int b) {
+#pragma unroll
+                    for (int p = 0; p < 3; ++p)
+                        k[b % 2][p] = *reinterpret_cast<const u32x4*>(
+                            Ks + p * L::KP + col * L::KROW + L::kslot(col, 2 * b + hf) * 16);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        k[b % 2][3 + i] = *reinterpret_cast<const u32x4*>(q1 + (2 * b + i) * 1024);
+                };
+                read(0);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    if (b + 1 < NB) read(b + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    const u32x4(&kb)[5] = k[b % 2];
+                    sl = mfma_bf16(kb[2], q[b], sl);
+                    s = mfma_bf16(kb[1], q[b], s);
+                    sl = mfma_bf16(kb[0], kb[4], sl);
+                    s = mfma_bf16(kb[0], kb[3], s);
+                    sl = mfma_bf16(kb[1], kb[3], sl);
+                    s = mfma_bf16(kb[0], q[b], s);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (kh == 0) stage_v();
+            u32x4 p[2][3];
+            if (live) {
+                s += sl;
+                // causal mask (tiles that reach past the wave's first query) and the
+                // query's running max / sum
+                if (kt * 32 + 31 > len + 32 * mytile) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int kpos = kt * 32 + 8 * (r / 4) + 4 * hf + r % 4;
+                        if (kpos > qpos || kpos >= total) s[r] = -INFINITY;
+                    }
+                }
+                float tmax = s[0];
+#pragma unroll
+                for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
+                tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+                tmax *= kLog2e;
+                // O^T = alpha O^T + V^T . P^T.  The rescale moves the accumulators through
+                // the VALU, so the reference the exponentials are taken against follows
+                // the running max only when some query's rises past it by 8 (2^8 a sum's
+                // terms at most): with random keys the max itself rises in most tiles.
+                if (__any(tmax > mrun + 8.0f)) {
+                    const float mnew = fmaxf(mrun, tmax);
+                    // (no live key yet: mrun and mnew are -inf, o and l zero)
+                    const float alpha = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(mrun - mnew);
+                    lrun *= alpha;
+#pragma unroll
+                    for (int t = 0; t < OT; ++t)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
+                    mrun = mnew;
+                }
+                const float ref = mrun == -INFINITY ? 0.0f : mrun;  // (all p are 0 then)
+                float tsum = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], kLog2e, -ref));
+                    tsum += s[r];
+                }
+                lrun += tsum + __shfl_xor(tsum, 32, 64);
+                split8(s, 0, p[0]);
+                split8(s, 8, p[1]);
+            }
+            __syncthreads();  // V of step n is staged, K of step n read
+            auto stage_k = [&] {
+                if (n + 1 < n1) {
+                    store(kK);
+                    request_v(n + 1);
+                }
+            };
+            if (kh == 1) stage_k();
+            if (live) {
+                // unit u: output tiles 2 (u / 2) and + 1, keys of MFMA u % 2; the next unit's
+                // parts are read ahead
+                u32x4 v[2][2][3];
+                auto read = [&](int u) {
+#pragma unroll
+                    for (int a = 0; a < 2; ++a)
+#pragma unroll
+                        for (int i = 0; i < 3; ++i)
+                            v[u % 2][a][i] = *reinterpret_cast<const u32x4*>(
+                                Vs + i * L::VP + (u / 2 * 2 + a) * 32 * 64 + voff +
+                                (((2 * (u % 2) + hf) ^ vsw) * 16));
+                };
+                read(0);
+#pragma unroll
+                for (int u = 0; u < OT; ++u) {
+                    if (u + 1 < OT) read(u + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    constexpr int kVi[6] = {2, 0, 1, 1, 0, 0}, kPi[6] = {0, 2, 1, 0, 1, 0};
+                    const int t = u / 2 * 2;
+#pragma unroll
+                    for (int i = 0; i < 6; ++i)
+#pragma unroll
+                        for (int a = 0; a < 2; ++a)
+                            o[t + a] = mfma_bf16(v[u % 2][a][kVi[i]], p[u % 2][kPi[i]], o[t + a]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (kh == 0) stage_k();
+        }
+
+        // the tile's two waves: the odd key tiles' sums through LDS to the even ones'
+        {
+            float* ox = reinterpret_cast<float*>(lds) + (qt * (D / 2 + 2)) * 64 + lane;
+            __syncthreads();
+            if (kh == 1) {
+                ox[0] = mrun;
+                ox[64] = lrun;
+#pragma unroll
+                for (int t = 0; t < OT; ++t)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) ox[(2 + 16 * t + e) * 64] = o[t][e];
+            }
+            __syncthreads();
+            if (kh == 1) continue;
+            const float m1 = ox[0], l1 = ox[64];
+            const float mm = fmaxf(mrun, m1);
+            // (a wave without live keys left -inf: weight 0)
+            const float f0 = mrun == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mrun - mm);
+            const float f1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - mm);
+            lrun = lrun * f0 + l1 * f1;
+            mrun = mm;
+#pragma unroll
+            for (int t = 0; t < OT; ++t)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    o[t][e] = fmaf(o[t][e], f0, ox[(2 + 16 * t + e) * 64] * f1);
+        }
+        if (qi >= m) continue;
+        // O[q][32 t + 8 u + 4 hf + 0..3] = o[t][4 u + 0..3] / l, a float4 each; or, split,
+        // partials as attn_merge_split_kernel reads them: (max, sum) at [q H + h][S], o at
+        // [q H + h][S][hd] after all the pairs (a query with no live tile in this split
+        // leaves (-inf, 0) and zeros, weight 0 in the merge)
+        const int64_t qc = ((int64_t)qi * H + h) * S + z;
+        float* orow = (S > 1 ? part + (int64_t)m * H * S * 2 + qc * D
+                             : out + (int64_t)qi * H * D + (int64_t)h * D) + 4 * hf;
+        float* ml = S > 1 ? part + 2 * qc : nullptr;
+        if (ml && hf == 0) *reinterpret_cast<float2*>(ml) = make_float2(mrun, lrun);
+        const float inv = S > 1 ? 1.0f : 1.0f / lrun;
+        float chk = lrun * 0.0f;
+#pragma unroll
+        for (int t = 0; t < OT; ++t)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float4 v = make_float4(o[t][4 * u] * inv, o[t][4 * u + 1] * inv,
+                                             o[t][4 * u + 2] * inv, o[t][4 * u + 3] * inv);
+                *reinterpret_cast<float4*>(orow + 32 * t + 8 * u) = v;
+                chk = fmaf(v.x, 0.0f, fmaf(v.y, 0.0f, fmaf(v.z, 0.0f, fmaf(v.w, 0.0f, chk))));
+            }
+        const int bad = chk != 0.0f;  // (inf and NaN leave NaN)
+        if (bad | __shfl_xor(bad, 32, 64)) {
+            // a non-finite query again in plain f32 over this split's keys, by the two
+            // lanes that hold it.  Rolled loops over the rotated query in LDS, 8 outputs a
+            // pass: it takes no registers from the loop above.
+            float* qf = reinterpret_cast<float*>(lds) + qt * NB * 8 * 64 + lane;  // [16 b's 8][64]
+            const float* row = qkv + (int64_t)qi * (H + 2 * KVH) * D + (int64_t)h * D;
+#pragma unroll 1
+            for (int i = 0; i < NB * 4; ++i) {
+                const int p = 16 * (i / 8) + 8 * hf + i % 8;
+                float sn, cs;
+                sincosf((float)qpos * inv_freq[p], &sn, &cs);
+                const float a = row[p], c = row[p + D / 2];
+                qf[i * 64] = (a * cs - c * sn) * scale;
+                qf[(i + NB * 4) * 64] = (a * sn + c * cs) * scale;
+            }
+            auto score = [&](int kk) {  // of key kk: both lanes return the whole dot
+                float sc = 0.0f;
+#pragma unroll 1
+                for (int i = 0; i < NB * 8; ++i)
+                    sc = fmaf(qf[i * 64], kg[(int64_t)kk * D + 16 * (i / 8) + 8 * hf + i % 8], sc);
+                return sc + __shfl_xor(sc, 32, 64);
+            };
+            const int k0 = 64 * n0, k1 = min(64 * n1, qpos + 1);
+            float mx = -INFINITY, l = 0.0f;
+#pragma unroll 1
+            for (int kk = k0; kk < k1; ++kk) mx = fmaxf(mx, score(kk));
+#pragma unroll 1
+            for (int kk = k0; kk < k1; ++kk) l += expf(score(kk) - mx);
+            if (ml && hf == 0) *reinterpret_cast<float2*>(ml) = make_float2(mx * kLog2e, l);
+            const float f = S > 1 ? 1.0f : 1.0f / l;
+#pragma unroll 1
+            for (int c = 0; c < D / 16; ++c) {  // outputs 16 c + 4 hf .. + 3 and + 8 ..
+                float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+                for (int kk = k0; kk < k1; ++kk) {
+                    const float pe = expf(score(kk) - mx);
+                    const float* vr = vg + (int64_t)kk * D + 16 * c + 4 * hf;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) a[j] = fmaf(pe, vr[8 * (j / 4) + j % 4], a[j]);
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j) orow[16 * c + 8 * (j / 4) + j % 4] = a[j] * f;
+            }
+        }
     }
 }
 
 // The merge of a split prompt call (S splits of each workgroup's key tiles, a handful):
-// a thread per (query q, head h, 4 dimensions); out = sum_z e^(M_z - M) o_z /
-// sum_z e^(M_z - M) l_z over the splits' (M_z, l_z, o_z) partials (a split in which the
+// a thread per (query q, head h, 4 dimensions); out = sum_z 2^(M_z - M) o_z /
+// sum_z 2^(M_z - M) l_z over the splits' (M_z, l_z, o_z) partials (a split in which the
 // query had no live key leaves M_z = -inf: weight 0).  The length advance and the
 // overflow report are attn_merge_kernel's.
 template <int D>
@@ -944,7 +1152,7 @@ __global__ __launch_bounds__(256) void attn_merge_split_kernel(const float* __re
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int z = 0; z < S; ++z) {
         const float2 p = ms[z];
-        const float f = p.x == -INFINITY ? 0.0f : expf(p.x - M);
+        const float f = p.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(p.x - M);
         const float4 v = po[(int64_t)z * (D / 4)];
         l = fmaf(p.y, f, l);
         o = make_float4(fmaf(v.x, f, o.x), fmaf(v.y, f, o.y), fmaf(v.z, f, o.z), fmaf(v.w, f, o.w));
@@ -953,45 +1161,45 @@ __global__ __launch_bounds__(256) void attn_merge_split_kernel(const float* __re
     reinterpret_cast<float4*>(out)[i] = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
 }
 
-template <int D, int NW>
-hipError_t launch_prefill_mfma(const KvCache& kv, const float* qkv, int m, int H, float* qw,
-                               float* part, int S, float* out, hipStream_t s) {
-    using L = MfmaPrefillLds<D, NW>;
-    static const bool attr = hipFuncSetAttribute((const void*)attn_prefill_mfma<D, NW>,
+// How a prompt call is dealt out: QT query tiles a block, blocks paired or not, S splits
+// of the key tiles.
+struct PromptPlan {
+    int qt, paired, S;
+};
+
+template <int D, int QT>
+hipError_t launch_prompt_qt(const KvCache& kv, const float* qkv, int m, int H, float* part,
+                            const PromptPlan& plan, float* out, hipStream_t s) {
+    using L = PromptLds<D, QT>;
+    static const bool attr = hipFuncSetAttribute((const void*)attn_prompt_kernel<D, QT>,
                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 (int)L::BYTES) == hipSuccess;
+                                                 L::BYTES) == hipSuccess;
     if (!attr) return hipErrorInvalidValue;
     const int KVH = (int)kv.n_kv_heads;
-    rope_append_kernel<D><<<dim3((unsigned)m, (unsigned)(H + KVH)), D / 2, 0, s>>>(
-        qkv, m, H, KVH, kv.state, 1.0f / sqrtf((float)D), kv.inv_freq, kv.k, kv.v,
-        (int)kv.max_seq, qw);
+    const float scale = 1.0f / sqrtf((float)D);
+    rope_append_kernel<D><<<dim3((unsigned)m, (unsigned)KVH), D / 2, 0, s>>>(
+        qkv, m, H, KVH, kv.state, scale, kv.inv_freq, kv.k, kv.v, (int)kv.max_seq, nullptr, H);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    // pairs of 32-query tiles, NW / 2 pairs a workgroup; S splits of the key tiles
-    const int pairs = ((m + 31) / 32 + 1) / 2;
-    attn_prefill_mfma<D, NW><<<dim3((unsigned)((pairs + NW / 2 - 1) / (NW / 2)), (unsigned)H,
-                                    (unsigned)S),
-                               64 * NW, L::BYTES, s>>>(qw, m, H, KVH, kv.state, kv.k, kv.v,
-                                                       (int)kv.max_seq, out, part);
+    const int blocks = (m + 32 * QT - 1) / (32 * QT);
+    const int grid = plan.paired ? (blocks + 1) / 2 : blocks;
+    attn_prompt_kernel<D, QT><<<dim3((unsigned)grid, (unsigned)H, (unsigned)plan.S), 128 * QT,
+                                L::BYTES, s>>>(qkv, m, H, KVH, kv.state, scale, kv.inv_freq, kv.k,
+                                               kv.v, (int)kv.max_seq, blocks, plan.paired, out,
+                                               part);
     e = hipGetLastError();
-    if (S == 1 || e != hipSuccess) return e;
+    if (plan.S == 1 || e != hipSuccess) return e;
     const int64_t merge_threads = (int64_t)m * H * (D / 4);
     attn_merge_split_kernel<D><<<(unsigned)((merge_threads + 255) / 256), 256, 0, s>>>(
-        part, m, H, S, out, kv.state, (int)kv.max_seq);
+        part, m, H, plan.S, out, kv.state, (int)kv.max_seq);
     return hipGetLastError();
 }
 
-// The largest workgroup (8, 4 or 2 waves of 32 queries) whose grid, with the call's S
-// key splits, still gives every CU a workgroup: eight waves are two a SIMD (the K and V
-// tiles in LDS allow only two workgroups a CU).
 template <int D>
-hipError_t launch_prefill_mfma_auto(const KvCache& kv, const float* qkv, int m, int H, float* qw,
-                                    float* part, int S, float* out, hipStream_t s) {
-    const int64_t cus = device_info().cu_count, pairs = ((m + 31) / 32 + 1) / 2;
-    auto wgs = [&](int nw) { return (pairs + nw / 2 - 1) / (nw / 2) * H * S; };
-    if (wgs(8) >= cus) return launch_prefill_mfma<D, 8>(kv, qkv, m, H, qw, part, S, out, s);
-    if (wgs(4) >= cus) return launch_prefill_mfma<D, 4>(kv, qkv, m, H, qw, part, S, out, s);
-    return launch_prefill_mfma<D, 2>(kv, qkv, m, H, qw, part, S, out, s);
+hipError_t launch_prompt(const KvCache& kv, const float* qkv, int m, int H, float* part,
+                         const PromptPlan& plan, float* out, hipStream_t s) {
+    return plan.qt == 4 ? launch_prompt_qt<D, 4>(kv, qkv, m, H, part, plan, out, s)
+                        : launch_prompt_qt<D, 2>(kv, qkv, m, H, part, plan, out, s);
 }
 
 template <int D, int BQ, int BK>
@@ -1005,7 +1213,7 @@ hipError_t launch_prefill_attn(const KvCache& kv, const float* qkv, int m, int H
     const int KVH = (int)kv.n_kv_heads;
     rope_append_kernel<D><<<dim3((unsigned)m, (unsigned)(H + KVH)), D / 2, 0, s>>>(
         qkv, m, H, KVH, kv.state, 1.0f / sqrtf((float)D), kv.inv_freq, kv.k, kv.v,
-        (int)kv.max_seq, qw);
+        (int)kv.max_seq, qw, 0);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     attn_prefill_kernel<D, BQ, BK><<<dim3((unsigned)((m + BQ - 1) / BQ), (unsigned)H), 256,
@@ -1017,17 +1225,47 @@ hipError_t launch_prefill_attn(const KvCache& kv, const float* qkv, int m, int H
 }  // namespace
 
 namespace {
-// Key-range splits of a prompt call on the matrix-core kernel: the largest of 1, 2, 4
-// that keeps the call's 32-query waves at most two a SIMD (m512 at 32 heads: 512
-// waves on 1024 SIMDs, 4 splits); 1 needs no partials and no merge.
-int prompt_split(int64_t m, int64_t H, int64_t D) {
-    if (D != 64 && D != 128) return 1;
-    const int64_t waves = (m + 31) / 32 * H, target = 8 * (int64_t)device_info().cu_count;
-    int S = 1;
-    while (S < 4 && waves * 2 * S <= target) S *= 2;
-    return S;
+// A prompt call's plan: the cheapest of 4- and 2-tile blocks, paired or not, with the key
+// tiles in 1, 2, 4 or 8 splits (at most two workgroups a CU), by the longest workgroup's
+// steps times the rounds over the CUs, plus the partials written, read and merged.  A step
+// of a 4-tile block was measured at 6.5 us (hd 128; 3.6 at hd 64), of a 2-tile one at 3/4 of
+// it; a block's queries and its merge cost about two steps.  Measured against every choice
+// (us a call, with the 21 of the rewind before it): m2048 at 32 heads of 128 paired 267,
+// unpaired 411, split in two 314; m500 behind 777 at 32 heads of 64 unpaired in two splits
+// 75, paired in four 82, whole 97; m250 at 32 heads of 64 2-tile blocks in two splits 49.
+constexpr int kMaxPromptSplit = 8;
+constexpr int64_t kPromptRounds = 2;  // workgroups a CU when the keys are split
+
+PromptPlan prompt_plan(int64_t m, int64_t H, int64_t D, int64_t len) {
+    if (D != 64 && D != 128) return {4, 0, 1};
+    const int64_t cus = device_info().cu_count;
+    PromptPlan best{4, 1, 1};
+    int64_t least = INT64_MAX;
+    for (int qt : {4, 2})
+        for (int paired = 1; paired >= 0; --paired) {
+            const int64_t blocks = (m + 32 * qt - 1) / (32 * qt);
+            const int64_t wgs = (paired ? (blocks + 1) / 2 : blocks) * H;
+            // the key steps (64 positions) of the first, last and so of a pair of blocks
+            const int64_t last = (len + m + 63) / 64, first = (len + std::min<int64_t>(m, 32 * qt) + 63) / 64;
+            const int64_t steps = paired && blocks > 1 ? first + last : last;
+            const int64_t nblk = paired && blocks > 1 ? 2 : 1;
+            const int64_t step_ns = (D == 128 ? 6500 : 3600) * (qt == 4 ? 4 : 3) / 4;
+            for (int S = 1; S <= kMaxPromptSplit; S *= 2) {
+                if (S > 1 && (wgs * S > kPromptRounds * cus || S > last)) break;
+                const int64_t rounds = (wgs * S + cus - 1) / cus;
+                int64_t ns = rounds * ((steps + S - 1) / S + 2 * nblk) * step_ns;
+                if (S > 1) ns += 3000 + S * m * H * D * 8 / 3000;
+                if (ns < least) {
+                    least = ns;
+                    best = {qt, paired, S};
+                }
+            }
+        }
+    return best;
 }
+// hd 256's rotated queries [H][m][hd] (the matrix-core kernel rotates its own)
 size_t prompt_q_bytes(int64_t m, int64_t H, int64_t D) {
+    if (D == 64 || D == 128) return 0;
     return ((size_t)m * H * D * sizeof(float) + 255) / 256 * 256;
 }
 }  // namespace
@@ -1037,27 +1275,26 @@ namespace {
 // any length (at most kMaxChunks chunks of (max, sum) and o[hd] per query), or the
 // prompt path's rotated queries [H][m][hd] followed, for a split call, by its S
 // partials per query.
-size_t attention_call_bytes(const KvCache& kv, int64_t m, int64_t H) {
+size_t attention_call_bytes(const KvCache& kv, int64_t m, int64_t H, int S) {
     const int64_t G = H / std::max<int64_t>(kv.n_kv_heads, 1), D = kv.head_dim;
     if (m * G <= kAttnMaxQ) return (size_t)m * H * kMaxChunks * (2 + D) * sizeof(float);
-    const int S = prompt_split(m, H, D);
     return prompt_q_bytes(m, H, D) + (S > 1 ? (size_t)m * H * S * (2 + D) * sizeof(float) : 0);
 }
 }  // namespace
 
-// Enough for every call of up to m tokens (what unillm_hip_attention_reserve grows to).
-// A call's need grows with m inside each regime -- decode, then prompts with 4, 2 and
-// 1 key splits -- but not across them (a split 512-token prompt takes more than an
-// unsplit 2048-token one), so the largest lies at the right end of a regime, clipped
-// to m.
+// Enough for every call of up to m tokens (what unillm_hip_attention_reserve grows to): the
+// longest decode step's partials, and a prompt's.  A split prompt's partial rows (S m H) are
+// at most kMaxPromptSplit m H, and, as its workgroups are at most kPromptRounds a CU and
+// hold at most two blocks of 128 queries each, at most 256 kPromptRounds CUs.
 size_t attention_workspace_bytes(const KvCache& kv, int64_t m, int64_t H) {
-    const int64_t G = H / std::max<int64_t>(kv.n_kv_heads, 1);
-    const int64_t target = 8 * (int64_t)device_info().cu_count;  // prompt_split's two a SIMD
-    const int64_t ends[4] = {m, kAttnMaxQ / G, 32 * (target / (4 * H)), 32 * (target / (2 * H))};
+    const int64_t G = H / std::max<int64_t>(kv.n_kv_heads, 1), D = kv.head_dim;
     size_t need = 0;
-    for (int64_t c : ends) {
-        c = std::min(c, m);
-        if (c >= 1) need = std::max(need, attention_call_bytes(kv, c, H));
+    const int64_t md = std::min(m, kAttnMaxQ / G);
+    if (md >= 1) need = attention_call_bytes(kv, md, H, 1);
+    if (m * G > kAttnMaxQ) {
+        const int64_t rows = std::min<int64_t>(kMaxPromptSplit * m * H,
+                                               256 * kPromptRounds * (int64_t)device_info().cu_count);
+        need = std::max(need, prompt_q_bytes(m, H, D) + (size_t)rows * (2 + D) * sizeof(float));
     }
     return need;
 }
@@ -1068,15 +1305,17 @@ hipError_t launch_attention(const KvCache& kv, const float* qkv, int64_t m, int6
     void* ws = nullptr;
     hipError_t e;
     if (m * (H / kv.n_kv_heads) > kAttnMaxQ) {
-        if ((e = stream_workspace(s, attention_call_bytes(kv, m, H), &ws, 2)) != hipSuccess)
+        // (captured: the length at a replay is not known; planned for an empty cache)
+        const PromptPlan plan = prompt_plan(m, H, D, std::max<int64_t>(len_hint, 0));
+        if ((e = stream_workspace(s, std::max<size_t>(attention_call_bytes(kv, m, H, plan.S), 16),
+                                  &ws, 2)) != hipSuccess)
             return e;
         float* qw = static_cast<float*>(ws);
         float* part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + prompt_q_bytes(m, H, D));
-        const int S = prompt_split(m, H, D);
         if (D == 64)
-            return launch_prefill_mfma_auto<64>(kv, qkv, (int)m, (int)H, qw, part, S, out, s);
+            return launch_prompt<64>(kv, qkv, (int)m, (int)H, part, plan, out, s);
         if (D == 128)
-            return launch_prefill_mfma_auto<128>(kv, qkv, (int)m, (int)H, qw, part, S, out, s);
+            return launch_prompt<128>(kv, qkv, (int)m, (int)H, part, plan, out, s);
         return launch_prefill_attn<256, 32, 32>(kv, qkv, (int)m, (int)H, qw, out, s);
     }
     // decode: chunks sized for the known length, or for the longest the cache holds

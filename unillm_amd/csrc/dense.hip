@@ -35,6 +35,7 @@
 
 #include "internal.hpp"
 #include "lds.hpp"
+#include "split.hpp"
 
 namespace unillm {
 namespace {
@@ -417,25 +418,16 @@ __device__ __forceinline__ f32x4 mfma_parts(u32x4 a, u32x4 b, f32x4 c) {
                                                        __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// two f32 (as bits) -> their upper halves packed, lo in the low half
-__device__ __forceinline__ uint32_t pack_hi(uint32_t lo, uint32_t hi) {
-    return __builtin_amdgcn_perm(hi, lo, 0x07060302u);
-}
-
-// 8 f32 weights -> three bf16 parts (truncation, as xsplit_kernel's; an infinity's or a
-// NaN's lower parts come out NaN: the output is recomputed)
+// 8 f32 weights -> three bf16 parts (an infinity's or a NaN's lower parts come out NaN:
+// the output is recomputed)
 __device__ __forceinline__ void split8(const u32x4 (&w)[2], u32x4 (&p)[3]) {
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
-        const uint32_t a = w[h / 2][2 * (h % 2)], b = w[h / 2][2 * (h % 2) + 1];
-        p[0][h] = pack_hi(a, b);
-        const float a1 = __uint_as_float(a) - __uint_as_float(a & 0xFFFF0000u);
-        const float b1 = __uint_as_float(b) - __uint_as_float(b & 0xFFFF0000u);
-        const uint32_t ua = __float_as_uint(a1), ub = __float_as_uint(b1);
-        p[1][h] = pack_hi(ua, ub);
-        const float a2 = a1 - __uint_as_float(ua & 0xFFFF0000u);
-        const float b2 = b1 - __uint_as_float(ub & 0xFFFF0000u);
-        p[2][h] = pack_hi(__float_as_uint(a2), __float_as_uint(b2));
+        uint32_t p0, p1, p2;
+        split2(w[h / 2][2 * (h % 2)], w[h / 2][2 * (h % 2) + 1], p0, p1, p2);
+        p[0][h] = p0;
+        p[1][h] = p1;
+        p[2][h] = p2;
     }
 }
 

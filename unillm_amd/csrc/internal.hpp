@@ -165,8 +165,8 @@ const DeviceInfo& device_info();
 // memory is held until the process ends.  Calls on one stream from several
 // host threads are ordered by the stream, the map by a mutex.
 // Slot 0 holds x in the MFMA paths' operand type; slot 1 the [gate | up] outputs
-// of a SwiGLU call off the GEMV path (both live during that call); slot 2 the
-// rotated queries and the per-chunk partials of decode attention; slot 3 an
+// of a SwiGLU call off the GEMV path (both live during that call); slot 2
+// attention's partials (and, for hd 256 prompts, the rotated queries); slot 3 an
 // aligned copy of x; slot kSyncSlot the batched decode's arrival tickets, zeroed
 // when allocated (every launch leaves them zero again); slot kDenseSlot a dense
 // weight's x in 16-bit parts and its split-k slabs.
