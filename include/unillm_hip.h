@@ -178,8 +178,8 @@ int unillm_hip_qmatmul_add(const unillm_qweight* w, const float* x_dev, int64_t 
  * tensor_core.rs:1385-1396: candle silu(v) = v / (1 + e^-v)).  On the GEMV path
  * (m = 1: k <= 8192 for Q4_0 / Q4_K, 4096 for Q8_0 / Q5_K / Q6_K; half that at m = 2,
  * a quarter at m = 3, 4) the gate and up rows meet in one wave and the
- * activation is its epilogue; otherwise the
- * [m, 2 I] product goes to a per-stream workspace and one elementwise pass
+ * activation is its epilogue, as it is the prefill's; the batched decode stores the
+ * [m, 2 I] product to a per-stream workspace and one elementwise pass
  * follows.  n odd is an error. */
 int unillm_hip_qmatmul_swiglu(const unillm_qweight* w, const float* x_dev, int64_t m,
                               float* act_dev, void* stream);

@@ -431,7 +431,8 @@ int dense_impl(const unillm_qweight* w, const float* x, int64_t m, float* y, int
 }
 
 // The matmul on `path` with epilogue `epi` (kEpiStore / kEpiAdd; kEpiSwiglu runs
-// fused on the GEMV, else as store into the stream's second workspace + swiglu).
+// fused on the GEMV and the prefill, else as store into the stream's second workspace +
+// swiglu).
 // `what` prefixes every error message (the caller's anyhow context).
 // fixed_ws != nullptr (the no-allocation entry point, store epilogue only): the MFMA
 // paths take their x operand from fixed_ws (fixed_bytes long), and nothing allocates.
@@ -502,7 +503,9 @@ int qmatmul_impl(const unillm_qweight* w, const float* x_dev, int64_t m, float* 
     }
     float* out = y_dev;
     int run_epi = epi;
-    if (epi == kEpiSwiglu && !(path == UNILLM_PATH_GEMV && gemv_supports_swiglu(*w, m))) {
+    if (epi == kEpiSwiglu && path != UNILLM_PATH_PREFILL_MFMA &&
+        !(path == UNILLM_PATH_DECODE_MFMA && prefill_takes_batch(*w, m)) &&
+        !(path == UNILLM_PATH_GEMV && gemv_supports_swiglu(*w, m))) {
         void* ws = nullptr;
         e = stream_workspace(s, (size_t)m * (size_t)w->n * sizeof(float), &ws, 1);
         if (e != hipSuccess) return fail_launch(e, what + ": workspace");

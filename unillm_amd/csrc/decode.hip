@@ -1338,7 +1338,8 @@ size_t decode_x_bytes(const QWeight& w, int64_t m) {
 
 size_t decode_workspace_bytes(const QWeight& w, int64_t m, const NormArgs& norm) {
     if (decode_one_launch(w, m, norm)) return 0;
-    return decode_x_bytes(w, m) + (size_t)decode_split(w, m) * 64 * sizeof(float);
+    const size_t own = decode_x_bytes(w, m) + (size_t)decode_split(w, m) * 64 * sizeof(float);
+    return prefill_takes_batch(w, m) ? std::max(own, prefill_call_bytes(w, m)) : own;
 }
 
 size_t decode_sync_bytes(const QWeight& w) { return xin_sync_bytes((w.n + DROWS - 1) / DROWS); }
@@ -1352,6 +1353,9 @@ hipError_t launch_decode_mfma(const QWeight& w, const float* x, int64_t m, float
     const bool q4 = w.qtype == UNILLM_QTYPE_Q4_0, k4 = w.qtype == UNILLM_QTYPE_Q4_K,
                k5 = w.qtype == UNILLM_QTYPE_Q5_K, k6 = w.qtype == UNILLM_QTYPE_Q6_K, wide = m > 32;
     hipError_t e = hipSuccess;
+    if (prefill_takes_batch(w, m))  // (deep or large weights at 33 .. 64 rows)
+        return launch_prefill_mfma(w, x, m, y, s, epi, norm, ws,
+                                   ws ? decode_workspace_bytes(w, m, norm) : 0);
     if (decode_one_launch(w, m, norm)) {
         // x converted by the kernel itself; the stream's workspace holds the row groups'
         // arrival tickets (zeroed when allocated, reset by each launch)

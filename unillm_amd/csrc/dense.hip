@@ -58,16 +58,15 @@ float* dense_wsc(const QWeight& w) {
 
 // ---- upload, dequant, layer norm ---------------------------------------------------------
 
-// dst row r (row_bytes) <- src row r (k elements of ES bytes, ES-aligned); the padding
-// was zeroed when the weight was allocated
+// dst row r (row_bytes) <- src row r (k elements), a workgroup a row; the padding was
+// zeroed when the weight was allocated
 template <class T>
 __global__ __launch_bounds__(256) void dense_upload_kernel(const T* __restrict__ src,
-                                                           uint8_t* __restrict__ dst, int64_t n,
-                                                           int64_t k, int64_t row_bytes) {
-    const int64_t count = n * k;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
-         i += (int64_t)gridDim.x * blockDim.x)
-        reinterpret_cast<T*>(dst + i / k * row_bytes)[i % k] = src[i];
+                                                           uint8_t* __restrict__ dst, int64_t k,
+                                                           int64_t row_bytes) {
+    const T* sr = src + (int64_t)blockIdx.x * k;
+    T* dr = reinterpret_cast<T*>(dst + (int64_t)blockIdx.x * row_bytes);
+    for (int64_t i = threadIdx.x; i < k; i += 256) dr[i] = sr[i];
 }
 
 // the same for F16, each row scaled (wsc[row] <- the undoing factor); a workgroup a row
@@ -766,22 +765,20 @@ size_t dense_extra_bytes(int qtype, int64_t n) {
 int64_t dense_row_bytes(int qtype, int64_t k) { return padded_k(k) * dense_elem_bytes(qtype); }
 
 hipError_t launch_dense_upload(const QWeight& w, const void* src, hipStream_t s) {
-    const int64_t count = w.n * w.k;
     if (w.qtype == UNILLM_QTYPE_F16) {
         dense_upload_f16_kernel<<<(unsigned)w.n, 256, 0, s>>>(static_cast<const uint16_t*>(src),
                                                               w.base, w.k, w.row_bytes, dense_wsc(w));
         return hipGetLastError();
     }
     if (w.k % kKPad == 0)
-        return hipMemcpyAsync(w.base, src, (size_t)count * dense_elem_bytes(w.qtype),
+        return hipMemcpyAsync(w.base, src, (size_t)w.n * (size_t)w.row_bytes,
                               hipMemcpyDeviceToDevice, s);
-    const int blocks = (int)std::min<int64_t>((count + 255) / 256, 8 * device_info().cu_count);
     if (w.qtype == UNILLM_QTYPE_F32)
-        dense_upload_kernel<<<blocks, 256, 0, s>>>(static_cast<const uint32_t*>(src), w.base, w.n,
-                                                   w.k, w.row_bytes);
+        dense_upload_kernel<<<(unsigned)w.n, 256, 0, s>>>(static_cast<const uint32_t*>(src), w.base,
+                                                          w.k, w.row_bytes);
     else
-        dense_upload_kernel<<<blocks, 256, 0, s>>>(static_cast<const uint16_t*>(src), w.base, w.n,
-                                                   w.k, w.row_bytes);
+        dense_upload_kernel<<<(unsigned)w.n, 256, 0, s>>>(static_cast<const uint16_t*>(src), w.base,
+                                                          w.k, w.row_bytes);
     return hipGetLastError();
 }
 

@@ -185,8 +185,8 @@ hipError_t launch_dequant(const QWeight& w, float* out, hipStream_t s);
 hipError_t launch_scale_absmax(const QWeight& w, uint32_t* out, hipStream_t s);
 hipError_t launch_quantize(int qtype, const float* w, int64_t n, int64_t k, uint8_t* out,
                            hipStream_t s);
-// epi: kEpiStore or kEpiAdd on every path; kEpiSwiglu on the GEMV only
-// (gemv_supports_swiglu), the other paths run it as store + swiglu_kernel.
+// epi: kEpiStore or kEpiAdd on every path; kEpiSwiglu on the GEMV (gemv_supports_swiglu) and
+// the prefill's tiles, the batched decode's own kernels run it as store + swiglu_kernel.
 hipError_t launch_gemv(const QWeight& w, const float* x, int64_t m, float* y, hipStream_t s,
                        int epi = kEpiStore, const NormArgs& norm = NormArgs{nullptr, nullptr, 0.f});
 // The MFMA paths take their x operand buffer from `ws` when it is given (at least
@@ -210,6 +210,9 @@ size_t decode_sync_bytes(const QWeight& w);
 // The prefill's workspace: this call's own need (cap > 0: in a fixed workspace of
 // cap bytes, which may pick a plan without a k split), and a bound for every call
 // of up to m rows (the size a reserve takes).
+// (prefill_takes_batch: calls of up to kDecodeMaxM rows that the batched decode's path
+// hands to the prefill's tiles)
+bool prefill_takes_batch(const QWeight& w, int64_t m);
 size_t prefill_call_bytes(const QWeight& w, int64_t m, size_t cap = 0);
 size_t prefill_workspace_bytes(const QWeight& w, int64_t m);
 // Both MFMA paths address weight bytes with 32-bit offsets: weights under 4 GiB.

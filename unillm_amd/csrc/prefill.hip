@@ -178,8 +178,8 @@ struct Ring {
     static constexpr int BH = KQ ? 2 * PBN * 4 : 0;  // K-quants: the step's group header per column
     static constexpr int STAGE = A + BP + BS + BH;
     // stages: 4 for 128-row tiles (four fit in LDS; ~10 % over three measured),
-    // 3 for 256-row tiles
-    static constexpr int STAGES = BM == 128 ? 4 : 3;
+    // 3 for 256-row tiles; four of 64-row tiles leave room for a second workgroup a CU
+    static constexpr int STAGES = BM <= 128 ? 4 : 3;
     // + the tile's row scales of x (f16 operands): BM floats after the ring
     static constexpr int BYTES = STAGES * STAGE + BM * 4;
     static constexpr int RS = STAGES * STAGE;
@@ -189,7 +189,7 @@ struct Ring {
 };
 
 template <int QT, int BM, int NW>
-__global__ __launch_bounds__(NW * 64, 1) void prefill_kernel(const uint8_t* __restrict__ base,
+__global__ __launch_bounds__(NW * 64, BM == 64 ? 4 : 1) void prefill_kernel(const uint8_t* __restrict__ base,
                                                               int64_t rb,
                                                               const uint16_t* __restrict__ xb,
                                                               float* __restrict__ y, int M, int N,
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(NW * 64, 1) void prefill_kernel(const uint8_t* __re
                                                               int units_pad, int S, int add,
                                                               float wscale, float oscale,
                                                               const float* __restrict__ rs,
-                                                              float* __restrict__ part) {
+                                                              float* __restrict__ part, int swi) {
     static_assert(NW == 8, "the ring's load split assumes 8 waves");
     constexpr int QB = Ring<QT, BM>::QB;  // payload bytes per block
     // waves: RW row groups x CW column groups; wave (rw, cw) owns rows BM / RW * rw ..
@@ -227,6 +227,14 @@ __global__ __launch_bounds__(NW * 64, 1) void prefill_kernel(const uint8_t* __re
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m0 = mt * BM, n0 = nt * PBN;
+    // SwiGLU on a [gate; up] weight (swi = I, its rows of each): the tile's 256 columns are
+    // 128 gate rows and the 128 up rows of the same outputs, a wave's column tile 0 its 16
+    // gate rows and column tile 1 their up rows, so both meet in one lane.  Weight row of
+    // tile column c:
+    auto wrow = [&](int c) {
+        if (!swi) return min(n0 + c, N - 1);
+        return min(nt * (PBN / 2) + c / 32 * 16 + c % 16, swi - 1) + (c % 32 < 16 ? 0 : swi);
+    };
     const uint32_t K = (uint32_t)KB * QK;
     const int ksteps = (KB + 1) / 2;
     // this unit's k steps [ks0, ks0 + nks)
@@ -250,11 +258,10 @@ __global__ __launch_bounds__(NW * 64, 1) void prefill_kernel(const uint8_t* __re
     uint32_t pcol_off[CPB / 2];
 #pragma unroll
     for (int u = 0; u < CPB / 2; ++u)
-        pcol_off[u] = (uint32_t)min(n0 + 32 * wv + u * (64 / CPB) + lane / CPB, N - 1) * (uint32_t)rb;
+        pcol_off[u] = (uint32_t)wrow(32 * wv + u * (64 / CPB) + lane / CPB) * (uint32_t)rb;
     const int pblk = (lane % CPB) / (QB / 16);
     const uint32_t phalf = (uint32_t)((lane % CPB) % (QB / 16)) * 16;
-    const uint32_t ssrc = (uint32_t)min(n0 + 32 * wv + lane % 32, N - 1) * (uint32_t)rb +
-                          (uint32_t)KB * QB;
+    const uint32_t ssrc = (uint32_t)wrow(32 * wv + lane % 32) * (uint32_t)rb + (uint32_t)KB * QB;
 
     // direct load q (0 .. R::DMA - 1, in this order) of this wave's loads of step ks
     auto issue_one = [&](int ks, int q) {
@@ -293,7 +300,8 @@ __global__ __launch_bounds__(NW * 64, 1) void prefill_kernel(const uint8_t* __re
     const int rw = wv / CW, cw = wv % CW;
     bool bval[TJ];
 #pragma unroll
-    for (int j = 0; j < TJ; ++j) bval[j] = n0 + WC * cw + 16 * j + fr < N;
+    for (int j = 0; j < TJ; ++j)
+        bval[j] = swi ? nt * (PBN / 2) + 16 * cw + fr < swi : n0 + WC * cw + 16 * j + fr < N;
     // f16 dequant constants of this lane (high nibbles: 1024 + 16 q, scale / 16)
     const bool hnib = kNib && g >= 2;
     const uint32_t nmask = hnib ? 0x00F000F0u : 0x000F000Fu;
@@ -493,6 +501,21 @@ __global__ __launch_bounds__(NW * 64, 1) void prefill_kernel(const uint8_t* __re
             *reinterpret_cast<const float4*>(ring + R::RS + (WR * rw + 16 * i + 4 * g) * 4);
         rsc[i] = make_float4(r4.x * oscale, r4.y * oscale, r4.z * oscale, r4.w * oscale);
     }
+    if (swi) {  // act = silu(gate) * up (candle's silu, v / (1 + e^-v))
+        const int col = nt * (PBN / 2) + 16 * cw + fr;
+        if (col >= swi) return;
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = m0 + WR * rw + 16 * i + 4 * g + e;
+                if (row >= M) continue;
+                const float f = e == 0 ? rsc[i].x : e == 1 ? rsc[i].y : e == 2 ? rsc[i].z : rsc[i].w;
+                const float gv = acc[i][0][e] * f, uv = acc[i][1][e] * f;
+                y[(int64_t)row * swi + col] = gv / (1.0f + expf(-gv)) * uv;
+            }
+        return;
+    }
 #pragma unroll
     for (int j = 0; j < TJ; ++j) {
         const int col = n0 + WC * cw + 16 * j + fr;
@@ -541,21 +564,59 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict_
     }
 }
 
+// act[r, c] = silu(g) u for the [gate; up] product of a split k: g and u the sums over the
+// slabs of columns c and I + c, scaled as split_sum_kernel scales them (candle's silu,
+// v / (1 + e^-v)); no pass over the [m, 2 I] product is made.
+__global__ __launch_bounds__(256) void split_swiglu_kernel(const float* __restrict__ part, int S,
+                                                           int64_t M, int64_t I,
+                                                           const float* __restrict__ rs,
+                                                           float oscale, int vec,
+                                                           float* __restrict__ act) {
+    const int64_t MN = M * 2 * I;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const int64_t w = vec ? I / 4 : I;  // units of a row
+    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < M * w; q += stride) {
+        const int64_t row = q / w, c = (q - row * w) * (vec ? 4 : 1);
+        const float f = rs[row] * oscale;
+        const float* g0 = part + row * 2 * I + c;
+        if (vec) {
+            f32x4 g = *reinterpret_cast<const f32x4*>(g0), u = *reinterpret_cast<const f32x4*>(g0 + I);
+            for (int sl = 1; sl < S; ++sl) {
+                g += *reinterpret_cast<const f32x4*>(g0 + sl * MN);
+                u += *reinterpret_cast<const f32x4*>(g0 + sl * MN + I);
+            }
+            f32x4 a;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] = g[e] * f / (1.0f + expf(-(g[e] * f))) * (u[e] * f);
+            *reinterpret_cast<f32x4*>(act + row * I + c) = a;
+        } else {
+            float g = g0[0], u = g0[I];
+            for (int sl = 1; sl < S; ++sl) {
+                g += g0[sl * MN];
+                u += g0[sl * MN + I];
+            }
+            act[row * I + c] = g * f / (1.0f + expf(-(g * f))) * (u * f);
+        }
+    }
+}
+
 // x is addressed with 32-bit element offsets: a launch takes at most this many rows
 int64_t prefill_chunk_rows(int64_t k, int bm) {
     return std::max<int64_t>(bm, ((int64_t)1 << 30) / k / bm * bm);
 }
 
+// epi: kEpiStore, kEpiAdd, or kEpiSwiglu (y is then act[m, n / 2])
 template <int QT, int BM>
 hipError_t launch_bm(const QWeight& w, const uint16_t* xb, const float* rs, int64_t m, float* y,
-                     int S, float* part, hipStream_t s, int add) {
-    const int64_t chunk = prefill_chunk_rows(w.k, BM);
+                     int S, float* part, hipStream_t s, int epi) {
+    const int64_t chunk = prefill_chunk_rows(w.k, BM), I = w.n / 2;
+    const bool act = epi == kEpiSwiglu;
     if (m > chunk) {  // row chunks below 2^30 elements (the plan never splits k here)
         if (S != 1) return hipErrorInvalidValue;
         for (int64_t r = 0; r < m; r += chunk) {
-            hipError_t e =
-                launch_bm<QT, BM>(w, xb + r * w.k, rs ? rs + r : nullptr, std::min(chunk, m - r),
-                                  y + r * w.n, 1, nullptr, s, add);
+            hipError_t e = launch_bm<QT, BM>(w, xb + r * w.k, rs ? rs + r : nullptr,
+                                             std::min(chunk, m - r), y + r * (act ? I : w.n), 1,
+                                             nullptr, s, epi);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
@@ -566,45 +627,43 @@ hipError_t launch_bm(const QWeight& w, const uint16_t* xb, const float* rs, int6
                                    Ring<QT, BM>::BYTES) == hipSuccess;
     }();
     if (!attr) return hipErrorInvalidValue;
+    const int swi = act && S == 1 ? (int)I : 0;  // (a split k's sums meet in a pass of their own)
     const int tiles_m = (int)((m + BM - 1) / BM);
-    const int tiles_n = (int)((w.n + PBN - 1) / PBN);
+    const int tiles_n = (int)(swi ? (I + PBN / 2 - 1) / (PBN / 2) : (w.n + PBN - 1) / PBN);
     const int tiles = tiles_m * tiles_n;
     const int units_pad = (tiles * S + 7) / 8 * 8;
     const float wscale = ldexpf(1.0f, -w.f16_exp), oscale = ldexpf(1.0f, w.f16_exp);
     prefill_kernel<QT, BM, kWaves><<<units_pad, kWaves * 64, Ring<QT, BM>::BYTES, s>>>(
         w.base, w.row_bytes, xb, y, (int)m, (int)w.n, (int)w.kb, tiles_n, tiles, units_pad, S,
-        add, wscale, oscale, rs, part);
+        epi == kEpiAdd, wscale, oscale, rs, part, swi);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || S == 1) return e;
-    const int vec = w.n % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
-    const int64_t q = m * w.n / (vec ? 4 : 1);
-    const int blocks = (int)std::min<int64_t>((q + 255) / 256, 8 * device_info().cu_count);
-    split_sum_kernel<<<blocks, 256, 0, s>>>(part, S, m, w.n, rs, oscale, add, vec, y);
+    const int64_t cols = act ? I : w.n;
+    const int vec = cols % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+    const int64_t q = m * cols / (vec ? 4 : 1);
+    const int blocks =
+        (int)std::min<int64_t>(std::max<int64_t>(1, (q + 255) / 256), 8 * device_info().cu_count);
+    if (act)
+        split_swiglu_kernel<<<blocks, 256, 0, s>>>(part, S, m, I, rs, oscale, vec, y);
+    else
+        split_sum_kernel<<<blocks, 256, 0, s>>>(part, S, m, w.n, rs, oscale, epi == kEpiAdd, vec, y);
     return hipGetLastError();
 }
 
-// Tile rows and k split.  256-row tiles when they give at least one tile per CU,
-// unless 128-row tiles take no more rounds.
-// A deep product (128 k steps or more) whose 256-row tiles fill at most half the
-// CUs takes those tiles with the k steps split over up to CUs / tiles workgroups, at
-// least 16 steps each: where the tiles fill 3/8 to 1/2 of the CUs (a split in two:
-// m2048 k14336 n4096, 128 tiles, 256 workgroups; Q4_0 776-796 -> 866 TFLOP/s a call,
-// Q8_0 759-774 -> 897-902 against one 128-row tile a CU), and for m > 256 where
-// plan_cost rates them no dearer than the 128-row plan (m1024 k14336 n4096, 64 tiles in
-// 4 slices: Q4_0 163-169 -> 154-156 us a call against 128 tiles of 128 rows in 2;
-// m768, 48 tiles in 5: 159-161 -> 126-127).  Else 128-row tiles; when those fill at
-// most half the CUs (a short, deep product), the k steps are split over up to 16
-// workgroups per tile, at least 8 steps each; unless (m > 256) plan_cost rates the
-// 256-row tiles unsplit cheaper.  Split slices' raw sums meet in
-// split_sum_kernel (slabs of the stream's workspace).  Calls beyond the 32-bit x
-// offsets (chunked) never split.
+// Tile rows and k split: the cheapest of 64-, 128- and 256-row tiles with the k steps in up
+// to 16 slices of at least 4 steps (a split grid at most one workgroup a CU), by the rounds
+// over the CUs times the steps of a workgroup times what a step was measured to take (ns;
+// taller tiles dequantize a weight once for more rows, which counts most where the dequant
+// is dear), plus a split's slabs written and read once (4 TB/s) and the summing launch.
+// Measured against every choice, us a call (graph replays): Q4_0 k4096 n4096 m100 27.5 (128
+// rows in 8) -> 23.5 (64 rows in 6), n5632 k2048 m128 25.7 -> 23.1; Q6_K k4096 n12288 m180
+// 65.6 (128 rows in 2) -> 49.9 (256 rows in 5), n28672 m256 115 -> 94 (256 in 2); Q4_K the
+// same 55.7 -> 47.7 and 92 -> 86.  Calls beyond the 32-bit x offsets (chunked) never split.
 struct PrefillPlan {
     int bm, S;
 };
-// the most 128-row tiles that split their k steps: half the CUs or fewer
-int64_t split_tiles_max() { return device_info().cu_count / 2; }
-// the most slices a k range splits into
-constexpr int64_t kMaxSlices = 16;
+// the most slices a k range splits into, and the fewest k steps a slice takes
+constexpr int64_t kMaxSlices = 16, kMinSteps = 4;
 size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
 // The workspace a plan takes: x as f16 rows | their scales | the split slabs
@@ -614,68 +673,74 @@ size_t plan_bytes(const QWeight& w, int64_t m, int S) {
     return up256((size_t)m * (size_t)w.k * 2) + up256((size_t)m * sizeof(float)) + slabs;
 }
 
-// The busiest CU's share of a plan: rounds x rows x k steps a workgroup, a 128-row
-// tile's rows counted at 8/7 of a 256-row tile's (770 against 889 TFLOP/s a kernel,
-// Q4_0 m512 and m2048 at k4096 n14336, unsplit)
-int64_t plan_cost(int64_t tiles, int64_t S, int bm, int64_t ksteps, int64_t cus) {
-    const int64_t rounds = (tiles * S + cus - 1) / cus;
-    return rounds * bm * ((ksteps + S - 1) / S) * (bm == 128 ? 8 : 7);
+// ns of a k step of 64, 128 and 256 rows (n28672 k4096, one workgroup a CU)
+int64_t step_ns(int qtype, int bm) {
+    const int i = bm == 64 ? 0 : bm == 128 ? 1 : 2;
+    static constexpr int64_t q4_0[3] = {880, 1100, 1500}, q8_0[3] = {1030, 1200, 1500},
+                             q4_k[3] = {1180, 1330, 1640}, q6_k[3] = {1550, 1720, 1860};
+    return qtype == UNILLM_QTYPE_Q4_0   ? q4_0[i]
+           : qtype == UNILLM_QTYPE_Q8_0 ? q8_0[i]
+           : qtype == UNILLM_QTYPE_Q4_K ? q4_k[i]
+                                        : q6_k[i];
 }
 
-// cap > 0: a caller's fixed workspace of cap bytes; a split plan that does not fit
-// falls back to a plan that does (at worst the 128-row tiles unsplit)
+// cap > 0: a caller's fixed workspace of cap bytes; a split plan that does not fit it is
+// not taken (at worst the tiles unsplit)
 PrefillPlan prefill_plan(const QWeight& w, int64_t m, size_t cap = 0) {
     const int64_t cus = device_info().cu_count;
-    const int64_t tiles_n = (w.n + PBN - 1) / PBN;
-    const int64_t t256 = (m + 255) / 256 * tiles_n;
-    const int64_t ksteps = (w.kb + 1) / 2;
-    const int64_t tiles = (m + 127) / 128 * tiles_n;
-    // a tile a CU or more: 128-row tiles where they take no more rounds, each half
-    // as long (k4096 n14336 m1100: 504 tiles against 280, two rounds each; Q4_0
-    // 233 -> 187-189 us a call, Q8_0 231-233 -> 205-207; a third round loses)
-    if (t256 >= cus)
-        return (tiles + cus - 1) / cus <= (t256 + cus - 1) / cus ? PrefillPlan{128, 1}
-                                                                 : PrefillPlan{256, 1};
-    int64_t S = 1;
-    if (tiles <= split_tiles_max() && m <= prefill_chunk_rows(w.k, 128))
-        S = std::max<int64_t>(1, std::min<int64_t>({kMaxSlices, cus / tiles, ksteps / 8}));
-    if (S > 1 && cap > 0 && plan_bytes(w, m, (int)S) > cap) S = 1;
-    if (ksteps >= 128 && 2 * t256 <= cus && m <= prefill_chunk_rows(w.k, 256)) {
-        const int64_t S2 = std::min<int64_t>({kMaxSlices, cus / t256, ksteps / 16});
-        const bool cheaper =
-            m > 256 && plan_cost(t256, S2, 256, ksteps, cus) <= plan_cost(tiles, S, 128, ksteps, cus);
-        if ((8 * t256 >= 3 * cus || cheaper) && (cap == 0 || plan_bytes(w, m, (int)S2) <= cap))
-            return {256, (int)S2};
+    const int64_t tiles_n = (w.n + PBN - 1) / PBN, ksteps = (w.kb + 1) / 2;
+    PrefillPlan best{128, 1};
+    int64_t least = INT64_MAX;
+    for (int bm : {64, 128, 256}) {
+        const int64_t tiles = (m + bm - 1) / bm * tiles_n;
+        for (int64_t S = 1; S <= kMaxSlices; ++S) {
+            if (S > 1 && (tiles * S > cus || ksteps < kMinSteps * S || m > prefill_chunk_rows(w.k, bm) ||
+                          (cap > 0 && plan_bytes(w, m, (int)S) > cap)))
+                break;
+            const int64_t rounds = (tiles * S + cus - 1) / cus;
+            int64_t ns = rounds * ((ksteps + S - 1) / S) * step_ns(w.qtype, bm);
+            if (S > 1) ns += 3000 + S * m * w.n * 8 / 4000;
+            if (ns < least) {
+                least = ns;
+                best = {bm, (int)S};
+            }
+        }
     }
-    // fewer 256-row tiles than CUs, but one round of them against two of 128-row
-    // tiles (k4096 n14336 m1024: 224 tiles against 448; Q4_0 166-171 -> 134 us a
-    // call, 20-25 % on every shape it picks)
-    if (m > 256 && plan_cost(t256, 1, 256, ksteps, cus) < plan_cost(tiles, S, 128, ksteps, cus))
-        return {256, 1};
-    return {128, (int)S};
+    return best;
 }
 
 }  // namespace
 
-// The call's own need (for a caller's fixed workspace of cap bytes, cap > 0, the
-// plan that fits it where one does), and a bound for every m' <= m (the slabs of 4
-// slices of the largest m' that can split), so that a reserve for m covers every
+// The call's own need (for a caller's fixed workspace of cap bytes, cap > 0, the plan
+// that fits it), and a bound for every m' <= m, so that a reserve for m covers every
 // shorter call.
 size_t prefill_call_bytes(const QWeight& w, int64_t m, size_t cap) {
     return plan_bytes(w, m, prefill_plan(w, m, cap).S);
 }
 
 size_t prefill_workspace_bytes(const QWeight& w, int64_t m) {
-    // slices x rows of any split: at most kMaxSlices m, and at most 128 CUs / (column
-    // tiles) with 128-row tiles (S <= CUs / tiles) or 256 CUs / (column tiles) with
-    // 256-row tiles (S <= CUs / tiles)
+    // slices x rows of any split: at most kMaxSlices m, and, as a split's tiles times its
+    // slices are at most the CUs, at most 256 CUs / (column tiles)
     const int64_t tiles_n = (w.n + PBN - 1) / PBN;
-    const int64_t sm = (w.kb + 1) / 2 < 16
-                           ? 0  // fewer than 2 x 8 k steps: never split
+    const int64_t sm = (w.kb + 1) / 2 < 2 * kMinSteps
+                           ? 0  // never split
                            : std::min<int64_t>(kMaxSlices * m,
                                                256 * device_info().cu_count / tiles_n);
     const size_t slabs = (size_t)sm * w.n * sizeof(float);
     return up256((size_t)m * (size_t)w.k * 2) + up256((size_t)m * sizeof(float)) + slabs;
+}
+
+// 49 .. 64 rows (Q8_0: 33 .. 64) of a deep or large weight run here rather than on the
+// batched decode, whose k slices of at most 1024 each add a tile's sums onto y: m64 k14336
+// n4096 Q4_0 32.9 -> 30.9 us a call, Q8_0 44.5 -> 35.2, Q4_K 44.6 -> 38.3, Q6_K 46.8 ->
+// 43.2; k4096 n28672 Q4_0 45.1 -> 42.9, Q8_0 59.2 -> 50.4, Q4_K 59.0 -> 54.8, but Q6_K 62.7
+// -> 67.8, n12288 Q4_0 23.9 -> 26.7 and n4096 15.8 -> 22.2.
+bool prefill_takes_batch(const QWeight& w, int64_t m) {
+    if (m > kDecodeMaxM || m <= (w.qtype == UNILLM_QTYPE_Q8_0 ? 32 : 48) || !mfma_supports(w))
+        return false;
+    const int64_t nk = w.n * w.k;
+    if (w.k > 8192) return nk >= (int64_t)40 << 20;
+    return nk >= (int64_t)96 << 20 && w.qtype != UNILLM_QTYPE_Q6_K && w.qtype != UNILLM_QTYPE_Q5_K;
 }
 
 hipError_t launch_prefill_mfma(const QWeight& w, const float* x, int64_t m, float* y,
@@ -696,14 +761,14 @@ hipError_t launch_prefill_mfma(const QWeight& w, const float* x, int64_t m, floa
         plan.S > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + xbytes +
                                               up256((size_t)m * sizeof(float)))
                    : nullptr;
-    const int add = epi == kEpiAdd;
     e = norm.gamma ? launch_norm_convert(x, m, w.k, norm, ws, y, 0, s, rs)
                    : launch_x_to_f16_rows(x, m, w.k, ws, rs, s);
     if (e != hipSuccess) return e;
     const uint16_t* xb = static_cast<const uint16_t*>(ws);
 #define UNILLM_PREFILL_LAUNCH(QTYPE)                                                          \
-    return plan.bm == 256 ? launch_bm<QTYPE, 256>(w, xb, rs, m, y, plan.S, part, s, add)     \
-                          : launch_bm<QTYPE, 128>(w, xb, rs, m, y, plan.S, part, s, add)
+    return plan.bm == 256   ? launch_bm<QTYPE, 256>(w, xb, rs, m, y, plan.S, part, s, epi)   \
+           : plan.bm == 128 ? launch_bm<QTYPE, 128>(w, xb, rs, m, y, plan.S, part, s, epi)   \
+                            : launch_bm<QTYPE, 64>(w, xb, rs, m, y, plan.S, part, s, epi)
     switch (w.qtype) {
         case UNILLM_QTYPE_Q4_0: UNILLM_PREFILL_LAUNCH(UNILLM_QTYPE_Q4_0);
         case UNILLM_QTYPE_Q8_0: UNILLM_PREFILL_LAUNCH(UNILLM_QTYPE_Q8_0);
