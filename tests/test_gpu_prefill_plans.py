@@ -90,7 +90,8 @@ def test_prefill_swiglu(qtype, m, I, k):
 @pytest.mark.parametrize("qtype,m,n,k,tiles", [
     (Q8_0, 33, 4096, 11008, True), (Q8_0, 32, 4096, 11008, False),
     (Q4_K, 49, 4096, 14336, True), (Q4_K, 48, 4096, 14336, False),
-    (Q6_K, 64, 3000, 14336, True), (Q4_0, 64, 2048, 8192, False)])
+    (Q6_K, 64, 3000, 14336, True), (Q4_0, 64, 2048, 8192, False),
+    (Q4_0, 64, 1024, 491520, False)])  # 60 MiB of x: slabs beside it would not fit the scratch
 def test_batch_on_the_prefill(qtype, m, n, k, tiles):
     print(f"batch on the prefill qtype={qtype} m={m} n={n} k={k}", flush=True)
     ql = _weight(qtype, n, k, 3)

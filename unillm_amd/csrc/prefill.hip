@@ -739,7 +739,8 @@ bool prefill_takes_batch(const QWeight& w, int64_t m) {
     if (m > kDecodeMaxM || m <= (w.qtype == UNILLM_QTYPE_Q8_0 ? 32 : 48) || !mfma_supports(w))
         return false;
     const int64_t nk = w.n * w.k;
-    if (w.k > 8192) return nk >= (int64_t)40 << 20;
+    // (to k 262144: x and the slabs, 16 MiB at 64 rows, then fit every scratch that x alone did)
+    if (w.k > 8192) return nk >= (int64_t)40 << 20 && w.k <= (int64_t)1 << 18;
     return nk >= (int64_t)96 << 20 && w.qtype != UNILLM_QTYPE_Q6_K && w.qtype != UNILLM_QTYPE_Q5_K;
 }
 
