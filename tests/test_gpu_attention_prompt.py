@@ -100,3 +100,18 @@ def test_prompt_non_finite(hd, what):
     fin = ref.isfinite()
     assert fin.any()
     assert ((out - ref)[fin].norm() / ref[fin].norm()).item() < TOL
+
+
+# every query of odd 32-query tiles non-finite: the tiles beside them in their workgroup
+# keep the bits they have without (each redone tile stays in its own part of LDS)
+@pytest.mark.parametrize("hd,m,H", [(64, 128, 4), (128, 128, 4), (64, 1024, 32), (128, 1024, 32)])
+def test_prompt_redone_tiles_leave_the_others(hd, m, H):
+    print(f"prompt redone tiles hd={hd} m={m} H={H}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + hd)
+    x = torch.randn(m, 3 * H * hd, device="cuda", generator=g)
+    clean = _run(x, H, H, hd, 0)
+    odd = torch.arange(m, device="cuda") // 32 % 2 == 1
+    x[odd, :H * hd] = float("nan")
+    out = _run(x, H, H, hd, 0)
+    assert out[odd].isnan().all()
+    assert torch.equal(out[~odd], clean[~odd])

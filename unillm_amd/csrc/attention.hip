@@ -1075,8 +1075,9 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
         if (bad | __shfl_xor(bad, 32, 64)) {
             // a non-finite query again in plain f32 over this split's keys, by the two
             // lanes that hold it.  Rolled loops over the rotated query in LDS, 8 outputs a
-            // pass: it takes no registers from the loop above.
-            float* qf = reinterpret_cast<float*>(lds) + qt * NB * 8 * 64 + lane;  // [16 b's 8][64]
+            // pass: it takes no registers from the loop above.  In the LDS of this tile's own
+            // odd-wave sums, which it has read; the other tiles' waves may still read theirs.
+            float* qf = reinterpret_cast<float*>(lds) + (qt * (D / 2 + 2)) * 64 + lane;  // [16 b's 8][64]
             const float* row = qkv + (int64_t)qi * (H + 2 * KVH) * D + (int64_t)h * D;
 #pragma unroll 1
             for (int i = 0; i < NB * 4; ++i) {
