@@ -18,7 +18,7 @@ Q4_K = 12
 Q5_0 = 6
 Q5_K = 13
 Q6_K = 14
-# dense projection weights (candle's dequantized f32 QMatMul): f32 rows on the device
+# dense projection weights (candle's dequantized f32 QMatMul): rows in their own type
 F32 = 0
 F16 = 1
 BF16 = 30
