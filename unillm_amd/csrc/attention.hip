@@ -913,8 +913,11 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
             if (live) {
 #pragma unroll
                 for (int e = 0; e < 16; ++e) s[e] = 0.0f, sl[e] = 0.0f;
-                // the next block's parts are read ahead of a block's MFMAs; two chains
-                // alternate, so no MFMA waits for the one before it
+                // the next block's parts are read ahead of a block's MFMAs.  The large product
+                // alone goes to s, one rounding a block: with the small ones dealt over both
+                // sums the two chains alternate without a wait (m2048 265 against 272 us a
+                // call), but short prompts' error rose above the f32 matrix cores' (m439, 32
+                // heads of 128: 2.43e-7 against 2.25e-7; now 2.04e-7)
                 u32x4 k[2][5];
                 auto read = [&](int b) {
 #pragma unroll
@@ -932,11 +935,11 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
                     __builtin_amdgcn_sched_barrier(0);
                     const u32x4(&kb)[5] = k[b % 2];
                     sl = mfma_bf16(kb[2], q[b], sl);
-                    s = mfma_bf16(kb[1], q[b], s);
                     sl = mfma_bf16(kb[0], kb[4], sl);
-                    s = mfma_bf16(kb[0], kb[3], s);
-                    sl = mfma_bf16(kb[1], kb[3], sl);
                     s = mfma_bf16(kb[0], q[b], s);
+                    sl = mfma_bf16(kb[1], kb[3], sl);
+                    sl = mfma_bf16(kb[1], q[b], sl);
+                    sl = mfma_bf16(kb[0], kb[3], sl);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -1048,7 +1051,7 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
             for (int t = 0; t < OT; ++t)
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
-                    o[t][e] = fmaf(o[t][e], f0, ox[(2 + 16 * t + e) * 64] * f1);
+                    o[t][e] = fmaf(ox[(2 + 16 * t + e) * 64], f1, o[t][e] * f0);
         }
         if (qi >= m) continue;
         // O[q][32 t + 8 u + 4 hf + 0..3] = o[t][4 u + 0..3] / l, a float4 each; or, split,
@@ -1061,13 +1064,18 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
         float* ml = S > 1 ? part + 2 * qc : nullptr;
         if (ml && hf == 0) *reinterpret_cast<float2*>(ml) = make_float2(mrun, lrun);
         const float inv = S > 1 ? 1.0f : 1.0f / lrun;
+        // o / l: the rounded product, corrected by its remainder
+        auto ratio = [&](float a) {
+            const float r = a * inv;
+            return S > 1 ? a : fmaf(fmaf(-r, lrun, a), inv, r);
+        };
         float chk = lrun * 0.0f;
 #pragma unroll
         for (int t = 0; t < OT; ++t)
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const float4 v = make_float4(o[t][4 * u] * inv, o[t][4 * u + 1] * inv,
-                                             o[t][4 * u + 2] * inv, o[t][4 * u + 3] * inv);
+                const float4 v = make_float4(ratio(o[t][4 * u]), ratio(o[t][4 * u + 1]),
+                                             ratio(o[t][4 * u + 2]), ratio(o[t][4 * u + 3]));
                 *reinterpret_cast<float4*>(orow + 32 * t + 8 * u) = v;
                 chk = fmaf(v.x, 0.0f, fmaf(v.y, 0.0f, fmaf(v.z, 0.0f, fmaf(v.w, 0.0f, chk))));
             }
@@ -1158,8 +1166,7 @@ __global__ __launch_bounds__(256) void attn_merge_split_kernel(const float* __re
         l = fmaf(p.y, f, l);
         o = make_float4(fmaf(v.x, f, o.x), fmaf(v.y, f, o.y), fmaf(v.z, f, o.z), fmaf(v.w, f, o.w));
     }
-    const float inv = 1.0f / l;
-    reinterpret_cast<float4*>(out)[i] = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+    reinterpret_cast<float4*>(out)[i] = make_float4(o.x / l, o.y / l, o.z / l, o.w / l);
 }
 
 // How a prompt call is dealt out: QT query tiles a block, blocks paired or not, S splits
