@@ -678,9 +678,9 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float* __restri
 // and the splits' VALU work beside them.  With the causal mask a block's work grows with
 // its position: taking blocks i and last - i one after the other gives every workgroup the
 // same (a form that paired a low and a high tile in two waves of one workgroup left one
-// wave a SIMD half the time).  Measured, kernel alone: m2048, 32 heads of 128: 239 us (144
-// TFLOP/s of f32 product; 391 on the f32 matrix cores, 270 in the paired form), m500 behind
-// 777, 32 heads of 64 over 4: 45 us and the merge's 4.6 (65.6 and 4.8).  At m2048 the matrix
+// wave a SIMD half the time).  Measured, kernel alone: m2048, 32 heads of 128: 222-250 us
+// (138-155 TFLOP/s of f32 product; 391 on the f32 matrix cores, 270 in the paired form), m500
+// behind 777, 32 heads of 64 over 4: 42 us and the merge's 4.5 (65.6 and 4.8).  At m2048 the matrix
 // cores are busy 41 % and the VALU 30 % of the cycles, and hardly at once.
 // A non-finite k or v makes 0 * inf terms in the split products: a query whose sum or
 // output comes out non-finite is recomputed in plain f32.
