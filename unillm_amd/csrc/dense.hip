@@ -32,6 +32,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "internal.hpp"
 #include "lds.hpp"
@@ -173,8 +174,12 @@ __device__ __forceinline__ bool non_finite(float v) {
 // for F32), U groups requested ahead of the ones being multiplied, so 128 bytes a lane
 // stay in flight across row ends.  x sits in LDS as two planes of 4 floats a group:
 // every read is 16 consecutive bytes a lane, free of bank conflicts.  Bound by the
-// weight stream: F16 k4096 n11008 (90 MB) 17.0 us a call (5.3 TB/s), against 228 us as
-// an f32 library GEMM of rows widened to f32.
+// weight stream at one token: F16 k4096 n11008 (90 MB) 16.3 us a call (5.5 TB/s), against 228
+// us as an f32 library GEMM of rows widened to f32.  From three tokens on, by x's reads from
+// LDS (32 bytes a token for 8 weights): two of the wave's rows are multiplied by each read,
+// with half the groups in flight for each.  F16 m4 29.4 -> 24.1 us, m8 45.4 -> 33.0; F32 m8
+// 53.6 -> 41.1 (a single last row runs alone: no products are made for rows past the end).
+// x is staged 16 bytes a lane where its rows allow it (m1 18.8 -> 18.1, called eagerly).
 constexpr int kGemvThreads = 1024;
 constexpr int64_t kGemvLds = 128 << 10;
 
@@ -211,66 +216,102 @@ __global__ __launch_bounds__(kGemvThreads, 1) void dense_gemv_kernel(
     f32x4* xs = reinterpret_cast<f32x4*>(smem);  // [M][2][G]
     const int G = (k + 7) / 8;
     const int lane = threadIdx.x & 63;
-    const int64_t wave = (int64_t)(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
+    const int64_t wave =
+        (int64_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
     const int64_t waves = (int64_t)(kGemvThreads / 64) * gridDim.x;
-    constexpr int U = QT == UNILLM_QTYPE_F32 ? 4 : M <= 4 ? 8 : 4;
+    constexpr int R = M >= 4 ? 2 : 1;  // rows at a time
+    constexpr int U = (QT == UNILLM_QTYPE_F32 ? 4 : M <= 4 ? 8 : 4) / R;
     const int T = (G + 64 * U - 1) / (64 * U);  // batches of U groups a lane in a row
 
-    auto request = [&](int64_t row, int t, Row8<QT>(&r)[U]) {
-        const uint8_t* p = base + row * row_bytes;
+    auto request = [&](int64_t row, int t, Row8<QT>(&r)[R][U]) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) r[u] = load8<QT>(p, min((t * U + u) * 64 + lane, G - 1));
+        for (int i = 0; i < R; ++i) {
+            if (row + i * waves >= n) break;
+            const uint8_t* p = base + (row + i * waves) * row_bytes;
+#pragma unroll
+            for (int u = 0; u < U; ++u) r[i][u] = load8<QT>(p, min((t * U + u) * 64 + lane, G - 1));
+        }
     };
     // the first batch is in flight while x is staged
-    Row8<QT> cur[U], nxt[U];
-    if (wave < n) request(wave, 0, cur);
-    float* xf = reinterpret_cast<float*>(smem);
-    for (int i = threadIdx.x; i < M * G * 8; i += kGemvThreads) {
-        const int t = i / (G * 8), c = i % (G * 8);
-        // plane (c / 4) % 2, group c / 8
-        xf[((t * 2 + (c / 4) % 2) * G + c / 8) * 4 + c % 4] =
-            t < m && c < k ? x[(int64_t)t * k + c] : 0.0f;
+    Row8<QT> cur[R][U] = {}, nxt[R][U] = {};
+    request(wave, 0, cur);
+    const bool vec = k % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+#pragma unroll
+    for (int t = 0; t < M; ++t) {
+        const float* xt = x + (int64_t)t * k;
+        for (int q = threadIdx.x; q < 2 * G; q += kGemvThreads) {
+            f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (t < m) {
+                if (vec) {
+                    if (4 * q < k) v = reinterpret_cast<const f32x4*>(xt)[q];
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (4 * q + e < k) v[e] = xt[4 * q + e];
+                }
+            }
+            xs[(t * 2 + q % 2) * G + q / 2] = v;
+        }
     }
     __syncthreads();
 
-    for (int64_t row = wave; row < n; row += waves) {
-        float acc[M];
+    float acc[R][M];
+    // batch b of the first `rows` rows
+    auto batch = [&](int b, auto rows) {
 #pragma unroll
-        for (int t = 0; t < M; ++t) acc[t] = 0.0f;
-        for (int b = 0; b < T; ++b) {
-            const bool last = b + 1 == T;
-            const int64_t nrow = last ? row + waves : row;
-            if (nrow < n) request(nrow, last ? 0 : b + 1, nxt);
+        for (int u = 0; u < U; ++u) {
+            const int g = (b * U + u) * 64 + lane;
+            if (g < G) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int g = (b * U + u) * 64 + lane;
-                if (g < G) {
+                for (int t = 0; t < M; ++t) {
+                    const f32x4 lo = xs[(t * 2) * G + g], hi = xs[(t * 2 + 1) * G + g];
 #pragma unroll
-                    for (int t = 0; t < M; ++t) {
-                        const f32x4 lo = xs[(t * 2) * G + g], hi = xs[(t * 2 + 1) * G + g];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[t] = fmaf(elem8<QT>(cur[u], e), lo[e], acc[t]);
+                    for (int i = 0; i < rows.value; ++i) {
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            acc[t] = fmaf(elem8<QT>(cur[u], 4 + e), hi[e], acc[t]);
+                            acc[i][t] = fmaf(elem8<QT>(cur[i][u], e), lo[e], acc[i][t]);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            acc[i][t] = fmaf(elem8<QT>(cur[i][u], 4 + e), hi[e], acc[i][t]);
                     }
                 }
             }
+        }
+    };
+    for (int64_t row0 = wave; row0 < n; row0 += R * waves) {
+        const bool whole = row0 + (R - 1) * waves < n;
 #pragma unroll
-            for (int u = 0; u < U; ++u) cur[u] = nxt[u];
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int t = 0; t < M; ++t) acc[i][t] = 0.0f;
+        for (int b = 0; b < T; ++b) {
+            const bool last = b + 1 == T;
+            request(last ? row0 + R * waves : row0, last ? 0 : b + 1, nxt);
+            if (whole) batch(b, std::integral_constant<int, R>{});
+            else batch(b, std::integral_constant<int, 1>{});
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+#pragma unroll
+                for (int u = 0; u < U; ++u) cur[i][u] = nxt[i][u];
         }
 #pragma unroll
-        for (int t = 0; t < M; ++t) {
-            float s = acc[t];
-            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-            if (lane == 0 && t < m) {
-                if constexpr (QT == UNILLM_QTYPE_F16) {
-                    const float f = wsc[row];
-                    s *= f;
-                    if (non_finite(s)) s = dense_dot<QT>(x + (int64_t)t * k, base + row * row_bytes, k, f);
+        for (int i = 0; i < R; ++i) {
+            const int64_t row = row0 + i * waves;
+            if (row >= n) break;
+#pragma unroll
+            for (int t = 0; t < M; ++t) {
+                float s = acc[i][t];
+                for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+                if (lane == 0 && t < m) {
+                    if constexpr (QT == UNILLM_QTYPE_F16) {
+                        const float f = wsc[row];
+                        s *= f;
+                        if (non_finite(s))
+                            s = dense_dot<QT>(x + (int64_t)t * k, base + row * row_bytes, k, f);
+                    }
+                    float* dst = y + (int64_t)t * n + row;
+                    *dst = add ? *dst + s : s;
                 }
-                float* dst = y + (int64_t)t * n + row;
-                *dst = add ? *dst + s : s;
             }
         }
     }
