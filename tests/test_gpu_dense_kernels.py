@@ -50,6 +50,20 @@ def test_dense_edges(dtype, m, n, k):
     assert torch.equal(ql.forward(buf[1:].view(m, k)), y)
 
 
+# the GEMV's row pairs (4096 waves on 256 CUs): one wave with a second row, all of them,
+# a single third row, one fewer; x rows that can and cannot be staged 16 bytes a lane
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(3, 4097, 264), (4, 8192, 511), (8, 8193, 130), (5, 12287, 64)])
+def test_dense_gemv_row_pairs(dtype, m, n, k):
+    print(f"dense row pairs {dtype} m={m} n={n} k={k}", flush=True)
+    w, x = _make(m, n, k, dtype, n)
+    ql = QuantLinear.from_dense(w)
+    y = ql.forward(x)
+    assert _err(y, x.double() @ w.double().t()) < TOL
+    for t in range(m):  # a token's bits do not depend on how many share the call
+        assert torch.equal(ql.forward(x[t:t + 1].contiguous())[0], y[t])
+
+
 # rows of very different size, and weights in the subnormal range of f16
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("m", [2, 40])
