@@ -254,7 +254,8 @@ int unillm_hip_kv_cache_truncate(unillm_kv_cache* c, int64_t len);
  * call past max_seq appends nothing, writes NaN and makes the next length query
  * or eager call fail with the overflow message; clear / truncate reset it.
  * Alignment: qkv_dev 16 bytes; out_dev 4 bytes on a decode step, 16 bytes on a
- * longer call (its kernels store 16 bytes at a time). */
+ * longer call (its kernels store 16 bytes at a time).  out_dev may share memory
+ * with qkv_dev. */
 int unillm_hip_attention_decode(unillm_kv_cache* c, const float* qkv_dev, int64_t m,
                                 int64_t n_heads, float* out_dev, void* stream);
 

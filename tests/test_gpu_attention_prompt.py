@@ -115,3 +115,43 @@ def test_prompt_redone_tiles_leave_the_others(hd, m, H):
     out = _run(x, H, H, hd, 0)
     assert out[odd].isnan().all()
     assert torch.equal(out[~odd], clean[~odd])
+
+
+# out over qkv (a caller that reuses the projection's buffer): the same bits as beside it;
+# unsplit plans, a split one, a decode step, hd 256; and inside a capture
+@pytest.mark.parametrize("hd,m,past,H,KVH", [(128, 300, 0, 32, 32), (64, 1000, 0, 32, 4),
+                                             (64, 40, 3000, 32, 4), (128, 1, 100, 8, 8),
+                                             (256, 40, 5, 4, 2)])
+def test_prompt_out_over_qkv(hd, m, past, H, KVH):
+    print(f"prompt out over qkv hd={hd} m={m} past={past} H={H} KVH={KVH}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m)
+    width = (H + 2 * KVH) * hd
+    x = torch.randn(past + m, width, device="cuda", generator=g)
+    want = _run(x, H, KVH, hd, past)
+    kv = KvCache(KVH, hd, past + m)
+    if past:
+        kv.attention(x[:past].contiguous(), H)
+    buf = torch.empty(2 * m * width, device="cuda")
+    qkv = buf[:m * width].view(m, width)
+    s = torch.cuda.Stream()
+    kv.reserve(m, H, stream=s)
+    for first in (0, 64, m * width - 64, m * width - m * H * hd):  # floats out lies behind qkv
+        out = buf[first:first + m * H * hd].view(m, H * hd)
+        qkv.copy_(x[past:])
+        assert torch.equal(kv.attention(qkv, H, out=out), want)
+        kv.truncate(past)
+    out = buf[:m * H * hd].view(m, H * hd)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s, capture_error_mode="thread_local"):
+        kv.attention(qkv, H, out=out, stream=s)
+    for i in range(3):
+        kv.truncate(past)
+        qkv.copy_(x[past:])
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            graph.replay()
+        s.synchronize()
+        # (a capture may split the keys otherwise)
+        assert ((out - want).norm() / want.norm()).item() < TOL
+    del graph

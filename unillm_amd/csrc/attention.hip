@@ -730,10 +730,10 @@ struct PromptLds {
 
 template <int D, int QT>
 __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
-    const float* __restrict__ qkv, int m, int H, int KVH, int* __restrict__ state, float scale,
-    const float* __restrict__ inv_freq, const float* __restrict__ kc,
-    const float* __restrict__ vc, int max_seq, int blocks, int paired, float* __restrict__ out,
-    float* __restrict__ part) {
+    const float* __restrict__ qrows, int64_t qstride, int m, int H, int KVH,
+    int* __restrict__ state, float scale, const float* __restrict__ inv_freq,
+    const float* __restrict__ kc, const float* __restrict__ vc, int max_seq, int blocks, int paired,
+    float* __restrict__ out, float* __restrict__ part) {
     using L = PromptLds<D, QT>;
     constexpr int OT = D / 32, NB = D / 16, NT = 128 * QT;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -854,7 +854,7 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
             uint8_t* qx = lds + (qt * NB * 64 + lane) * 16;  // part 0 of block b at b * 1024
             __syncthreads();  // the staging tiles are free (the block before is done)
             const int qr = min(qi, m - 1);
-            const float* row = qkv + (int64_t)qr * (H + 2 * KVH) * D + (int64_t)h * D;
+            const float* row = qrows + (int64_t)qr * qstride + (int64_t)h * D;
             typedef float f32x8 __attribute__((ext_vector_type(8)));
 #pragma unroll
             for (int bb = 0; bb < NB / 4; ++bb) {
@@ -1086,7 +1086,7 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
             // pass: it takes no registers from the loop above.  In the LDS of this tile's own
             // odd-wave sums, which it has read; the other tiles' waves may still read theirs.
             float* qf = reinterpret_cast<float*>(lds) + (qt * (D / 2 + 2)) * 64 + lane;  // [16 b's 8][64]
-            const float* row = qkv + (int64_t)qi * (H + 2 * KVH) * D + (int64_t)h * D;
+            const float* row = qrows + (int64_t)qi * qstride + (int64_t)h * D;
 #pragma unroll 1
             for (int i = 0; i < NB * 4; ++i) {
                 const int p = 16 * (i / 8) + 8 * hf + i % 8;
@@ -1175,8 +1175,17 @@ struct PromptPlan {
     int qt, paired, S;
 };
 
+// Whether an unsplit prompt call takes its queries from a copy: out shares memory with qkv.
+bool prompt_copies_q(const float* qkv, int64_t m, int64_t H, int64_t KVH, int64_t D, int S,
+                     const float* out) {
+    const uintptr_t q0 = reinterpret_cast<uintptr_t>(qkv), o0 = reinterpret_cast<uintptr_t>(out);
+    const uintptr_t q1 = q0 + (uintptr_t)(m * (H + 2 * KVH) * D) * sizeof(float),
+                    o1 = o0 + (uintptr_t)(m * H * D) * sizeof(float);
+    return S == 1 && q0 < o1 && o0 < q1;
+}
+
 template <int D, int QT>
-hipError_t launch_prompt_qt(const KvCache& kv, const float* qkv, int m, int H, float* part,
+hipError_t launch_prompt_qt(const KvCache& kv, const float* qkv, int m, int H, float* ws,
                             const PromptPlan& plan, float* out, hipStream_t s) {
     using L = PromptLds<D, QT>;
     static const bool attr = hipFuncSetAttribute((const void*)attn_prompt_kernel<D, QT>,
@@ -1189,25 +1198,37 @@ hipError_t launch_prompt_qt(const KvCache& kv, const float* qkv, int m, int H, f
         qkv, m, H, KVH, kv.state, scale, kv.inv_freq, kv.k, kv.v, (int)kv.max_seq, nullptr, H);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
+    // the attention kernel reads the queries while other workgroups store outputs: where out
+    // lies over qkv, from a copy (a split call stores no output before its merge)
+    const float* qrows = qkv;
+    int64_t qstride = (int64_t)(H + 2 * KVH) * D;
+    if (prompt_copies_q(qkv, m, H, KVH, D, plan.S, out)) {
+        const size_t width = (size_t)H * D * sizeof(float);
+        if ((e = hipMemcpy2DAsync(ws, width, qkv, (size_t)qstride * sizeof(float), width, (size_t)m,
+                                  hipMemcpyDeviceToDevice, s)) != hipSuccess)
+            return e;
+        qrows = ws;
+        qstride = (int64_t)H * D;
+    }
     const int blocks = (m + 32 * QT - 1) / (32 * QT);
     const int grid = plan.paired ? (blocks + 1) / 2 : blocks;
     attn_prompt_kernel<D, QT><<<dim3((unsigned)grid, (unsigned)H, (unsigned)plan.S), 128 * QT,
-                                L::BYTES, s>>>(qkv, m, H, KVH, kv.state, scale, kv.inv_freq, kv.k,
-                                               kv.v, (int)kv.max_seq, blocks, plan.paired, out,
-                                               part);
+                                L::BYTES, s>>>(qrows, qstride, m, H, KVH, kv.state, scale,
+                                               kv.inv_freq, kv.k, kv.v, (int)kv.max_seq, blocks,
+                                               plan.paired, out, ws);
     e = hipGetLastError();
     if (plan.S == 1 || e != hipSuccess) return e;
     const int64_t merge_threads = (int64_t)m * H * (D / 4);
     attn_merge_split_kernel<D><<<(unsigned)((merge_threads + 255) / 256), 256, 0, s>>>(
-        part, m, H, plan.S, out, kv.state, (int)kv.max_seq);
+        ws, m, H, plan.S, out, kv.state, (int)kv.max_seq);
     return hipGetLastError();
 }
 
 template <int D>
-hipError_t launch_prompt(const KvCache& kv, const float* qkv, int m, int H, float* part,
+hipError_t launch_prompt(const KvCache& kv, const float* qkv, int m, int H, float* ws,
                          const PromptPlan& plan, float* out, hipStream_t s) {
-    return plan.qt == 4 ? launch_prompt_qt<D, 4>(kv, qkv, m, H, part, plan, out, s)
-                        : launch_prompt_qt<D, 2>(kv, qkv, m, H, part, plan, out, s);
+    return plan.qt == 4 ? launch_prompt_qt<D, 4>(kv, qkv, m, H, ws, plan, out, s)
+                        : launch_prompt_qt<D, 2>(kv, qkv, m, H, ws, plan, out, s);
 }
 
 template <int D, int BQ, int BK>
@@ -1271,38 +1292,34 @@ PromptPlan prompt_plan(int64_t m, int64_t H, int64_t D, int64_t len) {
         }
     return best;
 }
-// hd 256's rotated queries [H][m][hd] (the matrix-core kernel rotates its own)
-size_t prompt_q_bytes(int64_t m, int64_t H, int64_t D) {
-    if (D == 64 || D == 128) return 0;
-    return ((size_t)m * H * D * sizeof(float) + 255) / 256 * 256;
-}
-}  // namespace
 
-namespace {
 // Workspace (slot 2) of one call of m tokens: the decode path's per-chunk partials at
-// any length (at most kMaxChunks chunks of (max, sum) and o[hd] per query), or the
-// prompt path's rotated queries [H][m][hd] followed, for a split call, by its S
-// partials per query.
-size_t attention_call_bytes(const KvCache& kv, int64_t m, int64_t H, int S) {
+// any length (at most kMaxChunks chunks of (max, sum) and o[hd] per query); at hd 256 the
+// prompt path's rotated queries [H][m][hd]; else a split prompt's S partials per query, or
+// the copied queries [m][H hd] of an unsplit one whose out lies over its qkv.
+size_t attention_call_bytes(const KvCache& kv, int64_t m, int64_t H, int S, bool copies_q) {
     const int64_t G = H / std::max<int64_t>(kv.n_kv_heads, 1), D = kv.head_dim;
     if (m * G <= kAttnMaxQ) return (size_t)m * H * kMaxChunks * (2 + D) * sizeof(float);
-    return prompt_q_bytes(m, H, D) + (S > 1 ? (size_t)m * H * S * (2 + D) * sizeof(float) : 0);
+    if (S > 1) return (size_t)m * H * S * (2 + D) * sizeof(float);
+    return D == 256 || copies_q ? (size_t)m * H * D * sizeof(float) : 0;
 }
 }  // namespace
 
 // Enough for every call of up to m tokens (what unillm_hip_attention_reserve grows to): the
 // longest decode step's partials, and a prompt's.  A split prompt's partial rows (S m H) are
 // at most kMaxPromptSplit m H, and, as its workgroups are at most kPromptRounds a CU and
-// hold at most two blocks of 128 queries each, at most 256 kPromptRounds CUs.
+// hold at most two blocks of 128 queries each, at most 256 kPromptRounds CUs; an unsplit
+// one's queries (rotated, or copied) are m H rows.
 size_t attention_workspace_bytes(const KvCache& kv, int64_t m, int64_t H) {
     const int64_t G = H / std::max<int64_t>(kv.n_kv_heads, 1), D = kv.head_dim;
     size_t need = 0;
     const int64_t md = std::min(m, kAttnMaxQ / G);
-    if (md >= 1) need = attention_call_bytes(kv, md, H, 1);
+    if (md >= 1) need = attention_call_bytes(kv, md, H, 1, false);
     if (m * G > kAttnMaxQ) {
         const int64_t rows = std::min<int64_t>(kMaxPromptSplit * m * H,
                                                256 * kPromptRounds * (int64_t)device_info().cu_count);
-        need = std::max(need, prompt_q_bytes(m, H, D) + (size_t)rows * (2 + D) * sizeof(float));
+        need = std::max({need, (size_t)rows * (2 + D) * sizeof(float),
+                         attention_call_bytes(kv, m, H, 1, true)});
     }
     return need;
 }
@@ -1315,16 +1332,13 @@ hipError_t launch_attention(const KvCache& kv, const float* qkv, int64_t m, int6
     if (m * (H / kv.n_kv_heads) > kAttnMaxQ) {
         // (captured: the length at a replay is not known; planned for an empty cache)
         const PromptPlan plan = prompt_plan(m, H, D, std::max<int64_t>(len_hint, 0));
-        if ((e = stream_workspace(s, std::max<size_t>(attention_call_bytes(kv, m, H, plan.S), 16),
-                                  &ws, 2)) != hipSuccess)
-            return e;
-        float* qw = static_cast<float*>(ws);
-        float* part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + prompt_q_bytes(m, H, D));
-        if (D == 64)
-            return launch_prompt<64>(kv, qkv, (int)m, (int)H, part, plan, out, s);
-        if (D == 128)
-            return launch_prompt<128>(kv, qkv, (int)m, (int)H, part, plan, out, s);
-        return launch_prefill_attn<256, 32, 32>(kv, qkv, (int)m, (int)H, qw, out, s);
+        const size_t need = attention_call_bytes(
+            kv, m, H, plan.S, prompt_copies_q(qkv, m, H, kv.n_kv_heads, D, plan.S, out));
+        if ((e = stream_workspace(s, std::max<size_t>(need, 16), &ws, 2)) != hipSuccess) return e;
+        float* f = static_cast<float*>(ws);
+        if (D == 64) return launch_prompt<64>(kv, qkv, (int)m, (int)H, f, plan, out, s);
+        if (D == 128) return launch_prompt<128>(kv, qkv, (int)m, (int)H, f, plan, out, s);
+        return launch_prefill_attn<256, 32, 32>(kv, qkv, (int)m, (int)H, f, out, s);
     }
     // decode: chunks sized for the known length, or for the longest the cache holds
     const int64_t L = len_hint >= 0 ? len_hint + m
