@@ -219,6 +219,19 @@ struct StreamWs {
 };
 std::mutex g_ws_mutex;
 std::map<std::pair<hipStream_t, int>, StreamWs> g_ws;
+// One lock per stream: a call of several launches hands data from one to the next through
+// the stream's workspaces, so threads that share a stream issue such calls one at a time.
+// (One for each, not one for all: a launch can block while its own stream's queue is full.)
+std::map<hipStream_t, std::mutex> g_stream_order;
+
+std::unique_lock<std::mutex> stream_order(hipStream_t s) {
+    std::mutex* order;
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        order = &g_stream_order[s];
+    }
+    return std::unique_lock<std::mutex>(*order);
+}
 // Buffers a workspace has outgrown.  A graph captured while one of them was
 // current still reads and writes it at every replay, so none is ever freed;
 // growth at least doubles a slot, so they add up to less than the slot itself.
@@ -470,6 +483,11 @@ int qmatmul_impl(const unillm_qweight* w, const float* x_dev, int64_t m, float* 
     if (int rc = ensure_init()) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e;
+    // (a single launch on the caller's own buffers needs no order)
+    std::unique_lock<std::mutex> order;
+    if (path != UNILLM_PATH_GEMV || !aligned16(x_dev) ||
+        (epi == kEpiSwiglu && !gemv_supports_swiglu(*w, m)))
+        order = stream_order(s);
     if (is_dense(w->qtype)) return dense_impl(w, x_dev, m, y_dev, path, s, epi, norm, what, fixed_ws);
     // x not on a 16-byte boundary (candle takes any contiguous f32): the kernels
     // load x 16 bytes at a time, so it is first copied, stream-ordered, into an
@@ -797,6 +815,7 @@ int unillm_hip_attention_decode(unillm_kv_cache* c, const float* qkv_dev, int64_
                     "attention: a prompt-length call (more than " +
                         std::to_string(attention_max_queries()) +
                         " queries a kv head) takes out 16-byte aligned");
+    const std::unique_lock<std::mutex> order = stream_order(s);
     if (capturing) {
         // the kernels read the length from the device at each replay: the grid covers
         // the longest the cache holds, and the host's copy is unknown afterwards

@@ -31,7 +31,6 @@
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
-#include <mutex>
 #include <type_traits>
 
 #include "internal.hpp"
@@ -775,15 +774,11 @@ hipError_t launch_gemm_bm(const QWeight& w, const float* x, int64_t m, float* y,
     return hipGetLastError();
 }
 
-std::mutex g_dense_mutex;
-
 template <int QT>
 hipError_t launch_dense_qt(const QWeight& w, const float* x, int64_t m, float* y, hipStream_t s,
                            int add) {
     if (dense_gemv_supports(w, m)) return launch_gemv_qt<QT>(w, x, m, y, s, add);
     const DensePlan p = dense_plan(w, m);
-    // a call's launches stay together: threads that share a stream share its workspace
-    std::lock_guard<std::mutex> lock(g_dense_mutex);
     void* ws = nullptr;
     const hipError_t e = stream_workspace(s, dense_bytes(w, m, p.S > 1 ? p.S * m : 0), &ws, kDenseSlot);
     if (e != hipSuccess) return e;

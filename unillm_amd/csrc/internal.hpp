@@ -163,7 +163,8 @@ const DeviceInfo& device_info();
 // later calls on the same stream (stream order makes the reuse safe: a call's
 // kernels finish before the next call's start).  Grows stream-ordered; the
 // memory is held until the process ends.  Calls on one stream from several
-// host threads are ordered by the stream, the map by a mutex.
+// host threads are issued one at a time (a lock per stream, held by the entry point through
+// its last launch), the map is guarded by a mutex.
 // Slot 0 holds x in the MFMA paths' operand type; slot 1 the [gate | up] outputs
 // of a SwiGLU call off the GEMV path (both live during that call); slot 2
 // attention's partials (and, for hd 256 prompts, the rotated queries); slot 3 an
