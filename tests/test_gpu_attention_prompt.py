@@ -155,3 +155,21 @@ def test_prompt_out_over_qkv(hd, m, past, H, KVH):
         # (a capture may split the keys otherwise)
         assert ((out - want).norm() / want.norm()).item() < TOL
     del graph
+
+
+# scores of -inf from position 128 on: a key split that holds no other key (m 40 behind 3000
+# takes eight) weighs nothing, and an unsplit call the same
+@pytest.mark.parametrize("hd,m,past,H,KVH", [(64, 40, 3000, 32, 4), (128, 40, 3000, 32, 4),
+                                             (128, 300, 0, 32, 32)])
+def test_prompt_keys_without_weight(hd, m, past, H, KVH):
+    print(f"prompt keys without weight hd={hd} m={m} past={past}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(hd + m)
+    x = torch.randn(past + m, (H + 2 * KVH) * hd, device="cuda", generator=g)
+    # the slowest rotation pair: its angle stays small, so a query of (1, 1) keeps both signs
+    q = x[:, :H * hd].view(-1, H, hd)
+    q[:, :, hd // 2 - 1] = q[:, :, hd - 1] = 1.0
+    x[128:, H * hd:(H + KVH) * hd].view(-1, KVH, hd)[:, :, hd // 2 - 1] = -math.inf
+    ref = _reference(x, H, KVH, hd, past)
+    assert ref.isfinite().all()
+    out = _run(x, H, KVH, hd, past)
+    assert ((out.double() - ref).norm() / ref.norm()).item() < TOL

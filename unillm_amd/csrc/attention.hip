@@ -1096,6 +1096,9 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
                 qf[i * 64] = (a * cs - c * sn) * scale;
                 qf[(i + NB * 4) * 64] = (a * sn + c * cs) * scale;
             }
+            // (a score of -inf has weight 0 also where no other is above it: a split without a
+            // live key)
+            auto weight = [&](float sc, float mx) { return sc == -INFINITY ? 0.0f : expf(sc - mx); };
             auto score = [&](int kk) {  // of key kk: both lanes return the whole dot
                 float sc = 0.0f;
 #pragma unroll 1
@@ -1108,7 +1111,7 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
 #pragma unroll 1
             for (int kk = k0; kk < k1; ++kk) mx = fmaxf(mx, score(kk));
 #pragma unroll 1
-            for (int kk = k0; kk < k1; ++kk) l += expf(score(kk) - mx);
+            for (int kk = k0; kk < k1; ++kk) l += weight(score(kk), mx);
             if (ml && hf == 0) *reinterpret_cast<float2*>(ml) = make_float2(mx * kLog2e, l);
             const float f = S > 1 ? 1.0f : 1.0f / l;
 #pragma unroll 1
@@ -1116,7 +1119,7 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
                 float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
                 for (int kk = k0; kk < k1; ++kk) {
-                    const float pe = expf(score(kk) - mx);
+                    const float pe = weight(score(kk), mx);
                     const float* vr = vg + (int64_t)kk * D + 16 * c + 4 * hf;
 #pragma unroll
                     for (int j = 0; j < 8; ++j) a[j] = fmaf(pe, vr[8 * (j / 4) + j % 4], a[j]);
