@@ -173,3 +173,55 @@ def test_prompt_keys_without_weight(hd, m, past, H, KVH):
     assert ref.isfinite().all()
     out = _run(x, H, KVH, hd, past)
     assert ((out.double() - ref).norm() / ref.norm()).item() < TOL
+
+
+# a NaN row in the middle of a tile, NaN and infinite values behind each other, and every row
+# non-finite, over plans that split and pair: exactly the outputs that see them, and soon: a
+# recompute costs a scan of the keys a query at most, dealt over the block's waves (m1500
+# all-inf v measured under 4 ms; the bar leaves room for a busy machine)
+@pytest.mark.parametrize("hd,m,past,H,KVH", [(64, 250, 0, 8, 4), (128, 250, 10, 8, 8),
+                                             (64, 45, 900, 32, 4), (128, 45, 900, 32, 4)])
+@pytest.mark.parametrize("what", ["row_nan", "v_nan_then_inf", "all_nan", "v_all_inf"])
+def test_prompt_redo(hd, m, past, H, KVH, what):
+    print(f"prompt redo hd={hd} m={m} past={past} {what}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(hd + m)
+    n = past + m
+    x = torch.randn(n, (H + 2 * KVH) * hd, device="cuda", generator=g)
+    v = x[:, (H + KVH) * hd:].view(n, KVH, hd)
+    if what == "row_nan":
+        x[past + 21] = math.nan
+    elif what == "v_nan_then_inf":
+        v[past + 3, 0, 5] = math.nan
+        v[past + 9, 1, 6] = math.inf
+        v[past + 30, 1, 6] = -math.inf
+        v[past + 40, 0, 7] = -math.inf
+    elif what == "all_nan":
+        x[past:] = math.nan
+    else:
+        v[past] = math.inf
+    ref = _reference(x, H, KVH, hd, past) if n <= 256 else None
+    if ref is None:  # each query's own keys: 0 * inf of a masked key is not part of it
+        ref = torch.stack([_reference(x[:past + t + 1], H, KVH, hd, past + t)[0]
+                           for t in range(m)])
+    ref = ref.float()
+    out = _run(x, H, KVH, hd, past)
+    assert torch.equal(out.isnan(), ref.isnan())
+    assert torch.equal(out[out.isinf()], ref[ref.isinf()])
+    fin = ref.isfinite()
+    if fin.any():
+        assert ((out - ref)[fin].norm() / ref[fin].norm()).item() < TOL
+
+
+def test_prompt_redo_cost():
+    H, hd, m = 32, 128, 1500
+    x = torch.randn(m, 3 * H * hd, device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    x[0, 2 * H * hd:] = math.inf  # every query of every head
+    kv = KvCache(H, hd, m)
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    kv.attention(x, H)
+    kv.clear()
+    a.record()
+    kv.attention(x, H)
+    b.record()
+    torch.cuda.synchronize()
+    assert a.elapsed_time(b) < 40.0

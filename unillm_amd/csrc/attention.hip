@@ -43,6 +43,7 @@
 // per-chunk results (chunks (hd + 2) floats per query, written and read once).
 #include <hip/hip_runtime.h>
 
+#include <limits.h>
 #include <math.h>
 
 #include <algorithm>
@@ -720,7 +721,7 @@ struct PromptLds {
     static constexpr int BYTES = Q1 + QT * (D / 16) * 2048;
     static constexpr int TASKS = 8 * D / (64 * NW);  // staging tasks a thread for two K (or V) tiles
     // a block's first query parts, and its odd waves' sums, pass through the staging tiles
-    static_assert(QT * (D / 16) * 1024 <= 4 * TILE && QT * (2 * D + 8) * 64 <= 4 * TILE, "");  // (a redone query too)
+    static_assert(QT * (D / 16) * 1024 <= 4 * TILE && QT * (2 * D + 8) * 64 <= 4 * TILE, "");  // (and its redone queries)
     // the slot of chunk c in key row r: 8 or 16 chunks a row
     __device__ static uint32_t kslot(uint32_t r, uint32_t c) {
         return D == 128 ? c ^ (r & 15) : c ^ ((r >> 1) & 7);
@@ -1027,19 +1028,21 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
         }
 
         // the tile's two waves: the odd key tiles' sums through LDS to the even ones'
-        {
-            float* ox = reinterpret_cast<float*>(lds) + (qt * (D / 2 + 2)) * 64 + lane;
-            __syncthreads();
-            if (kh == 1) {
-                ox[0] = mrun;
-                ox[64] = lrun;
+        int el = lane, eh = h;  // opaque: nothing below is computed ahead of the loops above
+        asm volatile("" : "+v"(el), "+s"(eh));
+        float* ox = reinterpret_cast<float*>(lds) + (qt * (D / 2 + 2)) * 64 + el;
+        uint32_t* redo = reinterpret_cast<uint32_t*>(lds + L::Q1);  // [QT] non-finite queries
+        __syncthreads();
+        if (kh == 1) {
+            ox[0] = mrun;
+            ox[64] = lrun;
 #pragma unroll
-                for (int t = 0; t < OT; ++t)
+            for (int t = 0; t < OT; ++t)
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) ox[(2 + 16 * t + e) * 64] = o[t][e];
-            }
-            __syncthreads();
-            if (kh == 1) continue;
+                for (int e = 0; e < 16; ++e) ox[(2 + 16 * t + e) * 64] = o[t][e];
+        }
+        __syncthreads();
+        if (kh == 0) {
             const float m1 = ox[0], l1 = ox[64];
             const float mm = fmaxf(mrun, m1);
             // (a wave without live keys left -inf: weight 0)
@@ -1047,86 +1050,182 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
             const float f1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - mm);
             lrun = lrun * f0 + l1 * f1;
             mrun = mm;
+            // O[q][32 t + 8 u + 4 hf + 0..3] = o[t][4 u + 0..3] / l, a float4 each; or, split,
+            // partials as attn_merge_split_kernel reads them: (max, sum) at [q H + h][S], o at
+            // [q H + h][S][hd] after all the pairs (a query with no live tile in this split
+            // leaves (-inf, 0) and zeros, weight 0 in the merge)
+            const float inv = S > 1 ? 1.0f : 1.0f / lrun;
+            // o / l: the rounded product, corrected by its remainder
+            auto ratio = [&](float a) {
+                const float r = a * inv;
+                return S > 1 ? a : fmaf(fmaf(-r, lrun, a), inv, r);
+            };
+            float chk = lrun * 0.0f;
 #pragma unroll
             for (int t = 0; t < OT; ++t)
 #pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    o[t][e] = fmaf(ox[(2 + 16 * t + e) * 64], f1, o[t][e] * f0);
-        }
-        if (qi >= m) continue;
-        // O[q][32 t + 8 u + 4 hf + 0..3] = o[t][4 u + 0..3] / l, a float4 each; or, split,
-        // partials as attn_merge_split_kernel reads them: (max, sum) at [q H + h][S], o at
-        // [q H + h][S][hd] after all the pairs (a query with no live tile in this split
-        // leaves (-inf, 0) and zeros, weight 0 in the merge)
-        const int64_t qc = ((int64_t)qi * H + h) * S + z;
-        float* orow = (S > 1 ? part + (int64_t)m * H * S * 2 + qc * D
-                             : out + (int64_t)qi * H * D + (int64_t)h * D) + 4 * hf;
-        float* ml = S > 1 ? part + 2 * qc : nullptr;
-        if (ml && hf == 0) *reinterpret_cast<float2*>(ml) = make_float2(mrun, lrun);
-        const float inv = S > 1 ? 1.0f : 1.0f / lrun;
-        // o / l: the rounded product, corrected by its remainder
-        auto ratio = [&](float a) {
-            const float r = a * inv;
-            return S > 1 ? a : fmaf(fmaf(-r, lrun, a), inv, r);
-        };
-        float chk = lrun * 0.0f;
-#pragma unroll
-        for (int t = 0; t < OT; ++t)
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const float4 v = make_float4(ratio(o[t][4 * u]), ratio(o[t][4 * u + 1]),
-                                             ratio(o[t][4 * u + 2]), ratio(o[t][4 * u + 3]));
-                *reinterpret_cast<float4*>(orow + 32 * t + 8 * u) = v;
-                chk = fmaf(v.x, 0.0f, fmaf(v.y, 0.0f, fmaf(v.z, 0.0f, fmaf(v.w, 0.0f, chk))));
-            }
-        const int bad = chk != 0.0f;  // (inf and NaN leave NaN)
-        if (bad | __shfl_xor(bad, 32, 64)) {
-            // a non-finite query again in plain f32 over this split's keys, by the two
-            // lanes that hold it.  Rolled loops over the rotated query in LDS, 8 outputs a
-            // pass: it takes no registers from the loop above.  In the LDS of this tile's own
-            // odd-wave sums, which it has read; the other tiles' waves may still read theirs.
-            float* qf = reinterpret_cast<float*>(lds) + (qt * (D / 2 + 2)) * 64 + lane;  // [16 b's 8][64]
-            const float* row = qrows + (int64_t)qi * qstride + (int64_t)h * D;
-#pragma unroll 1
-            for (int i = 0; i < NB * 4; ++i) {
-                const int p = 16 * (i / 8) + 8 * hf + i % 8;
-                float sn, cs;
-                sincosf((float)qpos * inv_freq[p], &sn, &cs);
-                const float a = row[p], c = row[p + D / 2];
-                qf[i * 64] = (a * cs - c * sn) * scale;
-                qf[(i + NB * 4) * 64] = (a * sn + c * cs) * scale;
-            }
-            // (a score of -inf has weight 0 also where no other is above it: a split without a
-            // live key)
-            auto weight = [&](float sc, float mx) { return sc == -INFINITY ? 0.0f : expf(sc - mx); };
-            auto score = [&](int kk) {  // of key kk: both lanes return the whole dot
-                float sc = 0.0f;
-#pragma unroll 1
-                for (int i = 0; i < NB * 8; ++i)
-                    sc = fmaf(qf[i * 64], kg[(int64_t)kk * D + 16 * (i / 8) + 8 * hf + i % 8], sc);
-                return sc + __shfl_xor(sc, 32, 64);
-            };
-            const int k0 = 64 * n0, k1 = min(64 * n1, qpos + 1);
-            float mx = -INFINITY, l = 0.0f;
-#pragma unroll 1
-            for (int kk = k0; kk < k1; ++kk) mx = fmaxf(mx, score(kk));
-#pragma unroll 1
-            for (int kk = k0; kk < k1; ++kk) l += weight(score(kk), mx);
-            if (ml && hf == 0) *reinterpret_cast<float2*>(ml) = make_float2(mx * kLog2e, l);
-            const float f = S > 1 ? 1.0f : 1.0f / l;
-#pragma unroll 1
-            for (int c = 0; c < D / 16; ++c) {  // outputs 16 c + 4 hf .. + 3 and + 8 ..
-                float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-                for (int kk = k0; kk < k1; ++kk) {
-                    const float pe = weight(score(kk), mx);
-                    const float* vr = vg + (int64_t)kk * D + 16 * c + 4 * hf;
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) a[j] = fmaf(pe, vr[8 * (j / 4) + j % 4], a[j]);
+                for (int e = 0; e < 16; ++e) {
+                    o[t][e] = ratio(fmaf(ox[(2 + 16 * t + e) * 64], f1, o[t][e] * f0));
+                    chk = fmaf(o[t][e], 0.0f, chk);
                 }
+            const int qi = 32 * mytile + el % 32;
+            bool bad = qi < m && chk != 0.0f;  // (inf and NaN leave NaN)
+            bad |= (bool)__shfl_xor((int)bad, 32, 64);
+            if (qi < m && !bad) {
+                const int64_t qc = ((int64_t)qi * H + eh) * S + z;
+                float* orow = (S > 1 ? part + (int64_t)m * H * S * 2 + qc * D
+                                     : out + (int64_t)qi * H * D + (int64_t)eh * D) + el / 32 * 4;
+                if (S > 1 && el < 32)
+                    *reinterpret_cast<float2*>(part + 2 * qc) = make_float2(mrun, lrun);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) orow[16 * c + 8 * (j / 4) + j % 4] = a[j] * f;
+                for (int t = 0; t < OT; ++t)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        *reinterpret_cast<float4*>(orow + 32 * t + 8 * u) = make_float4(
+                            o[t][4 * u], o[t][4 * u + 1], o[t][4 * u + 2], o[t][4 * u + 3]);
             }
+            const uint32_t mask = (uint32_t)__ballot(bad);  // (both halves of a query agree)
+            if (el == 0) redo[qt] = mask;
+        }
+        __syncthreads();
+        // A non-finite query again in plain f32 over this split's keys: the block's dealt over
+        // its waves, a whole wave each, 64 keys at a time: 8 lanes a key form its score, a lane
+        // a key its weight against the running max, then a lane D / 64 dimensions adds the
+        // weighted rows.  A row is NaN, and done, as soon as its query, its sum or all its
+        // outputs are, and without a look at the keys if it sees the NaN key that ended an
+        // earlier one.  m2048, 32 heads of 128, us a call (264 all finite): every row NaN 280,
+        // one NaN row in the middle of the prompt 770, an infinite v row at the start (every
+        // query redone in full) 5700.
+        int nan_key = INT_MAX;  // the first key known to hold a NaN
+        int tile = 0, turn = 0;
+        uint32_t left = __builtin_amdgcn_readfirstlane(redo[0]);
+        while (tile < QT) {
+            if (left == 0) {
+                if (++tile < QT) left = __builtin_amdgcn_readfirstlane(redo[tile]);
+                continue;
+            }
+            const int query = 32 * (t0 + tile) + __builtin_ctz(left);
+            left &= left - 1;
+            if (turn++ % L::NW != wv) continue;
+            float* qf = reinterpret_cast<float*>(lds) + wv * (D + 64);  // [D]
+            float* sc = qf + D;                                         // [64]
+            auto settle = [] {  // the wave's LDS stores before its reads after them
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            };
+            constexpr int DL = D / 64;  // dimensions a lane: DL el ..
+            typedef float dl_t __attribute__((ext_vector_type(DL)));
+            dl_t acc = 0.0f;
+            bool nan;
+            {
+                const float* row = qrows + (int64_t)query * qstride + (int64_t)eh * D;
+                const int p = el % (D / 2);
+                float sn, cs;
+                sincosf((float)(len + query) * inv_freq[p], &sn, &cs);
+                const float a = row[p], c = row[p + D / 2];
+                const float lo = (a * cs - c * sn) * scale, hi = (a * sn + c * cs) * scale;
+                nan = __any(lo != lo || hi != hi) || len + query >= nan_key;
+                settle();
+                qf[p] = lo;
+                qf[p + D / 2] = hi;
+                settle();
+            }
+            float mx = -INFINITY, l = 0.0f;
+            const int k0 = 64 * n0, k1 = min(64 * n1, len + query + 1);
+#pragma unroll 1
+            for (int kc0 = k0; kc0 < k1 && !nan; kc0 += 64) {
+                const float* qr = qf + el % 8 * (D / 8);
+#pragma unroll 1
+                for (int i0 = 0; i0 < 8; i0 += 4) {  // 32 keys, 4 a lane group
+                    float4 kr[4][D / 32];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int kk = min(kc0 + 8 * (i0 + i) + el / 8, k1 - 1);
+#pragma unroll
+                        for (int e = 0; e < D / 32; ++e)
+                            kr[i][e] = *reinterpret_cast<const float4*>(
+                                kg + (int64_t)kk * D + el % 8 * (D / 8) + 4 * e);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);  // (every load in flight before a use)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        float dot = 0.0f;
+#pragma unroll
+                        for (int e = 0; e < D / 32; ++e) {
+                            const float4 b = *reinterpret_cast<const float4*>(qr + 4 * e);
+                            dot = fmaf(kr[i][e].x, b.x, dot);
+                            dot = fmaf(kr[i][e].y, b.y, dot);
+                            dot = fmaf(kr[i][e].z, b.z, dot);
+                            dot = fmaf(kr[i][e].w, b.w, dot);
+                        }
+                        dot = group_sum<8>(dot);
+                        if (el % 8 == 0) sc[8 * (i0 + i) + el / 8] = dot;
+                    }
+                }
+                settle();
+                const float sv = kc0 + el < k1 ? sc[el] : -INFINITY;
+                const float mnew = fmaxf(mx, wave_max(sv));
+                const float alpha = mx == -INFINITY ? 0.0f : expf(mx - mnew);
+                // (a score of -inf has weight 0 also where no other is above it)
+                const float p = sv == -INFINITY ? 0.0f : expf(sv - mnew);
+                l = l * alpha + wave_add(p);
+                mx = mnew;
+                settle();
+                sc[el] = p;
+                settle();
+                const uint64_t pn = __ballot(p != p);
+                if (pn) {  // (the sum is NaN; a key with a NaN makes every later row's so)
+                    const int kk = kc0 + __builtin_ctzll(pn);
+                    const dl_t kv = *reinterpret_cast<const dl_t*>(kg + (int64_t)kk * D + DL * el);
+                    bool kn = false;
+#pragma unroll
+                    for (int i = 0; i < DL; ++i) kn |= kv[i] != kv[i];
+                    if (__any(kn)) nan_key = min(nan_key, kk);
+                    nan = true;
+                    break;
+                }
+                acc *= alpha;
+                const int nk = min(64, k1 - kc0);
+#pragma unroll 1
+                for (int j0 = 0; j0 < nk; j0 += 16) {
+                    dl_t vr[16];
+#pragma unroll
+                    for (int j = 0; j < 16; ++j)
+                        vr[j] = *reinterpret_cast<const dl_t*>(
+                            vg + (int64_t)(kc0 + min(j0 + j, nk - 1)) * D + DL * el);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int j = 0; j < 16; ++j)
+                        if (j0 + j < nk) {  // (a row past the last adds nothing, not 0 * inf)
+                            const float pj = sc[j0 + j];
+#pragma unroll
+                            for (int i = 0; i < DL; ++i) acc[i] = fmaf(pj, vr[j][i], acc[i]);
+                        }
+                }
+                settle();
+                bool all = true;
+#pragma unroll
+                for (int i = 0; i < DL; ++i) all &= acc[i] != acc[i];
+                nan = __any(l != l) || __all(all);
+            }
+            // split: the merge takes the max in units of log2 e, rounded as the matrix-core
+            // loop's are; the weights above are against the natural one
+            const float m2 = mx * kLog2e;
+            const float f = nan               ? __builtin_nanf("")
+                            : S == 1          ? 1.0f / l
+                            : mx == -INFINITY ? 1.0f
+                                              : __builtin_amdgcn_exp2f(fmaf(mx, kLog2e, -m2));
+            const int64_t qc = ((int64_t)query * H + eh) * S + z;
+            if (S > 1 && el == 0)
+                *reinterpret_cast<float2*>(part + 2 * qc) =
+                    nan ? make_float2(0.0f, f) : make_float2(m2, l * f);
+            float* orow = (S > 1 ? part + (int64_t)m * H * S * 2 + qc * D
+                                 : out + (int64_t)query * H * D + (int64_t)eh * D) +
+                          DL * el;
+            dl_t r = acc * f;
+            if (nan) r = f;
+            *reinterpret_cast<dl_t*>(orow) = r;
         }
     }
 }
