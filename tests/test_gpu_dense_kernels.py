@@ -98,3 +98,24 @@ def test_dense_non_finite(dtype, m, n, k):
     assert torch.equal(y[y.isinf()], ref[ref.isinf()])
     fin = ref.isfinite()
     assert ((y - ref)[fin].norm() / ref[fin].norm()).item() < TOL
+
+
+# sums of few terms, where a product's own rounding shows: within f32's bound, each FMA one
+# rounding (k 2^-24 of sum |x w|), and no worse than the f32 library product of the widened
+# weights (5 % for the draw)
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 8, 31, 32, 33, 64, 100])
+def test_dense_short_k(dtype, k):
+    m, n = 130, 300
+    w, x = _make(m, n, k, dtype, 77 + k)
+    if k == 1:  # a product whose parts cut off, not rounded, would lose the most
+        w[0], x[0] = 1 + 2 ** -7, 1 + 2 ** -7 - 2 ** -23
+        if dtype == torch.float32:
+            w[0] = 1 + 2 ** -7 - 2 ** -23
+    ql = QuantLinear.from_dense(w)
+    y, ref = ql.forward(x), x.double() @ w.double().t()
+    size = x.double().abs() @ w.double().abs().t()
+    assert ((y.double() - ref).abs() / size).max().item() <= k * 2 ** -24
+    assert _err(y, ref) <= 1.05 * _err(x @ w.float().t(), ref)
+    r = torch.randn_like(y)
+    assert _err(ql.forward_add(x, r.clone()), r.double() + ref) < TOL

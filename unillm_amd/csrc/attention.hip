@@ -656,8 +656,8 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float* __restri
 // second key tile (kh = w / QT), and the two waves of a tile merge their sums at the block's
 // end.  Both products keep f32's precision on the bf16 matrix cores: q, k, v and the
 // exponentials p are split exactly into three bf16 parts (split.hpp), and the six products
-// of parts that reach 2^-24 are summed in f32, the five small ones of q k in a sum of their
-// own.  The products are formed transposed so that no row reduction crosses more than two
+// of parts above 2^-24 of theirs are summed in f32, the five small ones of q k in a sum of
+// their own.  The products are formed transposed so that no row reduction crosses more than two
 // lanes and P never leaves the registers:
 //   S^T [32 keys][32 queries] = K . Q^T (v_mfma_f32_32x32x16_bf16: A lane l holds key
 //     l % 32, dimensions 8 (l / 32) .. + 7 of each 16; B the same of query l % 32, rotated
@@ -918,7 +918,8 @@ __global__ __launch_bounds__(128 * QT, QT == 4 ? 2 : 1) void attn_prompt_kernel(
                 // alone goes to s, one rounding a block: with the small ones dealt over both
                 // sums the two chains alternate without a wait (m2048 265 against 272 us a
                 // call), but short prompts' error rose above the f32 matrix cores' (m439, 32
-                // heads of 128: 2.43e-7 against 2.25e-7; now 2.04e-7)
+                // heads of 128: 2.43e-7 against 2.25e-7, with parts cut off; 1.62e-7 in a sum of
+                // their own with parts rounded)
                 u32x4 k[2][5];
                 auto read = [&](int b) {
 #pragma unroll

@@ -15,13 +15,16 @@
 //  - dense_gemm_kernel: 16-bit matrix cores at f32's precision.  x is split exactly
 //    into three 16-bit parts (xsplit_kernel), an F16 or BF16 weight is one part as it
 //    stands, an F32 weight is split in registers into three bf16 parts; the products
-//    of parts down to 2^-16 of the leading one are summed in f32 (3 per weight for F16
-//    and BF16, which is all of them; 6 for F32: the three left out are below 2^-24).
-//    gfx950's 16-bit matrix cores run 16 times its f32 ones, so 3 or 6 of them are
-//    still 5 or 2.7 times faster, and the error against f64 is below an f32 GEMM's,
-//    which rounds once a k (profiles/dense_weights.md has both).
+//    of parts are summed in f32, the leading one and the small ones each in a sum of their
+//    own (3 per weight for F16 and BF16, which is all of them; 6 for F32: the three left out
+//    are below 2^-24 of the product, split.hpp).  gfx950's 16-bit matrix cores run 16 times
+//    its f32 ones, so 3 or 6 of them are still 5 or 2.7 times faster, and the error against
+//    f64 is below an f32 GEMM's, which rounds once a k (profiles/dense_weights.md has both).
+//  - dense_short_kernel (k <= 4, m > 8): f32 FMAs.  So short a sum has few roundings in f32
+//    too, and the matrix cores' sums, which do not round to nearest, are the less exact ones
+//    (BF16, k 1 / 2 / 3, against f64: 3.3e-8 / 3.3e-8 / 3.2e-8, f32 2.6e-8 / 3.1e-8 / 3.6e-8).
 //
-// Both give the same bits on every call (no atomics; split-k slabs add in order), and
+// All give the same bits on every call (no atomics; split-k slabs add in order), and
 // an F16 or BF16 weight on the GEMV the same bits as its widened F32 copy.  A
 // non-finite x or weight makes 0 * inf terms in the split products, and scaled F16 rows
 // can overflow where the product does not: an output that comes out non-finite is
@@ -349,10 +352,39 @@ hipError_t launch_gemv_qt(const QWeight& w, const float* x, int64_t m, float* y,
     }
 }
 
+// ---- k <= 4, m > 8 -----------------------------------------------------------------------
+// A thread a column: its weights in registers, f32 FMAs over 64 rows of x.  Bound by the
+// store of y.
+constexpr int kShortK = 4;
+
+template <int QT>
+__global__ __launch_bounds__(256) void dense_short_kernel(const uint8_t* __restrict__ base,
+                                                          int64_t row_bytes,
+                                                          const float* __restrict__ wsc,
+                                                          const float* __restrict__ x, int64_t m,
+                                                          int64_t n, int k, float* __restrict__ y,
+                                                          int add) {
+    const int64_t col = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (col >= n) return;
+    float w[kShortK];  // (zeros past k: the row's padding)
+#pragma unroll
+    for (int i = 0; i < kShortK; ++i)
+        w[i] = widen1<QT>(base + col * row_bytes, i, row_factor<QT>(wsc, col));
+    for (int64_t row0 = (int64_t)blockIdx.y * 64; row0 < m; row0 += (int64_t)gridDim.y * 64)
+        for (int64_t row = row0; row < min(row0 + 64, m); ++row) {
+            float s = 0.0f;
+#pragma unroll
+            for (int i = 0; i < kShortK; ++i)
+                if (i < k) s = fmaf(x[row * k + i], w[i], s);
+            float* dst = y + row * n + col;
+            *dst = add ? *dst + s : s;
+        }
+}
+
 // ---- x in three 16-bit parts -------------------------------------------------------------
 // xp[p][m][kp]: x = part 0 + part 1 + part 2 exactly (rows padded with zeros to kp).
-// bf16 parts (BF16 and F32 weights): each part the upper 16 bits of what is left (8
-// significant bits each, 24 in all; truncation never overflows).  f16 parts (F16
+// bf16 parts (BF16 and F32 weights): each part what is left rounded to bf16 (split.hpp; a
+// finite value keeps a finite part 0).  f16 parts (F16
 // weights): the row is first scaled by the power of two that puts its largest magnitude
 // in [2^14, 2^15), undone on the output by rs[row]; each part is what is left rounded to
 // f16 (11 bits each, so the parts hold 2^-40 of the row's largest value).  A non-finite
@@ -401,15 +433,12 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x
             }
         } else {
             const uint32_t u = __float_as_uint(v);
-            p0 = (uint16_t)(u >> 16);
+            p0 = (uint16_t)pack_bf16(v, 0.0f);
             if (finite) {
-                const float r1 = v - __uint_as_float(u & 0xFFFF0000u);
-                const uint32_t u1 = __float_as_uint(r1);
-                const float r2 = r1 - __uint_as_float(u1 & 0xFFFF0000u);
-                p1 = (uint16_t)(u1 >> 16);
-                p2 = (uint16_t)(__float_as_uint(r2) >> 16);
-            } else if (u & 0x007FFFFFu) {
-                p0 |= 0x40;  // a NaN whose upper mantissa bits are zero stays a NaN
+                if ((p0 & 0x7F80u) == 0x7F80u) p0 = (uint16_t)(u >> 16);  // (rounded to infinity)
+                const float r1 = v - bf16_lo(p0);
+                p1 = (uint16_t)pack_bf16(r1, 0.0f);
+                p2 = (uint16_t)pack_bf16(r1 - bf16_lo(p1), 0.0f);
             }
         }
         o[i] = p0;
@@ -560,7 +589,7 @@ __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(
 #pragma unroll
         for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    f32x4 low[D::F32W ? TI : 1][D::F32W ? TJ : 1] = {};
+    f32x4 low[TI][TJ] = {};  // the small products' sums
 
     // prologue: three stages in flight; step 0's first fragments read
     constexpr int AHEAD = D::STAGES - 1;
@@ -603,33 +632,29 @@ __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(
             else if (j + 1 < nks)
                 read_first(j + 1, nf);
             __builtin_amdgcn_sched_barrier(0);  // (left free, the reads sink behind the MFMAs)
-            if constexpr (D::F32W) {
-                // the small products in sums of their own: one rounding of the large sum a
-                // 32 k, as with F16 and BF16 (in one sum, 1.3e-7 against 0.8e-7 for an f32
-                // GEMM at k 64)
+            // the small products in sums of their own: one rounding of the large sum a 32 k (F32
+            // in one sum, k 64: 1.3e-7 against 0.8e-7)
+            auto wpart = [&](int q, int p) { return D::F32W ? wb[q][p] : f.b[q][0]; };
 #pragma unroll
-                for (int q = 0; q < TJ; ++q) {
-                    low[i][q] = mfma_parts<false>(a[i % 2][2], wb[q][0], low[i][q]);
-                    acc[i][q] = mfma_parts<false>(a[i % 2][0], wb[q][0], acc[i][q]);
-                }
+            for (int q = 0; q < TJ; ++q) {
+                low[i][q] = mfma_parts<F16P>(a[i % 2][2], wpart(q, 0), low[i][q]);
+                acc[i][q] = mfma_parts<F16P>(a[i % 2][0], wpart(q, 0), acc[i][q]);
+            }
+            if constexpr (D::F32W) {
 #pragma unroll
                 for (int q = 0; q < TJ; ++q)
                     low[i][q] = mfma_parts<false>(a[i % 2][0], wb[q][2], low[i][q]);
 #pragma unroll
                 for (int q = 0; q < TJ; ++q)
                     low[i][q] = mfma_parts<false>(a[i % 2][1], wb[q][1], low[i][q]);
+            }
 #pragma unroll
-                for (int q = 0; q < TJ; ++q)
-                    low[i][q] = mfma_parts<false>(a[i % 2][1], wb[q][0], low[i][q]);
+            for (int q = 0; q < TJ; ++q)
+                low[i][q] = mfma_parts<F16P>(a[i % 2][1], wpart(q, 0), low[i][q]);
+            if constexpr (D::F32W) {
 #pragma unroll
                 for (int q = 0; q < TJ; ++q)
                     low[i][q] = mfma_parts<false>(a[i % 2][0], wb[q][1], low[i][q]);
-            } else {
-#pragma unroll
-                for (int p = NP - 1; p >= 0; --p)
-#pragma unroll
-                    for (int q = 0; q < TJ; ++q)
-                        acc[i][q] = mfma_parts<F16P>(a[i % 2][p], f.b[q][0], acc[i][q]);
             }
             if constexpr (i + 1 < TI)
                 asm volatile("s_waitcnt lgkmcnt(0)"
@@ -644,12 +669,10 @@ __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(
         step(j + 1, f1, f0);
     }
 
-    if constexpr (D::F32W) {
 #pragma unroll
-        for (int i = 0; i < TI; ++i)
+    for (int i = 0; i < TI; ++i)
 #pragma unroll
-            for (int q = 0; q < TJ; ++q) acc[i][q] += low[i][q];
-    }
+        for (int q = 0; q < TJ; ++q) acc[i][q] += low[i][q];
     // epilogue: lane holds rows 4 g + e, column fr of each 16 x 16 tile
 #pragma unroll
     for (int q = 0; q < TJ; ++q) {
@@ -778,6 +801,13 @@ template <int QT>
 hipError_t launch_dense_qt(const QWeight& w, const float* x, int64_t m, float* y, hipStream_t s,
                            int add) {
     if (dense_gemv_supports(w, m)) return launch_gemv_qt<QT>(w, x, m, y, s, add);
+    if (w.k <= kShortK) {
+        const dim3 grid((unsigned)((w.n + 255) / 256),
+                        (unsigned)std::min<int64_t>((m + 63) / 64, 65535));
+        dense_short_kernel<QT><<<grid, 256, 0, s>>>(w.base, w.row_bytes, dense_wsc(w), x, m, w.n,
+                                                    (int)w.k, y, add);
+        return hipGetLastError();
+    }
     const DensePlan p = dense_plan(w, m);
     void* ws = nullptr;
     const hipError_t e = stream_workspace(s, dense_bytes(w, m, p.S > 1 ? p.S * m : 0), &ws, kDenseSlot);
