@@ -119,3 +119,18 @@ def test_dense_short_k(dtype, k):
     assert _err(y, ref) <= 1.05 * _err(x @ w.float().t(), ref)
     r = torch.randn_like(y)
     assert _err(ql.forward_add(x, r.clone()), r.double() + ref) < TOL
+
+
+# an x far larger than the rest of its row, in a column of zero weights: the rest keeps f32's
+# precision on every path (GEMV, GEMM, split k)
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(8, 300, 512), (40, 300, 512), (40, 300, 4096), (200, 64, 512)])
+@pytest.mark.parametrize("outlier", [1e6, 1e9, 1e13, 1e30])
+def test_dense_outlier_behind_zero_weights(dtype, m, n, k, outlier):
+    w, x = _make(m, n, k, dtype, 21)
+    w[:, 9] = 0
+    x[:, 9] = outlier
+    x[::2, 20] = -outlier
+    w[:, 20] = 0
+    ql = QuantLinear.from_dense(w)
+    assert _err(ql.forward(x), x.double() @ w.double().t()) < TOL

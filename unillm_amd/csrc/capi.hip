@@ -151,9 +151,7 @@ int alloc_weight(int qtype, int64_t n, int64_t k, QWeight** out) {
     w->kb = is_dense(qtype) ? 0 : k / QK;
     w->row_bytes = is_dense(qtype) ? dense_row_bytes(qtype, k) : row_bytes_for(w->qtype, w->kb);
     // + a 256-byte tail slot for the scale reduction run at create
-    const size_t held = (size_t)n * (size_t)w->row_bytes +
-                        (is_dense(qtype) ? dense_extra_bytes(qtype, n) : 0);
-    w->bytes = ((held + 255) & ~(size_t)255) + 256;
+    w->bytes = (((size_t)n * (size_t)w->row_bytes + 255) & ~(size_t)255) + 256;
     void* mem = nullptr;
     hipError_t e = hipMalloc(&mem, w->bytes);
     if (e != hipSuccess) {

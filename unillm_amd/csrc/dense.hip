@@ -6,31 +6,31 @@
 // QMatMul whatever its GGML type (crates/runtime/src/weight_loader_core.rs:554-571),
 // so a GGUF with F16 projections takes this variant.  A weight is held in its own type
 // (a widening to f32 would double the bytes a decode step streams) as rows of
-// row_bytes, k padded with zeros to a multiple of 64 (an F16 row times the power of two
-// that puts its largest magnitude in [2^14, 2^15): exact, and undone on the output by the
-// factors behind the rows), and the product is f32:
+// row_bytes, k padded with zeros to a multiple of 64, and the product is f32:
 //
 //  - dense_gemv_kernel (m <= 8 where x fits in LDS): the weights widen in registers
 //    and every product is an f32 FMA.  Bound by the weight stream.
-//  - dense_gemm_kernel: 16-bit matrix cores at f32's precision.  x is split exactly
-//    into three 16-bit parts (xsplit_kernel), an F16 or BF16 weight is one part as it
-//    stands, an F32 weight is split in registers into three bf16 parts; the products
-//    of parts are summed in f32, the leading one and the small ones each in a sum of their
-//    own (3 per weight for F16 and BF16, which is all of them; 6 for F32: the three left out
-//    are below 2^-24 of the product, split.hpp).  gfx950's 16-bit matrix cores run 16 times
-//    its f32 ones, so 3 or 6 of them are still 5 or 2.7 times faster, and the error against
-//    f64 is below an f32 GEMM's, which rounds once a k (profiles/dense_weights.md has both).
+//  - dense_gemm_kernel: bf16 matrix cores at f32's precision.  x is split exactly into
+//    three bf16 parts (xsplit_kernel); a BF16 weight is one part as it stands, an F16 weight
+//    is split in registers into two, an F32 weight into three.  The products of parts are
+//    summed in f32, the leading one and the small ones each in a sum of their own: 3 a
+//    weight for BF16 (all of them), 5 for F16 and 6 for F32 (the ones left out come to
+//    0.5 and 0.9 times 2^-24 of the product at most, either sign).  gfx950's 16-bit matrix
+//    cores run 16 times its f32 ones, so up to 6 of them are still 2.7 times faster, and the
+//    error against f64 is below an f32 GEMM's, which rounds once a k
+//    (profiles/dense_weights.md has both).  bf16 has f32's range: a row of x keeps all its
+//    bits however far apart its values are.  (f16 parts, three products for F16, hold no
+//    element below 2^-40 of its row's largest: behind an outlier of 1e9 in a column of zero
+//    weights the product was off by 5.6e-4.)
 //  - dense_short_kernel (k <= 4, m > 8): f32 FMAs.  So short a sum has few roundings in f32
 //    too, and the matrix cores' sums, which do not round to nearest, are the less exact ones
 //    (BF16, k 1 / 2 / 3, against f64: 3.3e-8 / 3.3e-8 / 3.2e-8, f32 2.6e-8 / 3.1e-8 / 3.6e-8).
 //
 // All give the same bits on every call (no atomics; split-k slabs add in order), and
 // an F16 or BF16 weight on the GEMV the same bits as its widened F32 copy.  A
-// non-finite x or weight makes 0 * inf terms in the split products, and scaled F16 rows
-// can overflow where the product does not: an output that comes out non-finite is
-// recomputed as a plain f32 dot (dense_dot), so infinities propagate as f32 products
-// would.
-#include <hip/hip_bf16.h>
+// non-finite x or weight makes 0 * inf terms in the split products: an output that comes out
+// non-finite is recomputed as a plain f32 dot (dense_dot), so infinities propagate as f32
+// products would.
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
@@ -45,19 +45,12 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kKPad = 64;  // rows are padded with zeros to a multiple of this many weights
 
 int64_t padded_k(int64_t k) { return (k + kKPad - 1) / kKPad * kKPad; }
-
-// an F16 weight's row factors, behind its rows
-float* dense_wsc(const QWeight& w) {
-    return w.qtype == UNILLM_QTYPE_F16
-               ? reinterpret_cast<float*>(w.base + (size_t)w.n * (size_t)w.row_bytes)
-               : nullptr;
-}
 
 // ---- upload, dequant, layer norm ---------------------------------------------------------
 
@@ -72,59 +65,25 @@ __global__ __launch_bounds__(256) void dense_upload_kernel(const T* __restrict__
     for (int64_t i = threadIdx.x; i < k; i += 256) dr[i] = sr[i];
 }
 
-// the same for F16, each row scaled (wsc[row] <- the undoing factor); a workgroup a row
-__global__ __launch_bounds__(256) void dense_upload_f16_kernel(const uint16_t* __restrict__ src,
-                                                               uint8_t* __restrict__ dst,
-                                                               int64_t k, int64_t row_bytes,
-                                                               float* __restrict__ wsc) {
-    __shared__ uint32_t red[4];
-    const uint16_t* sr = src + (int64_t)blockIdx.x * k;
-    uint16_t* dr = reinterpret_cast<uint16_t*>(dst + (int64_t)blockIdx.x * row_bytes);
-    uint32_t mx = 0;  // largest finite magnitude (its bits order like the value)
-    for (int64_t i = threadIdx.x; i < k; i += 256) {
-        const uint32_t a = sr[i] & 0x7FFFu;
-        if (a < 0x7C00u) mx = max(mx, a);
-    }
-    for (int d = 32; d > 0; d >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, d));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    mx = max(max(red[0], red[1]), max(red[2], red[3]));
-    int e = 15;
-    if (mx) (void)frexpf(__half2float(__ushort_as_half((uint16_t)mx)), &e);
-    const int sh = max(15 - e, 0);  // never down: nothing is rounded
-    const float up = ldexpf(1.0f, sh);
-    for (int64_t i = threadIdx.x; i < k; i += 256)
-        dr[i] = __half_as_ushort(__float2half(__half2float(__ushort_as_half(sr[i])) * up));
-    if (threadIdx.x == 0) wsc[blockIdx.x] = ldexpf(1.0f, -sh);
-}
-
-// weight i of a row (F16: scaled back by its row's factor)
+// weight i of a row
 template <int QT>
-__device__ __forceinline__ float widen1(const uint8_t* row, int64_t i, float wsc) {
+__device__ __forceinline__ float widen1(const uint8_t* row, int64_t i) {
     if constexpr (QT == UNILLM_QTYPE_F32) return reinterpret_cast<const float*>(row)[i];
     const uint16_t v = reinterpret_cast<const uint16_t*>(row)[i];
-    if constexpr (QT == UNILLM_QTYPE_F16) return __half2float(__ushort_as_half(v)) * wsc;
+    if constexpr (QT == UNILLM_QTYPE_F16) return __half2float(__ushort_as_half(v));
     return __uint_as_float((uint32_t)v << 16);
-}
-
-// the factor of a row (F16), 1 otherwise
-template <int QT>
-__device__ __forceinline__ float row_factor(const float* wsc, int64_t row) {
-    if constexpr (QT == UNILLM_QTYPE_F16) return wsc[row];
-    return 1.0f;
 }
 
 // out[n, k] f32 <- the weight's values, widened exactly
 template <int QT>
 __global__ __launch_bounds__(256) void dense_widen_kernel(const uint8_t* __restrict__ base,
                                                           int64_t row_bytes,
-                                                          const float* __restrict__ wsc,
                                                           float* __restrict__ out, int64_t n,
                                                           int64_t k) {
     const int64_t count = n * k;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
          i += (int64_t)gridDim.x * blockDim.x)
-        out[i] = widen1<QT>(base + i / k * row_bytes, i % k, row_factor<QT>(wsc, i / k));
+        out[i] = widen1<QT>(base + i / k * row_bytes, i % k);
 }
 
 // out[r] = (x[r] - mean) / sqrt(var + eps) * gamma (+ beta), one workgroup a row: the
@@ -160,9 +119,9 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict_
 // The plain f32 dot of one output: what an output that came out non-finite is
 // recomputed with.
 template <int QT>
-__device__ __noinline__ float dense_dot(const float* x, const uint8_t* row, int64_t k, float wsc) {
+__device__ __noinline__ float dense_dot(const float* x, const uint8_t* row, int64_t k) {
     float s = 0.0f;
-    for (int64_t i = 0; i < k; ++i) s = fmaf(x[i], widen1<QT>(row, i, wsc), s);
+    for (int64_t i = 0; i < k; ++i) s = fmaf(x[i], widen1<QT>(row, i), s);
     return s;
 }
 
@@ -212,8 +171,8 @@ __device__ __forceinline__ float elem8(const Row8<QT>& r, int e) {
 // M: the token count the code is built for (m <= M; x past m is zero and not stored)
 template <int QT, int M>
 __global__ __launch_bounds__(kGemvThreads, 1) void dense_gemv_kernel(
-    const uint8_t* __restrict__ base, int64_t row_bytes, const float* __restrict__ wsc,
-    const float* __restrict__ x, int m, int64_t n, int k, float* __restrict__ y, int add) {
+    const uint8_t* __restrict__ base, int64_t row_bytes, const float* __restrict__ x, int m,
+    int64_t n, int k, float* __restrict__ y, int add) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     f32x4* xs = reinterpret_cast<f32x4*>(smem);  // [M][2][G]
     const int G = (k + 7) / 8;
@@ -305,12 +264,6 @@ __global__ __launch_bounds__(kGemvThreads, 1) void dense_gemv_kernel(
                 float s = acc[i][t];
                 for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
                 if (lane == 0 && t < m) {
-                    if constexpr (QT == UNILLM_QTYPE_F16) {
-                        const float f = wsc[row];
-                        s *= f;
-                        if (non_finite(s))
-                            s = dense_dot<QT>(x + (int64_t)t * k, base + row * row_bytes, k, f);
-                    }
                     float* dst = y + (int64_t)t * n + row;
                     *dst = add ? *dst + s : s;
                 }
@@ -337,7 +290,7 @@ hipError_t launch_gemv_m(const QWeight& w, const float* x, int64_t m, float* y, 
     // wave numbers run across workgroups, so few rows still spread over the CUs
     const int blocks = (int)std::min<int64_t>(device_info().cu_count, w.n);
     dense_gemv_kernel<QT, M><<<blocks, kGemvThreads, gemv_lds(m, w.k), s>>>(
-        w.base, w.row_bytes, dense_wsc(w), x, (int)m, w.n, (int)w.k, y, add);
+        w.base, w.row_bytes, x, (int)m, w.n, (int)w.k, y, add);
     return hipGetLastError();
 }
 
@@ -360,7 +313,6 @@ constexpr int kShortK = 4;
 template <int QT>
 __global__ __launch_bounds__(256) void dense_short_kernel(const uint8_t* __restrict__ base,
                                                           int64_t row_bytes,
-                                                          const float* __restrict__ wsc,
                                                           const float* __restrict__ x, int64_t m,
                                                           int64_t n, int k, float* __restrict__ y,
                                                           int add) {
@@ -369,7 +321,7 @@ __global__ __launch_bounds__(256) void dense_short_kernel(const uint8_t* __restr
     float w[kShortK];  // (zeros past k: the row's padding)
 #pragma unroll
     for (int i = 0; i < kShortK; ++i)
-        w[i] = widen1<QT>(base + col * row_bytes, i, row_factor<QT>(wsc, col));
+        w[i] = widen1<QT>(base + col * row_bytes, i);
     for (int64_t row0 = (int64_t)blockIdx.y * 64; row0 < m; row0 += (int64_t)gridDim.y * 64)
         for (int64_t row = row0; row < min(row0 + 64, m); ++row) {
             float s = 0.0f;
@@ -381,65 +333,25 @@ __global__ __launch_bounds__(256) void dense_short_kernel(const uint8_t* __restr
         }
 }
 
-// ---- x in three 16-bit parts -------------------------------------------------------------
-// xp[p][m][kp]: x = part 0 + part 1 + part 2 exactly (rows padded with zeros to kp).
-// bf16 parts (BF16 and F32 weights): each part what is left rounded to bf16 (split.hpp; a
-// finite value keeps a finite part 0).  f16 parts (F16
-// weights): the row is first scaled by the power of two that puts its largest magnitude
-// in [2^14, 2^15), undone on the output by rs[row]; each part is what is left rounded to
-// f16 (11 bits each, so the parts hold 2^-40 of the row's largest value).  A non-finite
-// value keeps its kind in part 0, the others zero.  One workgroup a row; bound by its
-// bytes (4 in, 6 out an element).
-template <bool F16P>
+// ---- x in three bf16 parts ---------------------------------------------------------------
+// xp[p][m][kp]: x = part 0 + part 1 + part 2 exactly (rows padded with zeros to kp), each
+// part what is left rounded to bf16 (split.hpp; a finite value keeps a finite part 0).  A
+// non-finite value keeps its kind in part 0, the others zero.  One workgroup a row; bound by
+// its bytes (4 in, 6 out an element).
 __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x, int64_t k,
                                                      int64_t kp, uint16_t* __restrict__ xp,
-                                                     int64_t plane, float* __restrict__ rs) {
+                                                     int64_t plane) {
     const float* xr = x + (int64_t)blockIdx.x * k;
     uint16_t* o = xp + (int64_t)blockIdx.x * kp;
-    const int tid = threadIdx.x;
-    float up = 1.0f;
-    if constexpr (F16P) {
-        __shared__ uint32_t red[4];
-        uint32_t mx = 0;  // largest finite magnitude (its bits order like the value)
-        for (int64_t i = tid; i < k; i += 256) {
-            const uint32_t a = __float_as_uint(xr[i]) & 0x7FFFFFFFu;
-            if (a < 0x7F800000u) mx = max(mx, a);
-        }
-        for (int d = 32; d > 0; d >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, d));
-        if ((tid & 63) == 0) red[tid >> 6] = mx;
-        __syncthreads();
-        mx = max(max(red[0], red[1]), max(red[2], red[3]));
-        int e = 0;
-        if (mx) (void)frexpf(__uint_as_float(mx), &e);
-        // |x| < 2^e; the factors stay normal f32 (a row below 2^-111 keeps fewer bits)
-        const int sh = min(max(15 - e, -113), 126);
-        up = ldexpf(1.0f, sh);
-        if (tid == 0) rs[blockIdx.x] = ldexpf(1.0f, -sh);
-    }
-    for (int64_t i = tid; i < kp; i += 256) {
+    for (int64_t i = threadIdx.x; i < kp; i += 256) {
         const float v = i < k ? xr[i] : 0.0f;
-        uint16_t p0, p1 = 0, p2 = 0;
-        const bool finite = (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u;
-        if constexpr (F16P) {
-            const float s = v * up;
-            const _Float16 h0 = (_Float16)s;
-            p0 = __builtin_bit_cast(uint16_t, h0);
-            if (finite) {
-                const float r1 = s - (float)h0;
-                const _Float16 h1 = (_Float16)r1;
-                const float r2 = r1 - (float)h1;
-                p1 = __builtin_bit_cast(uint16_t, h1);
-                p2 = __builtin_bit_cast(uint16_t, (_Float16)r2);
-            }
-        } else {
-            const uint32_t u = __float_as_uint(v);
-            p0 = (uint16_t)pack_bf16(v, 0.0f);
-            if (finite) {
-                if ((p0 & 0x7F80u) == 0x7F80u) p0 = (uint16_t)(u >> 16);  // (rounded to infinity)
-                const float r1 = v - bf16_lo(p0);
-                p1 = (uint16_t)pack_bf16(r1, 0.0f);
-                p2 = (uint16_t)pack_bf16(r1 - bf16_lo(p1), 0.0f);
-            }
+        const uint32_t u = __float_as_uint(v);
+        uint16_t p0 = (uint16_t)pack_bf16(v, 0.0f), p1 = 0, p2 = 0;
+        if (!non_finite(v)) {
+            if ((p0 & 0x7F80u) == 0x7F80u) p0 = (uint16_t)(u >> 16);  // (rounded to infinity)
+            const float r1 = v - bf16_lo(p0);
+            p1 = (uint16_t)pack_bf16(r1, 0.0f);
+            p2 = (uint16_t)pack_bf16(r1 - bf16_lo(p1), 0.0f);
         }
         o[i] = p0;
         o[plane + i] = p1;
@@ -455,9 +367,10 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x
 //   A  [3 parts][BM rows][64 B], the 16-byte chunk c of row r in slot c ^ f(r / 4 % 4),
 //      f = 0 3 2 1: the 16 lanes that an LDS read serves together touch all banks once;
 //   B  [BN rows][64 B], the same (F32: [BN][128 B], chunk c in slot c ^ r % 8).
-// Bound by the matrix cores at three products a weight (BF16 m512 k4096 n11008: 158 us a
-// call, 293 TFLOP/s of f32 product, against 451 us as an f32 library GEMM; 172 tiles on 256
-// CUs) and by the weight stream and the split's fixed cost at few rows (m16: 35 us).
+// Bound by the matrix cores (BF16 at three products a weight, m512 k4096 n11008: 159 us a
+// call, 290 TFLOP/s of f32 product, against 451 us as an f32 library GEMM; 172 tiles on 256
+// CUs.  F16 at five and the split of its weights: 251) and by the weight stream and the
+// split's fixed cost at few rows (m16: 37 us, F16 47).
 template <int QT, int BM>
 struct DTile {
     static constexpr bool F32W = QT == UNILLM_QTYPE_F32;
@@ -476,37 +389,44 @@ struct DTile {
 
 __device__ __forceinline__ uint32_t swz64(uint32_t row) { return (4u - ((row >> 2) & 3u)) & 3u; }
 
-template <bool F16P>
 __device__ __forceinline__ f32x4 mfma_parts(u32x4 a, u32x4 b, f32x4 c) {
-    if constexpr (F16P)
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                      __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                       __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// 8 f32 weights -> three bf16 parts (an infinity's or a NaN's lower parts come out NaN:
-// the output is recomputed)
-__device__ __forceinline__ void split8(const u32x4 (&w)[2], u32x4 (&p)[3]) {
+// A fragment's 8 weights -> their bf16 parts: three of an F32, two of an F16 (8 of its 11
+// bits, the rest), itself of a BF16 (an infinity's or a NaN's lower parts come out NaN: the
+// output is recomputed)
+template <int QT>
+__device__ __forceinline__ void split_weights(const u32x4 (&w)[QT == UNILLM_QTYPE_F32 ? 2 : 1],
+                                              u32x4 (&p)[3]) {
+    if constexpr (QT == UNILLM_QTYPE_BF16) p[0] = w[0];
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
-        uint32_t p0, p1, p2;
-        split2(w[h / 2][2 * (h % 2)], w[h / 2][2 * (h % 2) + 1], p0, p1, p2);
-        p[0][h] = p0;
-        p[1][h] = p1;
-        p[2][h] = p2;
+        if constexpr (QT == UNILLM_QTYPE_F32) {
+            uint32_t p0, p1, p2;
+            split2(w[h / 2][2 * (h % 2)], w[h / 2][2 * (h % 2) + 1], p0, p1, p2);
+            p[0][h] = p0;
+            p[1][h] = p1;
+            p[2][h] = p2;
+        } else if constexpr (QT == UNILLM_QTYPE_F16) {
+            const uint32_t u = w[0][h];  // (a bit cast of the element itself takes element 0)
+            const f16x2 v = __builtin_bit_cast(f16x2, u);
+            const float a = (float)v[0], b = (float)v[1];
+            const uint32_t p0 = pack_bf16(a, b);
+            p[0][h] = p0;
+            p[1][h] = pack_bf16(a - bf16_lo(p0), b - bf16_hi(p0));
+        }
     }
 }
 
 template <int QT, int BM>
 __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(
-    const uint8_t* __restrict__ base, int64_t row_bytes, const float* __restrict__ wsc,
-    const uint16_t* __restrict__ xp, int64_t plane, int64_t kp, const float* __restrict__ rs, const float* __restrict__ x,
-    int64_t k, float* __restrict__ y, int64_t M, int64_t N, int tiles_n, int tiles, int units_pad,
-    int S, int add, float* __restrict__ part) {
+    const uint8_t* __restrict__ base, int64_t row_bytes, const uint16_t* __restrict__ xp,
+    int64_t plane, int64_t kp, const float* __restrict__ x, int64_t k, float* __restrict__ y,
+    int64_t M, int64_t N, int tiles_n, int tiles, int units_pad, int S, int add,
+    float* __restrict__ part) {
     using D = DTile<QT, BM>;
-    constexpr bool F16P = QT == UNILLM_QTYPE_F16;
     constexpr int TI = D::TI, TJ = D::TJ, NP = D::NP;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
@@ -611,10 +531,8 @@ __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(
         if (j + AHEAD < nks) issue(j + AHEAD);
         const uint32_t st = (uint32_t)((j % D::STAGES) * D::STAGE);
         u32x4 wb[TJ][NP];
-        if constexpr (D::F32W) {
 #pragma unroll
-            for (int q = 0; q < TJ; ++q) split8(f.b[q], wb[q]);
-        }
+        for (int q = 0; q < TJ; ++q) split_weights<QT>(f.b[q], wb[q]);
         u32x4 a[2][NP];
 #pragma unroll
         for (int p = 0; p < NP; ++p) a[0][p] = f.a[p];
@@ -634,28 +552,20 @@ __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(
             __builtin_amdgcn_sched_barrier(0);  // (left free, the reads sink behind the MFMAs)
             // the small products in sums of their own: one rounding of the large sum a 32 k (F32
             // in one sum, k 64: 1.3e-7 against 0.8e-7)
-            auto wpart = [&](int q, int p) { return D::F32W ? wb[q][p] : f.b[q][0]; };
+            auto small = [&](int pa, int pb) {
+#pragma unroll
+                for (int q = 0; q < TJ; ++q)
+                    low[i][q] = mfma_parts(a[i % 2][pa], wb[q][pb], low[i][q]);
+            };
 #pragma unroll
             for (int q = 0; q < TJ; ++q) {
-                low[i][q] = mfma_parts<F16P>(a[i % 2][2], wpart(q, 0), low[i][q]);
-                acc[i][q] = mfma_parts<F16P>(a[i % 2][0], wpart(q, 0), acc[i][q]);
+                low[i][q] = mfma_parts(a[i % 2][2], wb[q][0], low[i][q]);
+                acc[i][q] = mfma_parts(a[i % 2][0], wb[q][0], acc[i][q]);
             }
-            if constexpr (D::F32W) {
-#pragma unroll
-                for (int q = 0; q < TJ; ++q)
-                    low[i][q] = mfma_parts<false>(a[i % 2][0], wb[q][2], low[i][q]);
-#pragma unroll
-                for (int q = 0; q < TJ; ++q)
-                    low[i][q] = mfma_parts<false>(a[i % 2][1], wb[q][1], low[i][q]);
-            }
-#pragma unroll
-            for (int q = 0; q < TJ; ++q)
-                low[i][q] = mfma_parts<F16P>(a[i % 2][1], wpart(q, 0), low[i][q]);
-            if constexpr (D::F32W) {
-#pragma unroll
-                for (int q = 0; q < TJ; ++q)
-                    low[i][q] = mfma_parts<false>(a[i % 2][0], wb[q][1], low[i][q]);
-            }
+            if constexpr (D::F32W) small(0, 2);
+            if constexpr (QT != UNILLM_QTYPE_BF16) small(1, 1);
+            small(1, 0);
+            if constexpr (QT != UNILLM_QTYPE_BF16) small(0, 1);
             if constexpr (i + 1 < TI)
                 asm volatile("s_waitcnt lgkmcnt(0)"
                              : "+v"(a[(i + 1) % 2][0]), "+v"(a[(i + 1) % 2][1]),
@@ -678,7 +588,6 @@ __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(
     for (int q = 0; q < TJ; ++q) {
         const int64_t col = n0 + (D::BN / 4) * cw + 16 * q + fr;
         if (col >= N) continue;
-        const float wf = row_factor<QT>(wsc, col);
 #pragma unroll
         for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -690,22 +599,19 @@ __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(
                     continue;
                 }
                 float v = acc[i][q][e];
-                if constexpr (F16P) v = v * wf * rs[row];
-                if (non_finite(v)) v = dense_dot<QT>(x + row * k, base + col * row_bytes, k, wf);
+                if (non_finite(v)) v = dense_dot<QT>(x + row * k, base + col * row_bytes, k);
                 float* dst = y + row * N + col;
                 *dst = add ? *dst + v : v;
             }
     }
 }
 
-// y (+)= the S slabs of a split k in slice order (scaled back for F16)
+// y (+)= the S slabs of a split k in slice order
 template <int QT>
 __global__ __launch_bounds__(256) void dense_sum_kernel(const float* __restrict__ part, int S,
                                                         int64_t M, int64_t N,
-                                                        const float* __restrict__ rs,
                                                         const uint8_t* __restrict__ base,
                                                         int64_t row_bytes,
-                                                        const float* __restrict__ wsc,
                                                         const float* __restrict__ x, int64_t k,
                                                         int add, float* __restrict__ y) {
     const int64_t MN = M * N;
@@ -714,19 +620,17 @@ __global__ __launch_bounds__(256) void dense_sum_kernel(const float* __restrict_
         const int64_t row = i / N, col = i % N;
         float v = part[i];
         for (int sl = 1; sl < S; ++sl) v += part[sl * MN + i];
-        const float wf = row_factor<QT>(wsc, col);
-        if constexpr (QT == UNILLM_QTYPE_F16) v = v * wf * rs[row];
-        if (non_finite(v)) v = dense_dot<QT>(x + row * k, base + col * row_bytes, k, wf);
+        if (non_finite(v)) v = dense_dot<QT>(x + row * k, base + col * row_bytes, k);
         y[i] = add ? y[i] + v : v;
     }
 }
 
 // Tile height and k split: the cheapest of 64- and 128-row tiles with k in up to 16
 // slices (at least 4 pairs of steps each, at most two workgroups a CU), by what a
-// workgroup's pair of steps was measured to take (64 / 128 rows: 1.5 / 2.35 us, F32 1.75
-// / 2.65) times the rounds over the CUs, plus a split's slabs written and read once
-// (3.5 TB/s) and the summing launch.  Measured against every choice, BF16 us a call:
-// k4096 n11008 m300 157.9 (128 rows, 129 tiles on 256 CUs) -> 107.0 (64 rows, 215),
+// workgroup's pair of steps was measured to take (64 / 128 rows: BF16 1.5 / 2.35 us, F16
+// 2.4 / 3.75, F32 1.75 / 2.65) times the rounds over the CUs, plus a split's slabs written
+// and read once (3.5 TB/s) and the summing launch.  Measured against every choice, BF16 us a
+// call: k4096 n11008 m300 157.9 (128 rows, 129 tiles on 256 CUs) -> 107.0 (64 rows, 215),
 // m512 158.7 (128, one slice; 64: 199.8); k4096 n2048 m128 36.2 -> 29.1 (64 rows in 12).
 struct DensePlan {
     int bm, S;
@@ -739,11 +643,12 @@ int64_t dense_bn(const QWeight& w) { return w.qtype == UNILLM_QTYPE_F32 ? 128 : 
 DensePlan dense_plan(const QWeight& w, int64_t m) {
     const int64_t cus = device_info().cu_count, kpairs = padded_k(w.k) / kKPad;
     const int64_t tiles_n = (w.n + dense_bn(w) - 1) / dense_bn(w);
-    const bool f32 = w.qtype == UNILLM_QTYPE_F32;
     DensePlan best{128, 1};
     int64_t least = INT64_MAX;
     for (int bm : {64, 128}) {
-        const int64_t pair_ns = bm == 64 ? (f32 ? 1750 : 1500) : (f32 ? 2650 : 2350);
+        const int64_t pair_ns = w.qtype == UNILLM_QTYPE_F32   ? (bm == 64 ? 1750 : 2650)
+                                : w.qtype == UNILLM_QTYPE_F16 ? (bm == 64 ? 2400 : 3750)
+                                                              : (bm == 64 ? 1500 : 2350);
         const int64_t tiles = (m + bm - 1) / bm * tiles_n;
         for (int64_t S = 1; S <= kDenseMaxSlices; ++S) {
             if (S > 1 && (S > kpairs / 4 || tiles * S > kDenseMaxRounds * cus)) break;
@@ -761,10 +666,9 @@ DensePlan dense_plan(const QWeight& w, int64_t m) {
 
 size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
-// x parts | row factors | slabs
+// x parts | slabs
 size_t dense_bytes(const QWeight& w, int64_t m, int64_t slab_rows) {
-    return up256((size_t)3 * m * padded_k(w.k) * 2) + up256((size_t)m * 4) +
-           (size_t)slab_rows * w.n * 4;
+    return up256((size_t)3 * m * padded_k(w.k) * 2) + (size_t)slab_rows * w.n * 4;
 }
 
 template <int QT, int BM>
@@ -777,9 +681,8 @@ hipError_t launch_gemm_bm(const QWeight& w, const float* x, int64_t m, float* y,
     if (!attr) return hipErrorInvalidValue;
     const int64_t kp = padded_k(w.k), plane = m * kp;
     uint16_t* xp = static_cast<uint16_t*>(ws);
-    float* rs = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + up256((size_t)3 * plane * 2));
-    float* part = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(rs) + up256((size_t)m * 4));
-    xsplit_kernel<QT == UNILLM_QTYPE_F16><<<(unsigned)m, 256, 0, s>>>(x, w.k, kp, xp, plane, rs);
+    float* part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + up256((size_t)3 * plane * 2));
+    xsplit_kernel<<<(unsigned)m, 256, 0, s>>>(x, w.k, kp, xp, plane);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const int64_t tiles_n = (w.n + D::BN - 1) / D::BN;
@@ -787,13 +690,13 @@ hipError_t launch_gemm_bm(const QWeight& w, const float* x, int64_t m, float* y,
     if (tiles * S > (int64_t)INT32_MAX - 8) return hipErrorInvalidValue;
     const int units_pad = (int)((tiles * S + 7) / 8 * 8);
     dense_gemm_kernel<QT, BM><<<units_pad, 512, D::BYTES, s>>>(
-        w.base, w.row_bytes, dense_wsc(w), xp, plane, kp, rs, x, w.k, y, m, w.n, (int)tiles_n, (int)tiles,
-        units_pad, S, add, part);
+        w.base, w.row_bytes, xp, plane, kp, x, w.k, y, m, w.n, (int)tiles_n, (int)tiles, units_pad,
+        S, add, part);
     if ((e = hipGetLastError()) != hipSuccess || S == 1) return e;
     const int blocks =
         (int)std::min<int64_t>((m * w.n + 255) / 256, 8 * (int64_t)device_info().cu_count);
-    dense_sum_kernel<QT><<<blocks, 256, 0, s>>>(part, S, m, w.n, rs, w.base, w.row_bytes,
-                                                dense_wsc(w), x, w.k, add, y);
+    dense_sum_kernel<QT><<<blocks, 256, 0, s>>>(part, S, m, w.n, w.base, w.row_bytes, x, w.k, add,
+                                                y);
     return hipGetLastError();
 }
 
@@ -804,8 +707,8 @@ hipError_t launch_dense_qt(const QWeight& w, const float* x, int64_t m, float* y
     if (w.k <= kShortK) {
         const dim3 grid((unsigned)((w.n + 255) / 256),
                         (unsigned)std::min<int64_t>((m + 63) / 64, 65535));
-        dense_short_kernel<QT><<<grid, 256, 0, s>>>(w.base, w.row_bytes, dense_wsc(w), x, m, w.n,
-                                                    (int)w.k, y, add);
+        dense_short_kernel<QT><<<grid, 256, 0, s>>>(w.base, w.row_bytes, x, m, w.n, (int)w.k, y,
+                                                    add);
         return hipGetLastError();
     }
     const DensePlan p = dense_plan(w, m);
@@ -824,18 +727,9 @@ bool is_dense(int qtype) {
 
 int dense_elem_bytes(int qtype) { return qtype == UNILLM_QTYPE_F32 ? 4 : 2; }
 
-size_t dense_extra_bytes(int qtype, int64_t n) {
-    return qtype == UNILLM_QTYPE_F16 ? (size_t)n * sizeof(float) : 0;
-}
-
 int64_t dense_row_bytes(int qtype, int64_t k) { return padded_k(k) * dense_elem_bytes(qtype); }
 
 hipError_t launch_dense_upload(const QWeight& w, const void* src, hipStream_t s) {
-    if (w.qtype == UNILLM_QTYPE_F16) {
-        dense_upload_f16_kernel<<<(unsigned)w.n, 256, 0, s>>>(static_cast<const uint16_t*>(src),
-                                                              w.base, w.k, w.row_bytes, dense_wsc(w));
-        return hipGetLastError();
-    }
     if (w.k % kKPad == 0)
         return hipMemcpyAsync(w.base, src, (size_t)w.n * (size_t)w.row_bytes,
                               hipMemcpyDeviceToDevice, s);
@@ -853,15 +747,15 @@ hipError_t launch_dense_widen(const QWeight& w, float* out, hipStream_t s) {
     const int blocks = (int)std::min<int64_t>((count + 255) / 256, 8 * device_info().cu_count);
     switch (w.qtype) {
         case UNILLM_QTYPE_F32:
-            dense_widen_kernel<UNILLM_QTYPE_F32><<<blocks, 256, 0, s>>>(w.base, w.row_bytes, dense_wsc(w), out,
+            dense_widen_kernel<UNILLM_QTYPE_F32><<<blocks, 256, 0, s>>>(w.base, w.row_bytes, out,
                                                                w.n, w.k);
             break;
         case UNILLM_QTYPE_F16:
-            dense_widen_kernel<UNILLM_QTYPE_F16><<<blocks, 256, 0, s>>>(w.base, w.row_bytes, dense_wsc(w), out,
+            dense_widen_kernel<UNILLM_QTYPE_F16><<<blocks, 256, 0, s>>>(w.base, w.row_bytes, out,
                                                                w.n, w.k);
             break;
         default:
-            dense_widen_kernel<UNILLM_QTYPE_BF16><<<blocks, 256, 0, s>>>(w.base, w.row_bytes, dense_wsc(w), out,
+            dense_widen_kernel<UNILLM_QTYPE_BF16><<<blocks, 256, 0, s>>>(w.base, w.row_bytes, out,
                                                                w.n, w.k);
     }
     return hipGetLastError();

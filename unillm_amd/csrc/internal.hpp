@@ -170,7 +170,7 @@ const DeviceInfo& device_info();
 // attention's partials (and, for hd 256 prompts, the rotated queries); slot 3 an
 // aligned copy of x; slot kSyncSlot the batched decode's arrival tickets, zeroed
 // when allocated (every launch leaves them zero again); slot kDenseSlot a dense
-// weight's x in 16-bit parts and its split-k slabs.
+// weight's x in bf16 parts and its split-k slabs.
 constexpr int kSyncSlot = 4;
 constexpr int kDenseSlot = 5;
 hipError_t stream_workspace(hipStream_t s, size_t bytes, void** out, int slot = 0);
@@ -239,11 +239,10 @@ hipError_t launch_x_to_f16_rows(const float* x, int64_t m, int64_t k, void* out,
 hipError_t launch_swiglu(const float* gu, int64_t m, int64_t I, float* act, hipStream_t s);
 
 // Dense (F32 / F16 / BF16) weights: rows in the weight's own type, k padded with zeros
-// (dense_row_bytes a row); F16 rows are held scaled by a power of two each.
+// (dense_row_bytes a row).
 bool is_dense(int qtype);
 int dense_elem_bytes(int qtype);
 int64_t dense_row_bytes(int qtype, int64_t k);
-size_t dense_extra_bytes(int qtype, int64_t n);  // behind the rows: F16's row factors
 // the weight's rows from its GGUF elements at src (device memory), on s
 hipError_t launch_dense_upload(const QWeight& w, const void* src, hipStream_t s);
 // out[n, k] f32 <- the weight's values
