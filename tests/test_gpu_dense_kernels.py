@@ -134,3 +134,33 @@ def test_dense_outlier_behind_zero_weights(dtype, m, n, k, outlier):
     w[:, 20] = 0
     ql = QuantLinear.from_dense(w)
     assert _err(ql.forward(x), x.double() @ w.double().t()) < TOL
+
+
+# rows of x that hold a NaN at their end, and an infinity at their start: right, and soon (the
+# first without a dot; m300 k4096 n2048 measured under 0.1 and 2 ms: the bars leave room for a
+# busy machine)
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(300, 2048, 4096), (40, 300, 1040), (30, 200, 71)])
+def test_dense_non_finite_rows(dtype, m, n, k):
+    w, x = _make(m, n, k, dtype, 3)
+    ql = QuantLinear.from_dense(w)
+    clean = ql.forward(x)
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(4)]
+    bad = x.clone()
+    bad[::2, k - 1] = float("nan")
+    inf = x.clone()
+    inf[1::2, 0] = float("inf")
+    torch.cuda.synchronize()
+    ev[0].record()
+    y = ql.forward(bad)
+    ev[1].record()
+    ev[2].record()
+    z = ql.forward(inf)
+    ev[3].record()
+    torch.cuda.synchronize()
+    assert y[::2].isnan().all() and torch.equal(y[1::2], clean[1::2])
+    ref = inf.double() @ w.double().t()
+    assert torch.equal(z.isnan(), ref.isnan()) and torch.equal(z[z.isinf()].double(), ref[ref.isinf()])
+    assert torch.equal(z[::2], clean[::2])
+    assert ev[0].elapsed_time(ev[1]) < 4.0
+    assert ev[2].elapsed_time(ev[3]) < 30.0

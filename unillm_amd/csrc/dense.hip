@@ -116,15 +116,6 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict_
         orow[i] = (xr[i] - mean) / sd * norm.gamma[i] + (norm.beta ? norm.beta[i] : 0.0f);
 }
 
-// The plain f32 dot of one output: what an output that came out non-finite is
-// recomputed with.
-template <int QT>
-__device__ __noinline__ float dense_dot(const float* x, const uint8_t* row, int64_t k) {
-    float s = 0.0f;
-    for (int64_t i = 0; i < k; ++i) s = fmaf(x[i], widen1<QT>(row, i), s);
-    return s;
-}
-
 __device__ __forceinline__ bool non_finite(float v) {
     return (__float_as_uint(v) & 0x7F800000u) == 0x7F800000u;
 }
@@ -166,6 +157,35 @@ __device__ __forceinline__ float elem8(const Row8<QT>& r, int e) {
     if constexpr (QT == UNILLM_QTYPE_F16)
         return (float)__builtin_bit_cast(_Float16, (uint16_t)(e % 2 ? u >> 16 : u & 0xFFFFu));
     return __uint_as_float(e % 2 ? u & 0xFFFF0000u : u << 16);
+}
+
+// The plain f32 dot of one output, in k order: what an output that came out non-finite is
+// recomputed with.  16 products' operands at a time in flight (more take registers from
+// dense_sum_kernel's waves), and done once the sum is NaN.
+template <int QT>
+__device__ __noinline__ float dense_dot(const float* x, const uint8_t* row, int64_t k) {
+    float s = 0.0f;
+    int64_t i = 0;
+    for (; i + 16 <= k && s == s; i += 16) {
+        Row8<QT> w[2];
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) w[u] = load8<QT>(row, (int)(i / 8) + u);
+        __builtin_memcpy(v, x + i, sizeof(v));
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s = fmaf(v[e], elem8<QT>(w[e / 8], e % 8), s);
+    }
+    for (; i < k && s == s; ++i) s = fmaf(x[i], widen1<QT>(row, i), s);
+    return s;
+}
+
+// A non-finite output again (nan: its row of x holds a NaN).  BF16 m512 k4096 n11008, us a
+// call (169 all finite): every row with a NaN 177, one row with an infinity 509, every row
+// 10700.
+template <int QT>
+__device__ __forceinline__ float dense_redo(uint32_t nan, const float* x, const uint8_t* row,
+                                            int64_t k) {
+    return nan ? __builtin_nanf("") : dense_dot<QT>(x, row, k);
 }
 
 // M: the token count the code is built for (m <= M; x past m is zero and not stored)
@@ -336,15 +356,19 @@ __global__ __launch_bounds__(256) void dense_short_kernel(const uint8_t* __restr
 // ---- x in three bf16 parts ---------------------------------------------------------------
 // xp[p][m][kp]: x = part 0 + part 1 + part 2 exactly (rows padded with zeros to kp), each
 // part what is left rounded to bf16 (split.hpp; a finite value keeps a finite part 0).  A
-// non-finite value keeps its kind in part 0, the others zero.  One workgroup a row; bound by
-// its bytes (4 in, 6 out an element).
+// non-finite value keeps its kind in part 0, the others zero.  nan_row[r]: whether row r holds
+// a NaN (its outputs then are NaN, without a look at the weights).  One workgroup a row; bound
+// by its bytes (4 in, 6 out an element).
 __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x, int64_t k,
                                                      int64_t kp, uint16_t* __restrict__ xp,
-                                                     int64_t plane) {
+                                                     int64_t plane,
+                                                     uint32_t* __restrict__ nan_row) {
     const float* xr = x + (int64_t)blockIdx.x * k;
     uint16_t* o = xp + (int64_t)blockIdx.x * kp;
+    int nan = 0;
     for (int64_t i = threadIdx.x; i < kp; i += 256) {
         const float v = i < k ? xr[i] : 0.0f;
+        nan |= v != v;
         const uint32_t u = __float_as_uint(v);
         uint16_t p0 = (uint16_t)pack_bf16(v, 0.0f), p1 = 0, p2 = 0;
         if (!non_finite(v)) {
@@ -357,6 +381,8 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x
         o[plane + i] = p1;
         o[2 * plane + i] = p2;
     }
+    nan = __syncthreads_or(nan);
+    if (threadIdx.x == 0) nan_row[blockIdx.x] = nan;
 }
 
 // ---- GEMM --------------------------------------------------------------------------------
@@ -423,9 +449,9 @@ __device__ __forceinline__ void split_weights(const u32x4 (&w)[QT == UNILLM_QTYP
 template <int QT, int BM>
 __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(
     const uint8_t* __restrict__ base, int64_t row_bytes, const uint16_t* __restrict__ xp,
-    int64_t plane, int64_t kp, const float* __restrict__ x, int64_t k, float* __restrict__ y,
-    int64_t M, int64_t N, int tiles_n, int tiles, int units_pad, int S, int add,
-    float* __restrict__ part) {
+    int64_t plane, int64_t kp, const uint32_t* __restrict__ nan_row,
+    const float* __restrict__ x, int64_t k, float* __restrict__ y, int64_t M,
+    int64_t N, int tiles_n, int tiles, int units_pad, int S, int add, float* __restrict__ part) {
     using D = DTile<QT, BM>;
     constexpr int TI = D::TI, TJ = D::TJ, NP = D::NP;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -599,7 +625,7 @@ __global__ __launch_bounds__(512, 1) void dense_gemm_kernel(
                     continue;
                 }
                 float v = acc[i][q][e];
-                if (non_finite(v)) v = dense_dot<QT>(x + row * k, base + col * row_bytes, k);
+                if (non_finite(v)) v = dense_redo<QT>(nan_row[row], x + row * k, base + col * row_bytes, k);
                 float* dst = y + row * N + col;
                 *dst = add ? *dst + v : v;
             }
@@ -612,6 +638,7 @@ __global__ __launch_bounds__(256) void dense_sum_kernel(const float* __restrict_
                                                         int64_t M, int64_t N,
                                                         const uint8_t* __restrict__ base,
                                                         int64_t row_bytes,
+                                                        const uint32_t* __restrict__ nan_row,
                                                         const float* __restrict__ x, int64_t k,
                                                         int add, float* __restrict__ y) {
     const int64_t MN = M * N;
@@ -620,7 +647,7 @@ __global__ __launch_bounds__(256) void dense_sum_kernel(const float* __restrict_
         const int64_t row = i / N, col = i % N;
         float v = part[i];
         for (int sl = 1; sl < S; ++sl) v += part[sl * MN + i];
-        if (non_finite(v)) v = dense_dot<QT>(x + row * k, base + col * row_bytes, k);
+        if (non_finite(v)) v = dense_redo<QT>(nan_row[row], x + row * k, base + col * row_bytes, k);
         y[i] = add ? y[i] + v : v;
     }
 }
@@ -666,9 +693,10 @@ DensePlan dense_plan(const QWeight& w, int64_t m) {
 
 size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
-// x parts | slabs
+// x parts | its rows' NaN flags | slabs
 size_t dense_bytes(const QWeight& w, int64_t m, int64_t slab_rows) {
-    return up256((size_t)3 * m * padded_k(w.k) * 2) + (size_t)slab_rows * w.n * 4;
+    return up256((size_t)3 * m * padded_k(w.k) * 2) + up256((size_t)m * 4) +
+           (size_t)slab_rows * w.n * 4;
 }
 
 template <int QT, int BM>
@@ -681,8 +709,10 @@ hipError_t launch_gemm_bm(const QWeight& w, const float* x, int64_t m, float* y,
     if (!attr) return hipErrorInvalidValue;
     const int64_t kp = padded_k(w.k), plane = m * kp;
     uint16_t* xp = static_cast<uint16_t*>(ws);
-    float* part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + up256((size_t)3 * plane * 2));
-    xsplit_kernel<<<(unsigned)m, 256, 0, s>>>(x, w.k, kp, xp, plane);
+    uint32_t* nan_row =
+        reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(ws) + up256((size_t)3 * plane * 2));
+    float* part = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(nan_row) + up256((size_t)m * 4));
+    xsplit_kernel<<<(unsigned)m, 256, 0, s>>>(x, w.k, kp, xp, plane, nan_row);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const int64_t tiles_n = (w.n + D::BN - 1) / D::BN;
@@ -690,13 +720,13 @@ hipError_t launch_gemm_bm(const QWeight& w, const float* x, int64_t m, float* y,
     if (tiles * S > (int64_t)INT32_MAX - 8) return hipErrorInvalidValue;
     const int units_pad = (int)((tiles * S + 7) / 8 * 8);
     dense_gemm_kernel<QT, BM><<<units_pad, 512, D::BYTES, s>>>(
-        w.base, w.row_bytes, xp, plane, kp, x, w.k, y, m, w.n, (int)tiles_n, (int)tiles, units_pad,
-        S, add, part);
+        w.base, w.row_bytes, xp, plane, kp, nan_row, x, w.k, y, m, w.n, (int)tiles_n, (int)tiles,
+        units_pad, S, add, part);
     if ((e = hipGetLastError()) != hipSuccess || S == 1) return e;
     const int blocks =
         (int)std::min<int64_t>((m * w.n + 255) / 256, 8 * (int64_t)device_info().cu_count);
-    dense_sum_kernel<QT><<<blocks, 256, 0, s>>>(part, S, m, w.n, w.base, w.row_bytes, x, w.k, add,
-                                                y);
+    dense_sum_kernel<QT><<<blocks, 256, 0, s>>>(part, S, m, w.n, w.base, w.row_bytes, nan_row, x,
+                                                w.k, add, y);
     return hipGetLastError();
 }
 
