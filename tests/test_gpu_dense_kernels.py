@@ -164,3 +164,29 @@ def test_dense_non_finite_rows(dtype, m, n, k):
     assert torch.equal(z[::2], clean[::2])
     assert ev[0].elapsed_time(ev[1]) < 4.0
     assert ev[2].elapsed_time(ev[3]) < 30.0
+
+
+# calls that run in several chunks of rows (k 65536: 640 rows each), and more rows than a
+# launch of one workgroup each holds (2^24): of x, and of a weight whose k is padded
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_dense_row_chunks(dtype):
+    m, n, k = 1300, 70, 65536
+    w, x = _make(m, n, k, dtype, 4)
+    ql = QuantLinear.from_dense(w)
+    y, ref = ql.forward(x), x.double() @ w.double().t()
+    assert _err(y, ref) < 4 * TOL  # (f32 rounds once a k: 4 times the sum length of TOL's)
+    for r in (0, 640, 1280):
+        assert torch.equal(ql.forward(x[r:r + 640].contiguous()), y[r:r + 640])
+
+
+def test_dense_very_many_rows():
+    m, n, k = (1 << 24) + 300, 3, 6
+    w, x = _make(m, n, k, torch.bfloat16, 6)
+    y = QuantLinear.from_dense(w).forward(x)
+    assert _err(y[-1000:], x[-1000:].double() @ w.double().t()) < TOL
+    assert _err(y[::4099], x[::4099].double() @ w.double().t()) < TOL
+    del x, y
+    w, x = _make(2, m, 2, torch.float16, 7)
+    ql = QuantLinear.from_dense(w)
+    assert _err(ql.forward(x), x.double() @ w.double().t()) < TOL
+    assert torch.equal(ql.dequantize()[-5000:], w[-5000:].float())

@@ -54,15 +54,17 @@ int64_t padded_k(int64_t k) { return (k + kKPad - 1) / kKPad * kKPad; }
 
 // ---- upload, dequant, layer norm ---------------------------------------------------------
 
-// dst row r (row_bytes) <- src row r (k elements), a workgroup a row; the padding was
-// zeroed when the weight was allocated
+// dst row r (row_bytes) <- src row r (k elements), a workgroup a row at a time; the padding
+// was zeroed when the weight was allocated
 template <class T>
 __global__ __launch_bounds__(256) void dense_upload_kernel(const T* __restrict__ src,
-                                                           uint8_t* __restrict__ dst, int64_t k,
-                                                           int64_t row_bytes) {
-    const T* sr = src + (int64_t)blockIdx.x * k;
-    T* dr = reinterpret_cast<T*>(dst + (int64_t)blockIdx.x * row_bytes);
-    for (int64_t i = threadIdx.x; i < k; i += 256) dr[i] = sr[i];
+                                                           uint8_t* __restrict__ dst, int64_t n,
+                                                           int64_t k, int64_t row_bytes) {
+    for (int64_t r = blockIdx.x; r < n; r += gridDim.x) {
+        const T* sr = src + r * k;
+        T* dr = reinterpret_cast<T*>(dst + r * row_bytes);
+        for (int64_t i = threadIdx.x; i < k; i += 256) dr[i] = sr[i];
+    }
 }
 
 // weight i of a row
@@ -693,6 +695,13 @@ DensePlan dense_plan(const QWeight& w, int64_t m) {
 
 size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
+// Rows of x a launch takes: their parts within 256 MiB (k 4096: 10880 rows, 85 tiles of 128),
+// so that a stream's workspace, which is kept, and the launch's 2^32 threads hold any m.
+int64_t dense_chunk_rows(const QWeight& w) {
+    const int64_t rows = ((int64_t)256 << 20) / (6 * padded_k(w.k));
+    return rows >= 128 ? rows / 128 * 128 : std::max<int64_t>(rows, 1);
+}
+
 // x parts | its rows' NaN flags | slabs
 size_t dense_bytes(const QWeight& w, int64_t m, int64_t slab_rows) {
     return up256((size_t)3 * m * padded_k(w.k) * 2) + up256((size_t)m * 4) +
@@ -741,12 +750,20 @@ hipError_t launch_dense_qt(const QWeight& w, const float* x, int64_t m, float* y
                                                     add);
         return hipGetLastError();
     }
-    const DensePlan p = dense_plan(w, m);
-    void* ws = nullptr;
-    const hipError_t e = stream_workspace(s, dense_bytes(w, m, p.S > 1 ? p.S * m : 0), &ws, kDenseSlot);
-    if (e != hipSuccess) return e;
-    return p.bm == 64 ? launch_gemm_bm<QT, 64>(w, x, m, y, p.S, ws, s, add)
-                      : launch_gemm_bm<QT, 128>(w, x, m, y, p.S, ws, s, add);
+    const int64_t chunk = dense_chunk_rows(w);
+    for (int64_t r = 0; r < m; r += chunk) {
+        const int64_t rows = std::min(chunk, m - r);
+        const DensePlan p = dense_plan(w, rows);
+        void* ws = nullptr;
+        hipError_t e =
+            stream_workspace(s, dense_bytes(w, rows, p.S > 1 ? p.S * rows : 0), &ws, kDenseSlot);
+        if (e != hipSuccess) return e;
+        e = p.bm == 64
+                ? launch_gemm_bm<QT, 64>(w, x + r * w.k, rows, y + r * w.n, p.S, ws, s, add)
+                : launch_gemm_bm<QT, 128>(w, x + r * w.k, rows, y + r * w.n, p.S, ws, s, add);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace
@@ -763,12 +780,14 @@ hipError_t launch_dense_upload(const QWeight& w, const void* src, hipStream_t s)
     if (w.k % kKPad == 0)
         return hipMemcpyAsync(w.base, src, (size_t)w.n * (size_t)w.row_bytes,
                               hipMemcpyDeviceToDevice, s);
+    // (a launch holds at most 2^32 threads: 2^24 rows of 256)
+    const unsigned blocks = (unsigned)std::min<int64_t>(w.n, (int64_t)1 << 20);
     if (w.qtype == UNILLM_QTYPE_F32)
-        dense_upload_kernel<<<(unsigned)w.n, 256, 0, s>>>(static_cast<const uint32_t*>(src), w.base,
-                                                          w.k, w.row_bytes);
+        dense_upload_kernel<<<blocks, 256, 0, s>>>(static_cast<const uint32_t*>(src), w.base, w.n,
+                                                   w.k, w.row_bytes);
     else
-        dense_upload_kernel<<<(unsigned)w.n, 256, 0, s>>>(static_cast<const uint16_t*>(src), w.base,
-                                                          w.k, w.row_bytes);
+        dense_upload_kernel<<<blocks, 256, 0, s>>>(static_cast<const uint16_t*>(src), w.base, w.n,
+                                                   w.k, w.row_bytes);
     return hipGetLastError();
 }
 
@@ -800,6 +819,7 @@ hipError_t launch_norm_rows(const float* x, int64_t m, int64_t k, const NormArgs
 // A bound for every call of up to m rows: the GEMV takes none; slices x rows of a split
 // are at most kDenseMaxSlices m, and at most 128 kDenseMaxRounds CUs / (column tiles).
 size_t dense_workspace_bytes(const QWeight& w, int64_t m) {
+    m = std::min(m, dense_chunk_rows(w));
     const int64_t tiles_n = (w.n + dense_bn(w) - 1) / dense_bn(w);
     const int64_t rows =
         padded_k(w.k) / kKPad < 8
