@@ -123,3 +123,30 @@ def test_batch_on_the_prefill(qtype, m, n, k, tiles):
         ql._h, x.data_ptr(), m, z.data_ptr(), int(torch.cuda.current_stream().cuda_stream)))
     torch.cuda.synchronize()
     assert close(z)
+
+
+# a batch's x is scaled by slices of at most 1024 k on the prefill's tiles too: a value far
+# larger than the rest of its row (behind 1024 zero weights) costs the other slices nothing
+@pytest.mark.parametrize("qtype", [Q4_0, Q8_0, Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("m,n,k", [(64, 4096, 14336), (50, 2900, 14592), (64, 28672, 4096)])
+def test_batch_outlier_keeps_the_other_slices(qtype, m, n, k):
+    print(f"batch outlier qtype={qtype} m={m} n={n} k={k}", flush=True)
+    size, elems, scales = BLOCK[qtype]
+    rng = np.random.default_rng(5)
+    b = rng.integers(0, 256, (n, k // elems, size), dtype=np.uint8)
+    for off in scales:
+        d = rng.uniform(0.5e-3, 2e-3, b.shape[:2]).astype(np.float16)
+        d[:, : 1024 // elems] = 0
+        b[:, :, off:off + 2] = d.view(np.uint8).reshape(n, -1, 2)
+    ql = QuantLinear.from_blocks(qtype, n, k, b.tobytes())
+    x = torch.randn(m, k, device="cuda", generator=torch.Generator("cuda").manual_seed(m))
+    x[:, 3] = 1e13
+    x[::2, 3] = 1e30
+    w = ql.dequantize()
+    assert not w[:, :1024].any()
+    ref = x[:, 1024:].double() @ w[:, 1024:].double().t()
+    y = ql.forward(x)
+    assert _err(y, ref) < TOL
+    r = torch.randn_like(y)
+    want = r.double() + ref
+    assert _err(ql.forward_add(x, r), want) < TOL

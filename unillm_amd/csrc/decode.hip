@@ -279,8 +279,6 @@ __global__ __launch_bounds__(128) void xprep_kernel(const float* __restrict__ x,
 // rotation put the rows (tokens) that one LDS read pass serves -- 8 or 16
 // consecutive lanes -- on distinct banks.
 constexpr int kMaxSliceChunks = 8;
-// most k slices of one row (a row of up to 256 * 8 * 128 = 262144 elements)
-constexpr int kMaxSplitSlices = 256;
 // At most this many k slices add into one output when the row groups alone leave
 // CUs idle: 8 for one 32-token tile (m16 n4096: 9.9 us a call against 11.1 with 4),
 // 4 for two (more slices contend on the same y lines with their atomics; m64 n4096:
@@ -1277,6 +1275,12 @@ hipError_t launch_norm_convert(const float* x, int64_t m, int64_t k, const NormA
     return hipGetLastError();
 }
 
+hipError_t launch_x_to_f16_slices(const float* x, int64_t m, int64_t k, int S, void* out,
+                                  float* rf, float* y, int64_t ny, hipStream_t s) {
+    xprep_kernel<<<(unsigned)(m * S), 128, 0, s>>>(x, k, S, static_cast<uint4*>(out), rf, y, ny);
+    return hipGetLastError();
+}
+
 hipError_t launch_x_to_f16_rows(const float* x, int64_t m, int64_t k, void* out, float* rs,
                                 hipStream_t s) {
     if (m <= 0) return hipSuccess;
@@ -1338,8 +1342,9 @@ size_t decode_x_bytes(const QWeight& w, int64_t m) {
 
 size_t decode_workspace_bytes(const QWeight& w, int64_t m, const NormArgs& norm) {
     if (decode_one_launch(w, m, norm)) return 0;
-    const size_t own = decode_x_bytes(w, m) + (size_t)decode_split(w, m) * 64 * sizeof(float);
-    return prefill_takes_batch(w, m) ? std::max(own, prefill_call_bytes(w, m)) : own;
+    const int S = decode_split(w, m);
+    const size_t own = decode_x_bytes(w, m) + (size_t)S * 64 * sizeof(float);
+    return prefill_takes_batch(w, m) ? std::max(own, prefill_call_bytes(w, m, 0, S)) : own;
 }
 
 size_t decode_sync_bytes(const QWeight& w) { return xin_sync_bytes((w.n + DROWS - 1) / DROWS); }
@@ -1353,9 +1358,10 @@ hipError_t launch_decode_mfma(const QWeight& w, const float* x, int64_t m, float
     const bool q4 = w.qtype == UNILLM_QTYPE_Q4_0, k4 = w.qtype == UNILLM_QTYPE_Q4_K,
                k5 = w.qtype == UNILLM_QTYPE_Q5_K, k6 = w.qtype == UNILLM_QTYPE_Q6_K, wide = m > 32;
     hipError_t e = hipSuccess;
-    if (prefill_takes_batch(w, m))  // (deep or large weights at 33 .. 64 rows)
+    if (prefill_takes_batch(w, m))  // (deep or large weights at 33 .. 64 rows; x scaled the same)
         return launch_prefill_mfma(w, x, m, y, s, epi, norm, ws,
-                                   ws ? decode_workspace_bytes(w, m, norm) : 0);
+                                   ws ? decode_workspace_bytes(w, m, norm) : 0,
+                                   decode_split(w, m));
     if (decode_one_launch(w, m, norm)) {
         // x converted by the kernel itself; the stream's workspace holds the row groups'
         // arrival tickets (zeroed when allocated, reset by each launch)
@@ -1393,9 +1399,7 @@ hipError_t launch_decode_mfma(const QWeight& w, const float* x, int64_t m, float
             hipSuccess)
             return e;
     } else {
-        xprep_kernel<<<(unsigned)(m * S), 128, 0, s>>>(x, w.k, S, static_cast<uint4*>(ws), rf, y,
-                                                        ny);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if ((e = launch_x_to_f16_slices(x, m, w.k, S, ws, rf, y, ny, s)) != hipSuccess) return e;
     }
     const _Float16* xh = static_cast<const _Float16*>(ws);
     if (k4)

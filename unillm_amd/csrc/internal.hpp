@@ -202,7 +202,7 @@ hipError_t launch_decode_mfma(const QWeight& w, const float* x, int64_t m, float
 hipError_t launch_prefill_mfma(const QWeight& w, const float* x, int64_t m, float* y,
                                hipStream_t s, int epi = kEpiStore,
                                const NormArgs& norm = NormArgs{nullptr, nullptr, 0.f},
-                               void* ws = nullptr, size_t ws_bytes = 0);
+                               void* ws = nullptr, size_t ws_bytes = 0, int slices = 0);
 // The batched decode's x operand workspace (0 where the kernel converts x itself),
 // and its arrival tickets.
 // (no default for norm: the size depends on it)
@@ -212,9 +212,10 @@ size_t decode_sync_bytes(const QWeight& w);
 // cap bytes, which may pick a plan without a k split), and a bound for every call
 // of up to m rows (the size a reserve takes).
 // (prefill_takes_batch: calls of up to kDecodeMaxM rows that the batched decode's path
-// hands to the prefill's tiles)
+// hands to the prefill's tiles; slices > 0: such a call, whose x is scaled by the batched
+// decode's k slices instead of by whole rows)
 bool prefill_takes_batch(const QWeight& w, int64_t m);
-size_t prefill_call_bytes(const QWeight& w, int64_t m, size_t cap = 0);
+size_t prefill_call_bytes(const QWeight& w, int64_t m, size_t cap = 0, int slices = 0);
 size_t prefill_workspace_bytes(const QWeight& w, int64_t m);
 // Both MFMA paths address weight bytes with 32-bit offsets: weights under 4 GiB.
 inline bool mfma_supports(const QWeight& w) {
@@ -227,6 +228,10 @@ inline bool mfma_supports(const QWeight& w) {
 hipError_t launch_norm_convert(const float* x, int64_t m, int64_t k, const NormArgs& norm,
                                void* out, float* y, int64_t ny, hipStream_t s,
                                float* rs = nullptr, int S = 0, float* rf = nullptr);
+// The same scaling of x[m, k] by S slices without a norm (the batched decode's: 128-k chunks
+// [s C / S, (s + 1) C / S) of C = ceil(k / 128), at most 8 each).
+hipError_t launch_x_to_f16_slices(const float* x, int64_t m, int64_t k, int S, void* out,
+                                  float* rf, float* y, int64_t ny, hipStream_t s);
 // x[m, k] (k % 32 == 0) -> f16 rows (round to nearest even) in the decode kernel's
 // element order (each aligned 8 as 0 2 1 3 4 6 5 7), each row scaled by a power
 // of two that puts its largest magnitude in [2^14, 2^15); rs[row] <- the factor
@@ -273,5 +278,7 @@ int64_t attention_max_positions();  // len + m per call
 
 constexpr int64_t kGemvMaxM = 4;
 constexpr int64_t kDecodeMaxM = 64;
+// most k slices of one row (a row of up to 256 * 8 * 128 = 262144 elements)
+constexpr int kMaxSplitSlices = 256;
 
 }  // namespace unillm

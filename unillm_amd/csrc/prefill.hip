@@ -188,16 +188,27 @@ struct Ring {
     static constexpr int DMA = AQ + CPB / 2 + 1 + (KQ ? 1 : 0);  // direct loads per wave per stage
 };
 
-template <int QT, int BM, int NW>
-__global__ __launch_bounds__(NW * 64, BM == 64 ? 4 : 1) void prefill_kernel(const uint8_t* __restrict__ base,
-                                                              int64_t rb,
-                                                              const uint16_t* __restrict__ xb,
-                                                              float* __restrict__ y, int M, int N,
-                                                              int KB, int tiles_n, int tiles,
-                                                              int units_pad, int S, int add,
-                                                              float wscale, float oscale,
-                                                              const float* __restrict__ rs,
-                                                              float* __restrict__ part, int swi) {
+// Slice s of the SD slices that the batched decode scales a row's k by: 128-k chunks
+// [s C / SD, (s + 1) C / SD) of C = ceil(k / 128), so k steps from twice that on.
+__host__ __device__ __forceinline__ int slice_step(int s, int SD, int C) {
+    return 2 * (int)((int64_t)s * C / SD);
+}
+__host__ __device__ __forceinline__ int slice_of_step(int ks, int SD, int C) {
+    int s = (int)((int64_t)(ks / 2) * SD / C);
+    while (slice_step(s + 1, SD, C) <= ks) ++s;
+    return s;
+}
+
+// SEG: x is scaled by slices of a row's k (SD of them, rs[s * 64 + row], m <= 64), as the
+// batched decode scales it, and a slice's sums are scaled back and added to the total where
+// the slice ends; else by whole rows (rs[row]).
+template <int QT, int BM, int NW, bool SEG>
+__global__ __launch_bounds__(NW * 64, BM == 64 && !SEG ? 4 : 1) void prefill_kernel(
+    const uint8_t* __restrict__ base, int64_t rb, const uint16_t* __restrict__ xb,
+    float* __restrict__ y, int M, int N, int KB, int tiles_n, int tiles, int units_pad, int S,
+    int add, float wscale, float oscale, const float* __restrict__ rs, int SD,
+    float* __restrict__ part, int swi) {
+    static_assert(!SEG || BM == 64, "slice factors for 64 rows");
     static_assert(NW == 8, "the ring's load split assumes 8 waves");
     constexpr int QB = Ring<QT, BM>::QB;  // payload bytes per block
     // waves: RW row groups x CW column groups; wave (rw, cw) owns rows BM / RW * rw ..
@@ -333,10 +344,19 @@ __global__ __launch_bounds__(NW * 64, BM == 64 ? 4 : 1) void prefill_kernel(cons
     for (int i = 0; i < TI; ++i)
 #pragma unroll
         for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 tot[SEG ? TI : 1][TJ] = {};  // SEG: the slices' sums, scaled back
+    // SEG: the slice being summed and the step it ends before
+    const int chunks = (KB + 3) / 4;
+    const int seg0 = SEG ? slice_of_step(ks0, SD, chunks) : 0;
+    int seg = seg0, seg_end = SEG ? slice_step(seg0 + 1, SD, chunks) : 0;
 
-    // prologue: the tile's row scales (f16 operands; wave 0, ahead of its ring loads, so
-    // the ring's waits cover them), then stages 0 .. kStages - 2 in flight
-    if (wv == 0) {
+    // prologue: the tile's row scales, or the factors of this unit's slices (f16 operands;
+    // wave 0, ahead of its ring loads, so the ring's waits cover them), then stages
+    // 0 .. kStages - 2 in flight
+    if (SEG && wv == 0) {
+        const int last = slice_of_step(ks0 + nks - 1, SD, chunks);
+        for (int q = seg0; q <= last; ++q) dma4(rs + 64 * q + lane, ring + R::RS + (q - seg0) * 256);
+    } else if (wv == 0) {
 #pragma unroll
         for (int q = 0; q < BM / 64; ++q)
             dma4(rs + min(m0 + 64 * q + lane, M - 1), ring + R::RS + q * 256);
@@ -472,6 +492,30 @@ __global__ __launch_bounds__(NW * 64, BM == 64 ? 4 : 1) void prefill_kernel(cons
             static_assert(SPC >= 1, "a load slot for every direct load");
             if (issue_next && f % SPC == 0 && f / SPC < R::DMA) issue_one(ks + kStages - 1, f / SPC);
         }
+        if constexpr (SEG) {
+            if (ks + 1 == seg_end || j + 1 == nks) {
+                const uint32_t fa = ring0 + R::RS + (uint32_t)(seg - seg0) * 256 + 16 * g;
+                u32x4 fac[TI];
+                static_assert(TI == 4, "64 rows");
+                constexpr_for<TI>([&](auto I) { fac[I.value] = lds_read128<I.value * 64>(fa); });
+                asm volatile("s_waitcnt lgkmcnt(0)"
+                             : "+v"(fac[0]), "+v"(fac[1]), "+v"(fac[2]), "+v"(fac[3]));
+#pragma unroll
+                for (int i = 0; i < TI; ++i)
+#pragma unroll
+                    for (int c = 0; c < TJ; ++c) {
+                        tot[i][c] += acc[i][c] * __builtin_bit_cast(f32x4, fac[i]);
+                        acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+                seg_end = slice_step(++seg + 1, SD, chunks);
+            }
+        }
+    }
+    if constexpr (SEG) {
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) acc[i][j] = tot[i][j];
     }
 
     // ---- epilogue: lane holds C[4 (l / 16) + e][l % 16] of each 16 x 16 tile.  One
@@ -498,7 +542,8 @@ __global__ __launch_bounds__(NW * 64, BM == 64 ? 4 : 1) void prefill_kernel(cons
 #pragma unroll
     for (int i = 0; i < TI; ++i) {
         const float4 r4 =
-            *reinterpret_cast<const float4*>(ring + R::RS + (WR * rw + 16 * i + 4 * g) * 4);
+            SEG ? make_float4(1.0f, 1.0f, 1.0f, 1.0f)
+                : *reinterpret_cast<const float4*>(ring + R::RS + (WR * rw + 16 * i + 4 * g) * 4);
         rsc[i] = make_float4(r4.x * oscale, r4.y * oscale, r4.z * oscale, r4.w * oscale);
     }
     if (swi) {  // act = silu(gate) * up (candle's silu, v / (1 + e^-v))
@@ -534,7 +579,8 @@ __global__ __launch_bounds__(NW * 64, BM == 64 ? 4 : 1) void prefill_kernel(cons
     }
 }
 
-// y[r, c] (+)= (sum over the S slabs of part[s][r][c], in slice order) * rs[r] * oscale:
+// y[r, c] (+)= (sum over the S slabs of part[s][r][c], in slice order) * rs[r] * oscale
+// (rs null: 1):
 // the k slices of a split prefill, in a fixed order (the result does not depend on
 // which slice finished first).  Four columns a thread when vec (n % 4 == 0 and y on
 // a 16-byte boundary).
@@ -550,7 +596,7 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict_
             f32x4 v = *reinterpret_cast<const f32x4*>(part + 4 * q);
             for (int sl = 1; sl < S; ++sl)
                 v += *reinterpret_cast<const f32x4*>(part + sl * MN + 4 * q);
-            v *= rs[4 * q / N] * oscale;
+            v *= rs ? rs[4 * q / N] * oscale : oscale;
             f32x4* dst = reinterpret_cast<f32x4*>(y + 4 * q);
             *dst = add ? *dst + v : v;
         }
@@ -559,7 +605,7 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict_
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < MN; i += stride) {
         float v = part[i];
         for (int sl = 1; sl < S; ++sl) v += part[sl * MN + i];
-        v *= rs[i / N] * oscale;
+        v *= rs ? rs[i / N] * oscale : oscale;
         y[i] = add ? y[i] + v : v;
     }
 }
@@ -577,7 +623,7 @@ __global__ __launch_bounds__(256) void split_swiglu_kernel(const float* __restri
     const int64_t w = vec ? I / 4 : I;  // units of a row
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < M * w; q += stride) {
         const int64_t row = q / w, c = (q - row * w) * (vec ? 4 : 1);
-        const float f = rs[row] * oscale;
+        const float f = rs ? rs[row] * oscale : oscale;
         const float* g0 = part + row * 2 * I + c;
         if (vec) {
             f32x4 g = *reinterpret_cast<const f32x4*>(g0), u = *reinterpret_cast<const f32x4*>(g0 + I);
@@ -600,32 +646,44 @@ __global__ __launch_bounds__(256) void split_swiglu_kernel(const float* __restri
     }
 }
 
+constexpr int kMaxLds = 160 << 10;
+
+// The most slices (of SD) that the k steps of one of S units touch.
+int unit_slices(const QWeight& w, int S, int SD) {
+    const int ksteps = (int)((w.kb + 1) / 2), chunks = (int)((w.kb + 3) / 4);
+    int most = 1;
+    for (int sp = 0; sp < S; ++sp) {
+        const int a = (int)((int64_t)sp * ksteps / S), b = (int)((int64_t)(sp + 1) * ksteps / S);
+        most = std::max(most, slice_of_step(b - 1, SD, chunks) - slice_of_step(a, SD, chunks) + 1);
+    }
+    return most;
+}
+
 // x is addressed with 32-bit element offsets: a launch takes at most this many rows
 int64_t prefill_chunk_rows(int64_t k, int bm) {
     return std::max<int64_t>(bm, ((int64_t)1 << 30) / k / bm * bm);
 }
 
-// epi: kEpiStore, kEpiAdd, or kEpiSwiglu (y is then act[m, n / 2])
-template <int QT, int BM>
-hipError_t launch_bm(const QWeight& w, const uint16_t* xb, const float* rs, int64_t m, float* y,
-                     int S, float* part, hipStream_t s, int epi) {
+// epi: kEpiStore, kEpiAdd, or kEpiSwiglu (y is then act[m, n / 2]).  SD: the slices x is
+// scaled by (rs their factors), 0 for whole rows.
+template <int QT, int BM, bool SEG = false>
+hipError_t launch_bm(const QWeight& w, const uint16_t* xb, const float* rs, int SD, int64_t m,
+                     float* y, int S, float* part, hipStream_t s, int epi) {
     const int64_t chunk = prefill_chunk_rows(w.k, BM), I = w.n / 2;
     const bool act = epi == kEpiSwiglu;
     if (m > chunk) {  // row chunks below 2^30 elements (the plan never splits k here)
         if (S != 1) return hipErrorInvalidValue;
         for (int64_t r = 0; r < m; r += chunk) {
-            hipError_t e = launch_bm<QT, BM>(w, xb + r * w.k, rs ? rs + r : nullptr,
-                                             std::min(chunk, m - r), y + r * (act ? I : w.n), 1,
-                                             nullptr, s, epi);
+            hipError_t e =
+                launch_bm<QT, BM>(w, xb + r * w.k, rs + r, 0, std::min(chunk, m - r),
+                                  y + r * (act ? I : w.n), 1, nullptr, s, epi);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
     }
-    static bool attr = [] {
-        return hipFuncSetAttribute((const void*)prefill_kernel<QT, BM, kWaves>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   Ring<QT, BM>::BYTES) == hipSuccess;
-    }();
+    static const bool attr = hipFuncSetAttribute((const void*)prefill_kernel<QT, BM, kWaves, SEG>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 SEG ? kMaxLds : Ring<QT, BM>::BYTES) == hipSuccess;
     if (!attr) return hipErrorInvalidValue;
     const int swi = act && S == 1 ? (int)I : 0;  // (a split k's sums meet in a pass of their own)
     const int tiles_m = (int)((m + BM - 1) / BM);
@@ -633,9 +691,11 @@ hipError_t launch_bm(const QWeight& w, const uint16_t* xb, const float* rs, int6
     const int tiles = tiles_m * tiles_n;
     const int units_pad = (tiles * S + 7) / 8 * 8;
     const float wscale = ldexpf(1.0f, -w.f16_exp), oscale = ldexpf(1.0f, w.f16_exp);
-    prefill_kernel<QT, BM, kWaves><<<units_pad, kWaves * 64, Ring<QT, BM>::BYTES, s>>>(
+    const int lds = SEG ? Ring<QT, BM>::RS + 256 * unit_slices(w, S, SD) : Ring<QT, BM>::BYTES;
+    if (lds > kMaxLds) return hipErrorInvalidValue;
+    prefill_kernel<QT, BM, kWaves, SEG><<<units_pad, kWaves * 64, lds, s>>>(
         w.base, w.row_bytes, xb, y, (int)m, (int)w.n, (int)w.kb, tiles_n, tiles, units_pad, S,
-        epi == kEpiAdd, wscale, oscale, rs, part, swi);
+        epi == kEpiAdd, wscale, oscale, rs, SD, part, swi);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || S == 1) return e;
     const int64_t cols = act ? I : w.n;
@@ -643,10 +703,12 @@ hipError_t launch_bm(const QWeight& w, const uint16_t* xb, const float* rs, int6
     const int64_t q = m * cols / (vec ? 4 : 1);
     const int blocks =
         (int)std::min<int64_t>(std::max<int64_t>(1, (q + 255) / 256), 8 * device_info().cu_count);
+    const float* row_scale = SEG ? nullptr : rs;
     if (act)
-        split_swiglu_kernel<<<blocks, 256, 0, s>>>(part, S, m, I, rs, oscale, vec, y);
+        split_swiglu_kernel<<<blocks, 256, 0, s>>>(part, S, m, I, row_scale, oscale, vec, y);
     else
-        split_sum_kernel<<<blocks, 256, 0, s>>>(part, S, m, w.n, rs, oscale, epi == kEpiAdd, vec, y);
+        split_sum_kernel<<<blocks, 256, 0, s>>>(part, S, m, w.n, row_scale, oscale, epi == kEpiAdd,
+                                                vec, y);
     return hipGetLastError();
 }
 
@@ -666,11 +728,16 @@ struct PrefillPlan {
 constexpr int64_t kMaxSlices = 16, kMinSteps = 4;
 size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
+// The scales of x's rows, or of their SD slices
+size_t scale_bytes(int64_t m, int SD) {
+    return up256((SD > 0 ? (size_t)SD * 64 : (size_t)m) * sizeof(float));
+}
+
 // The workspace a plan takes: x as f16 rows | their scales | the split slabs
 // ([S][m][n] f32)
-size_t plan_bytes(const QWeight& w, int64_t m, int S) {
+size_t plan_bytes(const QWeight& w, int64_t m, int S, int SD) {
     const size_t slabs = S > 1 ? (size_t)S * m * w.n * sizeof(float) : 0;
-    return up256((size_t)m * (size_t)w.k * 2) + up256((size_t)m * sizeof(float)) + slabs;
+    return up256((size_t)m * (size_t)w.k * 2) + scale_bytes(m, SD) + slabs;
 }
 
 // ns of a k step of 64, 128 and 256 rows (n28672 k4096, one workgroup a CU)
@@ -686,16 +753,18 @@ int64_t step_ns(int qtype, int bm) {
 
 // cap > 0: a caller's fixed workspace of cap bytes; a split plan that does not fit it is
 // not taken (at worst the tiles unsplit)
-PrefillPlan prefill_plan(const QWeight& w, int64_t m, size_t cap = 0) {
+// (SD > 0: 64-row tiles, the cheapest for m <= 64 in any case)
+PrefillPlan prefill_plan(const QWeight& w, int64_t m, size_t cap = 0, int SD = 0) {
     const int64_t cus = device_info().cu_count;
     const int64_t tiles_n = (w.n + PBN - 1) / PBN, ksteps = (w.kb + 1) / 2;
     PrefillPlan best{128, 1};
     int64_t least = INT64_MAX;
     for (int bm : {64, 128, 256}) {
+        if (SD > 0 && bm > 64) break;
         const int64_t tiles = (m + bm - 1) / bm * tiles_n;
         for (int64_t S = 1; S <= kMaxSlices; ++S) {
             if (S > 1 && (tiles * S > cus || ksteps < kMinSteps * S || m > prefill_chunk_rows(w.k, bm) ||
-                          (cap > 0 && plan_bytes(w, m, (int)S) > cap)))
+                          (cap > 0 && plan_bytes(w, m, (int)S, SD) > cap)))
                 break;
             const int64_t rounds = (tiles * S + cus - 1) / cus;
             int64_t ns = rounds * ((ksteps + S - 1) / S) * step_ns(w.qtype, bm);
@@ -714,8 +783,8 @@ PrefillPlan prefill_plan(const QWeight& w, int64_t m, size_t cap = 0) {
 // The call's own need (for a caller's fixed workspace of cap bytes, cap > 0, the plan
 // that fits it), and a bound for every m' <= m, so that a reserve for m covers every
 // shorter call.
-size_t prefill_call_bytes(const QWeight& w, int64_t m, size_t cap) {
-    return plan_bytes(w, m, prefill_plan(w, m, cap).S);
+size_t prefill_call_bytes(const QWeight& w, int64_t m, size_t cap, int slices) {
+    return plan_bytes(w, m, prefill_plan(w, m, cap, slices).S, slices);
 }
 
 size_t prefill_workspace_bytes(const QWeight& w, int64_t m) {
@@ -727,7 +796,8 @@ size_t prefill_workspace_bytes(const QWeight& w, int64_t m) {
                            : std::min<int64_t>(kMaxSlices * m,
                                                256 * device_info().cu_count / tiles_n);
     const size_t slabs = (size_t)sm * w.n * sizeof(float);
-    return up256((size_t)m * (size_t)w.k * 2) + up256((size_t)m * sizeof(float)) + slabs;
+    return up256((size_t)m * (size_t)w.k * 2) +
+           std::max(scale_bytes(m, 0), scale_bytes(0, kMaxSplitSlices)) + slabs;
 }
 
 // 49 .. 64 rows (Q8_0: 33 .. 64) of a deep or large weight run here rather than on the
@@ -746,30 +816,36 @@ bool prefill_takes_batch(const QWeight& w, int64_t m) {
 
 hipError_t launch_prefill_mfma(const QWeight& w, const float* x, int64_t m, float* y,
                                hipStream_t s, int epi, const NormArgs& norm, void* ws,
-                               size_t ws_bytes) {
+                               size_t ws_bytes, int slices) {
     // weight bytes are addressed with 32-bit offsets (pcol_off, ssrc)
     if (!mfma_supports(w)) return hipErrorInvalidValue;
     // x as f16 rows with their power-of-two scales in the workspace: the GEMM
     // re-reads x once per 256-column tile, so it reads half the bytes, and no
     // conversion sits in its inner loop.  A split k's slabs follow.
-    const PrefillPlan plan = prefill_plan(w, m, ws ? ws_bytes : 0);
+    const PrefillPlan plan = prefill_plan(w, m, ws ? ws_bytes : 0, slices);
     const size_t xbytes = up256((size_t)m * (size_t)w.k * 2);
+    const size_t need = plan_bytes(w, m, plan.S, slices);
     hipError_t e = hipSuccess;
-    if (ws && plan_bytes(w, m, plan.S) > ws_bytes) return hipErrorInvalidValue;
-    if (!ws && (e = stream_workspace(s, plan_bytes(w, m, plan.S), &ws)) != hipSuccess) return e;
+    if (ws && need > ws_bytes) return hipErrorInvalidValue;
+    if (!ws && (e = stream_workspace(s, need, &ws)) != hipSuccess) return e;
     float* rs = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + xbytes);
-    float* part =
-        plan.S > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + xbytes +
-                                              up256((size_t)m * sizeof(float)))
-                   : nullptr;
-    e = norm.gamma ? launch_norm_convert(x, m, w.k, norm, ws, y, 0, s, rs)
+    float* part = plan.S > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + xbytes +
+                                                        scale_bytes(m, slices))
+                             : nullptr;
+    if (norm.gamma)
+        e = launch_norm_convert(x, m, w.k, norm, ws, y, 0, s, slices ? nullptr : rs, slices,
+                                slices ? rs : nullptr);
+    else
+        e = slices ? launch_x_to_f16_slices(x, m, w.k, slices, ws, rs, y, 0, s)
                    : launch_x_to_f16_rows(x, m, w.k, ws, rs, s);
     if (e != hipSuccess) return e;
     const uint16_t* xb = static_cast<const uint16_t*>(ws);
-#define UNILLM_PREFILL_LAUNCH(QTYPE)                                                          \
-    return plan.bm == 256   ? launch_bm<QTYPE, 256>(w, xb, rs, m, y, plan.S, part, s, epi)   \
-           : plan.bm == 128 ? launch_bm<QTYPE, 128>(w, xb, rs, m, y, plan.S, part, s, epi)   \
-                            : launch_bm<QTYPE, 64>(w, xb, rs, m, y, plan.S, part, s, epi)
+#define UNILLM_PREFILL_LAUNCH(QTYPE)                                                               \
+    return slices           ? launch_bm<QTYPE, 64, true>(w, xb, rs, slices, m, y, plan.S, part, s, \
+                                                         epi)                                      \
+           : plan.bm == 256 ? launch_bm<QTYPE, 256>(w, xb, rs, 0, m, y, plan.S, part, s, epi)      \
+           : plan.bm == 128 ? launch_bm<QTYPE, 128>(w, xb, rs, 0, m, y, plan.S, part, s, epi)      \
+                            : launch_bm<QTYPE, 64>(w, xb, rs, 0, m, y, plan.S, part, s, epi)
     switch (w.qtype) {
         case UNILLM_QTYPE_Q4_0: UNILLM_PREFILL_LAUNCH(UNILLM_QTYPE_Q4_0);
         case UNILLM_QTYPE_Q8_0: UNILLM_PREFILL_LAUNCH(UNILLM_QTYPE_Q8_0);
