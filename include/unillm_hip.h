@@ -250,7 +250,9 @@ int unillm_hip_kv_cache_truncate(unillm_kv_cache* c, int64_t len);
  * each appends to it.
  * Graph capture: the kernels read the cache length from device memory and
  * advance it there, so a captured call appends at the next position on every
- * replay (a decode step captured once serves successive tokens).  A replayed
+ * replay (a decode step captured once serves successive tokens).  How a captured
+ * call divides the keys among workgroups is fixed at capture: a decode step's for
+ * max_seq, a longer call's for 512 positions in all.  A replayed
  * call past max_seq appends nothing, writes NaN and makes the next length query
  * or eager call fail with the overflow message; clear / truncate reset it.
  * Alignment: qkv_dev 16 bytes; out_dev 4 bytes on a decode step, 16 bytes on a

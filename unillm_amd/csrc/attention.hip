@@ -1367,8 +1367,16 @@ namespace {
 // 75, paired in four 82, whole 97; m250 at 32 heads of 64 2-tile blocks in two splits 49.
 constexpr int kMaxPromptSplit = 8;
 constexpr int64_t kPromptRounds = 2;  // workgroups a CU when the keys are split
+// A captured call serves any length its cache reaches, and plans for this many positions in
+// all and at most four splits.  Planned for an empty cache, up to 256 tokens keep their keys
+// whole or in two, and a replay behind thousands of positions runs on a few workgroups (m32,
+// 32 heads of 128, us at 0 / 2032 / 4064 positions: 26 / 149 / 267, now 30 / 64 / 97; m256, 32
+// heads of 64 over 4, at 0 / 1920 / 3840: 30 / 104 / 174, now 29 / 69 / 110).  Eight splits take 33 / 51
+// / 65 at m32, but 46 at 0 for m128 against 36.
+constexpr int64_t kCapturedPositions = 512;
+constexpr int kCapturedSplit = 4;
 
-PromptPlan prompt_plan(int64_t m, int64_t H, int64_t D, int64_t len) {
+PromptPlan prompt_plan(int64_t m, int64_t H, int64_t D, int64_t len, int most_splits) {
     if (D != 64 && D != 128) return {4, 0, 1};
     const int64_t cus = device_info().cu_count;
     PromptPlan best{4, 1, 1};
@@ -1382,7 +1390,7 @@ PromptPlan prompt_plan(int64_t m, int64_t H, int64_t D, int64_t len) {
             const int64_t steps = paired && blocks > 1 ? first + last : last;
             const int64_t nblk = paired && blocks > 1 ? 2 : 1;
             const int64_t step_ns = (D == 128 ? 6500 : 3600) * (qt == 4 ? 4 : 3) / 4;
-            for (int S = 1; S <= kMaxPromptSplit; S *= 2) {
+            for (int S = 1; S <= most_splits; S *= 2) {
                 if (S > 1 && (wgs * S > kPromptRounds * cus || S > last)) break;
                 const int64_t rounds = (wgs * S + cus - 1) / cus;
                 int64_t ns = rounds * ((steps + S - 1) / S + 2 * nblk) * step_ns;
@@ -1433,8 +1441,12 @@ hipError_t launch_attention(const KvCache& kv, const float* qkv, int64_t m, int6
     void* ws = nullptr;
     hipError_t e;
     if (m * (H / kv.n_kv_heads) > kAttnMaxQ) {
-        // (captured: the length at a replay is not known; planned for an empty cache)
-        const PromptPlan plan = prompt_plan(m, H, D, std::max<int64_t>(len_hint, 0));
+        // captured, the length at a replay is not known: planned for kCapturedPositions
+        const int64_t len =
+            len_hint >= 0 ? len_hint
+                          : std::max<int64_t>(0, std::min<int64_t>(kCapturedPositions, kv.max_seq) - m);
+        const PromptPlan plan =
+            prompt_plan(m, H, D, len, len_hint >= 0 ? kMaxPromptSplit : kCapturedSplit);
         const size_t need = attention_call_bytes(
             kv, m, H, plan.S, prompt_copies_q(qkv, m, H, kv.n_kv_heads, D, plan.S, out));
         if ((e = stream_workspace(s, std::max<size_t>(need, 16), &ws, 2)) != hipSuccess) return e;
