@@ -195,3 +195,36 @@ def test_qmatmul_reserve_covers_every_shorter_call(n, k):
         s.synchronize()
         assert torch.equal(y, eager), m
         del g
+
+
+def test_swiglu_reserve_holds_what_its_calls_take():
+    # a SwiGLU call past 64 rows has its activation in the tiles: no [m, n] product is kept
+    # for it (2048 rows of 28672: 235 MB); the calls that do keep one fit in a capture
+    n, k = 28672, 512
+    _, ql = _weight(n, k, seed=5)
+    h = ctypes.c_void_p()
+    _capi.check(_capi.lib().unillm_hip_stream_create(ctypes.byref(h)))
+    s = torch.cuda.ExternalStream(h.value)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    ql.reserve(2048, swiglu=True, stream=s)
+    s.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 200 << 20
+    for m in (2048, 65, 64, 40, 5, 3):
+        x = _x(m, k, seed=m)
+        want = ql.forward_swiglu(x)
+        out = torch.empty(m, n // 2, device="cuda")
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s, capture_error_mode="thread_local"):
+            ql.forward_swiglu(x, out=out, stream=s)
+        for _ in range(2):
+            out.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(s):
+                g.replay()
+            s.synchronize()
+            # (the batched decode adds its slices in any order)
+            assert ((out - want).norm() / want.norm()).item() < 1e-5
+        del g

@@ -627,9 +627,11 @@ int unillm_hip_qmatmul_reserve(const unillm_qweight* w, int64_t m, int swiglu, v
     hipError_t e = stream_workspace(s, x0, &p, 0);
     // the batched decode's arrival tickets
     if (e == hipSuccess) e = stream_workspace(s, decode_sync_bytes(*w), &p, kSyncSlot);
-    // slot 1: the [gate | up] product of a SwiGLU call off the GEMV path
+    // slot 1: the [gate | up] product of a SwiGLU call on the batched decode's own kernels (or a
+    // GEMV without the epilogue): never past kDecodeMaxM rows
     if (e == hipSuccess && swiglu)
-        e = stream_workspace(s, (size_t)m * (size_t)w->n * sizeof(float), &p, 1);
+        e = stream_workspace(
+            s, (size_t)std::min<int64_t>(m, kDecodeMaxM) * (size_t)w->n * sizeof(float), &p, 1);
     // slot 3: the aligned copy of an x that sits only on a 4-byte boundary (any path)
     if (e == hipSuccess) e = stream_workspace(s, (size_t)m * (size_t)w->k * sizeof(float), &p, 3);
     return e == hipSuccess ? UNILLM_OK : fail_launch(e, "reserve");

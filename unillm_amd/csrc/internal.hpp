@@ -166,7 +166,8 @@ const DeviceInfo& device_info();
 // host threads are issued one at a time (a lock per stream, held by the entry point through
 // its last launch), the map is guarded by a mutex.
 // Slot 0 holds x in the MFMA paths' operand type; slot 1 the [gate | up] outputs
-// of a SwiGLU call off the GEMV path (both live during that call); slot 2
+// of a SwiGLU call that is neither fused on the GEMV nor on the prefill's tiles, and of a dense
+// weight's (both live during that call); slot 2
 // attention's partials (and, for hd 256 prompts, the rotated queries); slot 3 an
 // aligned copy of x; slot kSyncSlot the batched decode's arrival tickets, zeroed
 // when allocated (every launch leaves them zero again); slot kDenseSlot a dense
