@@ -53,8 +53,8 @@ extern "C" {
 /* Dense projection weights (GGML F32 / F16 / BF16).  candle's QMatMul::from_arc
  * dequantizes such a tensor to f32 and multiplies in f32 (its Tensor variant);
  * the reference's loader wraps every *_proj / lm_head tensor in a QMatMul whatever
- * its type (crates/runtime/src/weight_loader_core.rs:554-571).  Stored here as f32
- * rows (F16 and BF16 widen exactly) and multiplied by an f32 GEMM; any k >= 1. */
+ * its type (crates/runtime/src/weight_loader_core.rs:554-571).  Stored here in its
+ * own type and multiplied at f32's precision; any k >= 1. */
 #define UNILLM_QTYPE_F32 0
 #define UNILLM_QTYPE_F16 1
 #define UNILLM_QTYPE_BF16 30
@@ -148,9 +148,10 @@ int unillm_hip_qmatmul(const unillm_qweight* w, const float* x_dev, int64_t m, f
  * a 64 MiB scratch array that the library holds on each GPU from load to process
  * end, instead of the stream's workspace.  Limits: x 16-byte aligned; the scratch
  * takes m * k * 2 bytes (+ 4 m for prefill, + S * m * n * 4 when a prefill
- * splits k into S <= 16 slices; a split that would not fit gives way to the
- * 128-row plan that fits, at worst unsplit, agreeing with unillm_hip_qmatmul to
- * f32 rounding): calls beyond 64 MiB fail with
+ * splits k into S <= 16 slices; a split that would not fit is not taken, the
+ * result agreeing with unillm_hip_qmatmul to f32 rounding; a batch of 33 .. 64 rows
+ * that runs on the prefill's tiles takes 256 bytes a k slice of at most 1024 in
+ * place of the 4 m): calls beyond 64 MiB fail with
  * UNILLM_ERR_UNSUPPORTED before any launch.  All calls on one GPU share its
  * scratch: calls that overlap in time on one GPU (concurrent streams, or threads
  * without ordering) race and must not be issued. */

@@ -3,10 +3,10 @@
 candle's QMatMul::from_arc keeps such a tensor as a dequantized f32 tensor and
 multiplies in f32 (its Tensor variant); the reference's loader wraps every *_proj /
 lm_head tensor in a QMatMul whatever its type (weight_loader_core.rs:554-571).  The
-device holds the f32 rows (F16 and BF16 widen exactly) and runs an f32 GEMM.
+device holds the rows in their own type and forms the same f32 product.
 
-References: numpy float64 of the same widened weights (exact), x in f64; the f32
-GEMM's rounding over k terms stays near 1e-7 relative, so the bar is 1e-5 normwise.
+References: numpy float64 of the same widened weights (exact), x in f64; an f32
+sum's rounding over k terms stays near 1e-7 relative, so the bar is 1e-5 normwise.
 The epilogues (residual add, SwiGLU, layer norm in front) are checked against the
 same f64 formulas as the quantized paths' tests.
 """
@@ -82,7 +82,7 @@ def test_dense_from_torch_tensor_equals_from_bytes():
     assert a.qtype == F16 and a.shape == (n, k)
     x = torch.randn(m, k, device="cuda")
     assert torch.equal(a.forward(x), b.forward(x))
-    # and as f32 rows: the same as an f32 weight holding the widened values
+    # the same bits as an f32 weight holding the widened values (m 5: the GEMV's f32 FMAs)
     c = QuantLinear.from_dense(wt.float())
     assert torch.equal(c.forward(x), a.forward(x))
 

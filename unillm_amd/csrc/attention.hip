@@ -662,7 +662,8 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float* __restri
 //   S^T [32 keys][32 queries] = K . Q^T (v_mfma_f32_32x32x16_bf16: A lane l holds key
 //     l % 32, dimensions 8 (l / 32) .. + 7 of each 16; B the same of query l % 32, rotated
 //     (RoPE), scaled and split once a block by the tile's two waves: part 0 in registers,
-//     parts 1 and 2 in LDS, which leaves registers for two waves a SIMD);
+//     parts 1 and 2 in LDS, which leaves registers for two waves a SIMD: all 256 of them at
+//     hd 128, with 10 spilled, a few of those read back in each key step);
 //   a lane's 16 accumulators are 16 keys of ONE query (rows 8 (r / 4) + 4 (l / 32) +
 //     r % 4, column l % 32): the query's max and sum over the tile are a 16-value
 //     register reduction and one exchange with lane l ^ 32;

@@ -1,4 +1,5 @@
-// prefill.hip -- fused dequant + f16 MFMA GEMM for prefill (m >= 65).
+// prefill.hip -- fused dequant + f16 MFMA GEMM for prefill (m >= 65, and batches of 33 .. 64
+// rows on deep or large weights, prefill_takes_batch).
 //
 // y[m, n] = x[m, k] . dequant(W)[n, k]^T, the prefill call of QMatMul::forward
 // (crates/runtime/src/models_v2/llama.rs:1188, 1329), fp32 accumulation on the
@@ -18,7 +19,7 @@
 // per 256-column tile, so half the bytes, and no conversion sits in its inner
 // loop.
 //
-// Tile per workgroup: BM rows of x (BM = 256 or 128) x 256 weight rows
+// Tile per workgroup: BM rows of x (BM = 256, 128 or 64) x 256 weight rows
 // (output columns), k in steps of 64 (two blocks).  Eight waves (two per
 // SIMD) side by side: wave w owns all BM rows x columns 32 w .. 32 w + 31,
 // BM / 16 x 2 MFMA tiles of 16 x 16, fp32 accumulators in registers.
@@ -177,8 +178,9 @@ struct Ring {
     static constexpr int BS = 2 * PBN * 4;
     static constexpr int BH = KQ ? 2 * PBN * 4 : 0;  // K-quants: the step's group header per column
     static constexpr int STAGE = A + BP + BS + BH;
-    // stages: 4 for 128-row tiles (four fit in LDS; ~10 % over three measured),
-    // 3 for 256-row tiles; four of 64-row tiles leave room for a second workgroup a CU
+    // stages: 4 for 64- and 128-row tiles (four fit in LDS; ~10 % over three measured at
+    // 128), 3 for 256-row tiles.  Two workgroups a CU fit with 64-row tiles of Q4_0 only
+    // (73,984 bytes; Q4_K 82,176, Q8_0 106,752, Q5_K and Q6_K 114,944 of 163,840)
     static constexpr int STAGES = BM <= 128 ? 4 : 3;
     // + the tile's row scales of x (f16 operands): BM floats after the ring
     static constexpr int BYTES = STAGES * STAGE + BM * 4;
@@ -801,10 +803,19 @@ size_t prefill_workspace_bytes(const QWeight& w, int64_t m) {
 }
 
 // 49 .. 64 rows (Q8_0: 33 .. 64) of a deep or large weight run here rather than on the
-// batched decode, whose k slices of at most 1024 each add a tile's sums onto y: m64 k14336
-// n4096 Q4_0 32.9 -> 30.9 us a call, Q8_0 44.5 -> 35.2, Q4_K 44.6 -> 38.3, Q6_K 46.8 ->
-// 43.2; k4096 n28672 Q4_0 45.1 -> 42.9, Q8_0 59.2 -> 50.4, Q4_K 59.0 -> 54.8, but Q6_K 62.7
-// -> 67.8, n12288 Q4_0 23.9 -> 26.7 and n4096 15.8 -> 22.2.
+// batched decode, whose k slices of at most 1024 each add a tile's sums onto y.  us a call,
+// batched decode -> here (graph replays):
+//   m64 k14336 n4096: Q4_0 32.1 -> 29.3, Q8_0 41.9 -> 31.5, Q4_K 43.8 -> 34.5, Q5_K 45.6 ->
+//   40.8, Q6_K 45.1 -> 40.6; k11008 n4096: 28.9 -> 27.4, 38.3 -> 28.3, 38.0 -> 30.2, 39.5 ->
+//   31.9, 39.0 -> 31.7; k16384 n16384: 85.4 -> 73.6, 106.3 -> 89.0, 104.9 -> 95.7, 112.7 ->
+//   115.2, 109.8 -> 117.1;
+//   m64 k4096 n28672: Q4_0 42.9 -> 42.0, Q8_0 58.1 -> 48.7, Q4_K 56.1 -> 52.8, but Q5_K 62.1
+//   -> 66.1, Q6_K 61.4 -> 65.6, and n12288 Q4_0 22.9 -> 25.0.
+// Row counts off 8 gain more (m49 k14336 n4096 Q6_K 43.7 -> 39.6, k16384 n16384 150.8 ->
+// 113.7); at 56 and 64 rows Q5_K and Q6_K lose up to 9 % at some sizes past 8192 deep (k14336
+// n6144 50.9 -> 54.8, n8192 78.6 -> 68.0).  The lines lie between the sizes measured: at n k of
+// 86 Mi (k4096 n22016, on the batched decode) Q4_0 would take 35.6 here for 37.1, Q4_K 42.6
+// for 44.5, Q8_0 46.2 for 46.4.
 bool prefill_takes_batch(const QWeight& w, int64_t m) {
     if (m > kDecodeMaxM || m <= (w.qtype == UNILLM_QTYPE_Q8_0 ? 32 : 48) || !mfma_supports(w))
         return false;
