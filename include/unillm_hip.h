@@ -131,9 +131,11 @@ int unillm_hip_qmatmul(const unillm_qweight* w, const float* x_dev, int64_t m, f
  * have; x not on a 16-byte boundary is first copied (stream-ordered) into an
  * aligned per-stream buffer, since the kernels load it 16 bytes at a time.
  *
- * Workspace.  The MFMA paths (and SwiGLU off the GEMV path) use per-stream
+ * Workspace.  The MFMA paths, SwiGLU where it is a pass of its own, and dense
+ * weights past their GEMV use per-stream
  * device buffers that grow on first use and are then kept for later calls on
- * that stream.  Growing allocates, which cannot be recorded into a HIP graph: a
+ * that stream.  Host threads may share a stream: a call that uses them holds the
+ * stream's lock until its last launch is issued.  Growing allocates, which cannot be recorded into a HIP graph: a
  * call that would grow a buffer while its stream is being captured fails with
  * UNILLM_ERR_UNSUPPORTED and a message naming the size.  Reserve the buffers
  * before capturing (unillm_hip_qmatmul_reserve / unillm_hip_attention_reserve),
