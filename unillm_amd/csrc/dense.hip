@@ -128,8 +128,8 @@ __device__ __forceinline__ bool non_finite(float v) {
 // for F32), U groups requested ahead of the ones being multiplied, so 128 bytes a lane
 // stay in flight across row ends.  x sits in LDS as two planes of 4 floats a group:
 // every read is 16 consecutive bytes a lane, free of bank conflicts.  Bound by the
-// weight stream at one token: F16 k4096 n11008 (90 MB) 16.3 us a call (5.5 TB/s), against 228
-// us as an f32 library GEMM of rows widened to f32.  From three tokens on, by x's reads from
+// weight stream at one token: F16 k4096 n11008 (90 MB) 16.3 us in the kernel (5.5 TB/s; 17.9 a
+// call in an eager loop), against 228 us as an f32 library GEMM of rows widened to f32.  From three tokens on, by x's reads from
 // LDS (32 bytes a token for 8 weights): two of the wave's rows are multiplied by each read,
 // with half the groups in flight for each.  F16 m4 29.4 -> 24.1 us, m8 45.4 -> 33.0; F32 m8
 // 53.6 -> 41.1 (a single last row runs alone: no products are made for rows past the end).
