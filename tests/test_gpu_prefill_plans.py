@@ -150,3 +150,35 @@ def test_batch_outlier_keeps_the_other_slices(qtype, m, n, k):
     r = torch.randn_like(y)
     want = r.double() + ref
     assert _err(ql.forward_add(x, r), want) < TOL
+
+
+# a batch takes the faster of the batched decode and the prefill's tiles: sizes where the tiles
+# (asked for by path) lose a fifth to a third, and one where the decode does
+@pytest.mark.parametrize("qtype,m,n,k,tiles", [(Q6_K, 64, 24576, 9216, False),
+                                               (Q4_0, 56, 24576, 11008, False),
+                                               (Q8_0, 40, 24576, 11008, False),
+                                               (Q4_0, 64, 3072, 14336, False),
+                                               (Q8_0, 64, 4096, 14336, True)])
+def test_batch_takes_the_faster_kernels(qtype, m, n, k, tiles):
+    print(f"batch speed qtype={qtype} m={m} n={n} k={k}", flush=True)
+    # (in turn over weights that together outgrow the 256 MiB cache, as a model meets them: one
+    # weight that stays in the cache measures even at 24576 columns)
+    qls = [_weight(qtype, n, k, i) for i in range(2 if n * k > 1 << 27 else 6)]
+    x = torch.randn(m, k, device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    out = torch.empty(m, n, device="cuda")
+
+    def timed(**path):
+        best = 1e9
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for i in range(24):
+                qls[i % len(qls)].forward(x, out=out, **path)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    timed()
+    auto, asked = timed(), timed(path=PATH_PREFILL_MFMA)
+    assert auto < asked * (1.1 if tiles else 0.95)

@@ -803,26 +803,48 @@ size_t prefill_workspace_bytes(const QWeight& w, int64_t m) {
 }
 
 // 49 .. 64 rows (Q8_0: 33 .. 64) of a deep or large weight run here rather than on the
-// batched decode, whose k slices of at most 1024 each add a tile's sums onto y.  us a call,
-// batched decode -> here (graph replays):
-//   m64 k14336 n4096: Q4_0 32.1 -> 29.3, Q8_0 41.9 -> 31.5, Q4_K 43.8 -> 34.5, Q5_K 45.6 ->
-//   40.8, Q6_K 45.1 -> 40.6; k11008 n4096: 28.9 -> 27.4, 38.3 -> 28.3, 38.0 -> 30.2, 39.5 ->
-//   31.9, 39.0 -> 31.7; k16384 n16384: 85.4 -> 73.6, 106.3 -> 89.0, 104.9 -> 95.7, 112.7 ->
-//   115.2, 109.8 -> 117.1;
-//   m64 k4096 n28672: Q4_0 42.9 -> 42.0, Q8_0 58.1 -> 48.7, Q4_K 56.1 -> 52.8, but Q5_K 62.1
-//   -> 66.1, Q6_K 61.4 -> 65.6, and n12288 Q4_0 22.9 -> 25.0.
-// Row counts off 8 gain more (m49 k14336 n4096 Q6_K 43.7 -> 39.6, k16384 n16384 150.8 ->
-// 113.7); at 56 and 64 rows Q5_K and Q6_K lose up to 9 % at some sizes past 8192 deep (k14336
-// n6144 50.9 -> 54.8, n8192 78.6 -> 68.0).  The lines lie between the sizes measured: at n k of
-// 86 Mi (k4096 n22016, on the batched decode) Q4_0 would take 35.6 here for 37.1, Q4_K 42.6
-// for 44.5, Q8_0 46.2 for 46.4.
+// batched decode, whose k slices of at most 1024 each add a tile's sums onto y, where that was
+// measured faster: each type at k 2048 .. 28672, n 2048 .. 49152, 2 to 7 row counts (1484
+// sizes, graph replays, two weights in turn).  Of those taken 8 are more than 3 % slower than
+// the batched decode (Q4_K k14336 n16384 6 and 10 %, the others below 6); all in all a call
+// takes 0.81 times the batched decode's time, and would take 0.81 with the best choice
+// everywhere.  us a call, batched decode -> here:
+//  - rows off 8, where the batched decode's adds cost half as much again: Q6_K k16384 n16384 m49
+//    155.4 -> 115.5, k14336 n4096 45.6 -> 36.1; Q4_0 from n 4096 on, or 2560 past k 16384
+//    (k28672 n2048 31.3 -> 36.8: not taken);
+//  - rows by 8 with Q8_0 and Q4_K where the tiles and their k slices fill the CUs (m64 k14336
+//    n4096 Q8_0 44.5 -> 31.6, Q4_K 45.2 -> 35.8; at n 24576, 192 workgroups, Q4_K k9216 99.0 ->
+//    113.5: not taken); below n 4096, whose 16 slices a tile leave CUs idle, past k 16384, and
+//    Q8_0 from 49 rows on (k14336 n3072 m64 33.0 -> 29.9, m40 28.6 -> 28.7);
+//  - Q4_0, whose decode is the cheapest, where the CUs fill from n 8192 on, 6144 at k 11008, 4096
+//    at k 14336 (m64 k14336 n4096 32.9 -> 30.9, n8192 51.5 -> 39.4; k9216 n5120 25.1 -> 27.7: not
+//    taken);
+//  - Q5_K and Q6_K, whose dequant is the dearest, at n 4096 and 8192, where the decode's adds
+//    meet on few channels (Q6_K m64 k14336 46.3 -> 36.9 and 70.9 -> 64.4, k16384 49.2 -> 36.4),
+//    and below n 4096 to k 14336 (even: k14336 n3072 34.4 -> 34.4); elsewhere they lose up to a
+//    third (k9216 n24576 m64 111.2 -> 137.2, m56 101.0 -> 137.1).
 bool prefill_takes_batch(const QWeight& w, int64_t m) {
-    if (m > kDecodeMaxM || m <= (w.qtype == UNILLM_QTYPE_Q8_0 ? 32 : 48) || !mfma_supports(w))
+    const int q = w.qtype;
+    if (m > kDecodeMaxM || m <= (q == UNILLM_QTYPE_Q8_0 ? 32 : 48) || !mfma_supports(w))
         return false;
+    const bool dear = q == UNILLM_QTYPE_Q5_K || q == UNILLM_QTYPE_Q6_K;
     const int64_t nk = w.n * w.k;
     // (to k 262144: x and the slabs, 16 MiB at 64 rows, then fit every scratch that x alone did)
-    if (w.k > 8192) return nk >= (int64_t)40 << 20 && w.k <= (int64_t)1 << 18;
-    return nk >= (int64_t)96 << 20 && w.qtype != UNILLM_QTYPE_Q6_K && w.qtype != UNILLM_QTYPE_Q5_K;
+    if (w.k > (int64_t)1 << 18 || nk < (int64_t)(w.k > 8192 ? 40 : 96) << 20 ||
+        (w.k <= 8192 && dear))
+        return false;
+    const bool deepest = w.k > 16384 && w.n >= 2560;
+    if (m % 8 != 0) return q != UNILLM_QTYPE_Q4_0 || w.n >= 4096 || deepest;
+    if (dear) return (w.n % 4096 == 0 && w.n <= 8192) || (w.n <= 4096 && w.k <= 14336);
+    if (w.n < 4096)
+        return (q == UNILLM_QTYPE_Q8_0 && (m > 48 || deepest)) ||
+               (q == UNILLM_QTYPE_Q4_K && deepest);
+    // (full: too many tiles to split and still one workgroup a CU, or 13 / 16 of the CUs with k
+    // split)
+    const int64_t tiles = (w.n + PBN - 1) / PBN, cus = device_info().cu_count;
+    const bool full = 2 * tiles > cus || 16 * tiles * prefill_plan(w, m, 0, 1).S >= 13 * cus;
+    return full && (q != UNILLM_QTYPE_Q4_0 || w.n >= 8192 || w.k >= 14336 ||
+                    (w.n >= 6144 && w.k >= 11008));
 }
 
 hipError_t launch_prefill_mfma(const QWeight& w, const float* x, int64_t m, float* y,
